@@ -474,10 +474,19 @@ __device__ __forceinline__ void bin_offsets_block(const uint64_t* __restrict__ k
   }
 }
 
-__global__ __launch_bounds__(kThreads) void k_bin_offsets(const uint64_t* __restrict__ kv,
-                                                          const uint32_t* __restrict__ chunk_lo, uint32_t nch,
-                                                          int32_t* __restrict__ bo, uint64_t ncells_p1) {
-  bin_offsets_block(kv, chunk_lo, nch, bo, ncells_p1, blockIdx.x);
+// bin_offsets[c] = number of sorted keys < c by a binary search per cell
+// (c = blk * kThreads + thread), for grids below kRunSearchMinCells cells.
+__device__ __forceinline__ void cell_search_block(const uint64_t* __restrict__ kv, uint32_t n,
+                                                  int32_t* __restrict__ bo, uint32_t ncells_p1, uint32_t blk) {
+  const uint32_t c = blk * kThreads + threadIdx.x;
+  if (c >= ncells_p1) return;
+  uint32_t lo = 0, hi = n;
+  while (lo < hi) {
+    const uint32_t mid = lo + ((hi - lo) >> 1);
+    if (kv_key(kv[mid]) < c) lo = mid + 1;
+    else hi = mid;
+  }
+  bo[c] = (int32_t)lo;
 }
 
 // First and one-past-last sorted position of the run of `key` (its cell)
@@ -535,13 +544,19 @@ __device__ __forceinline__ uint32_t run_end(const uint64_t* __restrict__ kv, uin
   return hi;
 }
 
-// Cell count from which the permutation and block-row kernels find a cell's
-// bounds in the sorted keys near k (run_start / run_end, which the previous
-// kernels left in cache) instead of loading them from bin_offsets, whose
-// entries are then scattered over a large array (2^22 cells = 16 MB, four
-// times an XCD's L2): 0.339 -> 0.326 ms for instantiate at cfg5, while at
-// cfg1 the dependent loads of the search cost 5 us more than the cached
-// bin_offsets loads.
+// Cell count that divides the two ways of making bin_offsets and of finding a
+// cell's bounds.  From it on, bin_offsets is a store stream over chunks of
+// cells (bin_offsets_block) and the block-row kernel finds a cell's bounds in
+// the sorted keys near k (run_start / run_end, which the previous kernels
+// left in cache), because the entries are scattered over a large array (2^22
+// cells = 16 MB, four times an XCD's L2): 0.339 -> 0.326 ms for instantiate
+// at cfg5.  Below it a chunk of 1024 cells holds many particles, which one
+// workgroup walks, while a search per cell is a chain of log2(n) loads that
+// every cell takes at the same time, and needs no chunk table: with the
+// permutation in the same launch 6 us, where the chunk table, the chunks and
+// the permutation took 57 us for 8 K cells of 65536 particles (2D box), 56 us
+// for 8 K cells of 60033 and 68 us for 2 M cells of 250007.  The block-row
+// kernel loads its bounds from bin_offsets, which is in cache.
 constexpr uint64_t kRunSearchMinCells = 1ull << 22;
 
 // Permutation (destination slot of every input particle), in grid mode
@@ -551,20 +566,22 @@ constexpr uint64_t kRunSearchMinCells = 1ull << 22;
 // alone: unit_len[k] = particles of the unit starting at k (a run of up to
 // kUnitParticles particles of a cell with two or more, starting at a
 // multiple of kUnitParticles in the cell), 0 for the other particles of such
-// a cell, -1 for a particle alone in its cell; the unit-start flag is 1
-// where unit_len > 0.  When both are made they go to flags64 as masks, per
-// wave of 64 sorted positions w: flags64[2w] the block starts, flags64[2w + 1]
-// the unit starts (bit l: position 64w + l), and flags64[2 nw + w] their
-// counts (blocks in the low half, units in the high half; nw = the number of
-// waves), which one scan of nw words turns into each wave's first block row
-// and unit slot; else one flag per position to flags32.  The cell's first
-// position comes from bin_offsets or, with bo null, from the sorted keys.
+// a cell, -1 for a particle alone in its cell; a unit starts where unit_len >
+// 0.  With UNITS the flags go to flags64 as masks, per wave of 64 sorted
+// positions w: flags64[2w] the block starts (none without BLOCKS),
+// flags64[2w + 1] the unit starts (bit l: position 64w + l), and flags64[2 nw
+// + w] their counts (blocks in the low half, units in the high half; nw = the
+// number of waves), whose prefix gives each wave's first block row and unit
+// slot; else one flag per position goes to flags32.
+// Cell runs are read off the wave's mask of run heads; only a run that began
+// before the wave is searched for (run_start, once per wave), and only one
+// that leaves it looks at the next keys.
 template <bool BLOCKS, bool UNITS>
 __device__ __forceinline__ void permutation_block(const uint64_t* __restrict__ kv, uint32_t n, uint32_t N,
-                                                  int32_t* __restrict__ perm, const int32_t* __restrict__ bo,
-                                                  uint32_t maxp, uint32_t* __restrict__ flags32,
-                                                  uint64_t* __restrict__ flags64, int32_t* __restrict__ unit_len,
-                                                  int32_t* __restrict__ inv, uint32_t blk) {
+                                                  int32_t* __restrict__ perm, uint32_t maxp,
+                                                  uint32_t* __restrict__ flags32, uint64_t* __restrict__ flags64,
+                                                  int32_t* __restrict__ unit_len, int32_t* __restrict__ inv,
+                                                  uint32_t blk) {
   const uint32_t k = blk * kThreads + threadIdx.x;
   if (k >= n) return;
   const uint64_t w = kv[k];
@@ -573,55 +590,64 @@ __device__ __forceinline__ void permutation_block(const uint64_t* __restrict__ k
   perm[src] = (int32_t)(k - cloud);
   if (inv != nullptr) inv[k] = (int32_t)(src - cloud);
   if constexpr (BLOCKS || UNITS) {
-    const uint32_t key = kv_key(w);
-    const uint32_t rs = bo != nullptr ? (uint32_t)bo[key] : run_start(kv, k, key);
-    const uint32_t bf = BLOCKS && (k - rs) % maxp == 0 ? 1u : 0u;
-    uint32_t uf = 0;
+    const uint32_t key = kv_key(w), lane = (uint32_t)__lane_id(), k0 = k - lane;
+    uint32_t before = __shfl_up(key, 1, kWave);
+    if (lane == 0) before = k > 0 ? kv_key(kv[k - 1]) : ~key;
+    const uint64_t heads = __ballot(before != key);
+    const uint64_t upto = heads & (~0ull >> (63u - lane));
+    const uint32_t rs = upto ? k0 + 63u - (uint32_t)__clzll(upto) : run_start(kv, k0, key);
+    const bool bf = BLOCKS && (k - rs) % maxp == 0;
+    bool uf = false;
     if constexpr (UNITS) {
-      const bool alone = k == rs && (k + 1 == n || kv_key(kv[k + 1]) != key);
+      // one past the run's last position, or any bound >= k + kUnitParticles
+      const uint64_t after = lane == 63u ? 0ull : heads >> (lane + 1u);
+      uint32_t re = after ? k + 1u + (uint32_t)__builtin_ctzll(after) : min(k0 + (uint32_t)kWave, n);
+      if (k0 + (uint32_t)kWave < n) {  // wave-uniform, and every lane is active
+        const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)key, 63);
+        const uint32_t p = k0 + (uint32_t)kWave + lane;
+        const bool same = lane < (uint32_t)kUnitParticles - 1u && p < n && kv_key(kv[p]) == last;
+        const uint64_t run = __ballot(same);
+        if (!after) re += (uint32_t)__builtin_ctzll(~run);
+      }
       int32_t ul = -1;
-      if (!alone) {
-        ul = 0;
-        if ((k - rs) % (uint32_t)kUnitParticles == 0) {
-          uint32_t len = 1;
-          while (len < (uint32_t)kUnitParticles && k + len < n && kv_key(kv[k + len]) == key) ++len;
-          ul = (int32_t)len;
-          uf = 1;
-        }
+      if (k != rs || re != k + 1u) {  // not alone in its cell
+        uf = (k - rs) % (uint32_t)kUnitParticles == 0;
+        ul = uf ? (int32_t)min((uint32_t)kUnitParticles, re - k) : 0;
       }
       unit_len[k] = ul;
-    }
-    if constexpr (BLOCKS && UNITS) {
       // k runs over 64 consecutive positions a wave (kThreads is a multiple
       // of 64): its lane 0 holds the wave's first position, which is below n
       // whenever any lane of the wave is
-      const uint64_t bm = __ballot(bf != 0u), um = __ballot(uf != 0u);
-      if (__lane_id() == 0) {
-        const uint32_t w = k >> 6, nw = (n + 63) >> 6;
-        flags64[2 * (uint64_t)w] = bm;
-        flags64[2 * (uint64_t)w + 1] = um;
-        flags64[2 * (uint64_t)nw + w] = (uint64_t)__popcll(bm) | ((uint64_t)__popcll(um) << 32);
+      const uint64_t bm = __ballot(bf), um = __ballot(uf);
+      if (flags64 != nullptr) {
+        if (lane == 0) {
+          const uint32_t wv = k >> 6, nw = (n + 63) >> 6;
+          flags64[2 * (uint64_t)wv] = bm;
+          flags64[2 * (uint64_t)wv + 1] = um;
+          flags64[2 * (uint64_t)nw + wv] = (uint64_t)__popcll(bm) | ((uint64_t)__popcll(um) << 32);
+        }
+        return;
       }
-    } else {
-      flags32[k] = BLOCKS ? bf : uf;
     }
+    flags32[k] = (BLOCKS ? bf : uf) ? 1u : 0u;
   }
 }
 
+// The permutation and bin_offsets of a grid below kRunSearchMinCells cells in
+// one launch (the permutation does not read bin_offsets): the cells' searches
+// in the first nb_cells workgroups.
 template <bool BLOCKS, bool UNITS>
-__global__ __launch_bounds__(kThreads) void k_permutation(const uint64_t* __restrict__ kv, uint32_t n,
-                                                          uint32_t N, int32_t* __restrict__ perm,
-                                                          const int32_t* __restrict__ bo, uint32_t maxp,
-                                                          uint32_t* __restrict__ flags32,
-                                                          uint64_t* __restrict__ flags64,
-                                                          int32_t* __restrict__ unit_len,
-                                                          int32_t* __restrict__ inv) {
-  permutation_block<BLOCKS, UNITS>(kv, n, N, perm, bo, maxp, flags32, flags64, unit_len, inv, blockIdx.x);
+__global__ __launch_bounds__(kThreads) void k_search_permutation(
+    const uint64_t* __restrict__ kv, int32_t* __restrict__ bo, uint32_t ncells_p1, uint32_t nb_cells, uint32_t n,
+    uint32_t N, int32_t* __restrict__ perm, uint32_t maxp, uint32_t* __restrict__ flags32,
+    uint64_t* __restrict__ flags64, int32_t* __restrict__ unit_len, int32_t* __restrict__ inv) {
+  if (blockIdx.x < nb_cells) cell_search_block(kv, n, bo, ncells_p1, blockIdx.x);
+  else
+    permutation_block<BLOCKS, UNITS>(kv, n, N, perm, maxp, flags32, flags64, unit_len, inv, blockIdx.x - nb_cells);
 }
 
-// bin_offsets and the permutation in one launch, for grids whose permutation
-// finds cell bounds in the sorted keys (it does not read bin_offsets): one
-// permutation workgroup after every `every` chunk workgroups, so that the
+// The same from kRunSearchMinCells cells on, with bin_offsets as a store
+// stream over chunks of cells: one permutation workgroup after every `every` chunk workgroups, so that the
 // latency-bound permutation runs under the bin_offsets store stream instead
 // of after it (the dispatcher starts workgroups in order; with all
 // permutation workgroups first the two did not overlap).
@@ -634,7 +660,7 @@ __global__ __launch_bounds__(kThreads) void k_offsets_permutation(
   const uint32_t b = blockIdx.x, q = b / (every + 1), r = b % (every + 1);
   if (q < nb_perm) {
     if (r == every)
-      permutation_block<BLOCKS, UNITS>(kv, n, N, perm, nullptr, maxp, flags32, flags64, unit_len, inv, q);
+      permutation_block<BLOCKS, UNITS>(kv, n, N, perm, maxp, flags32, flags64, unit_len, inv, q);
     else if (q * every + r < nb_bo) bin_offsets_block(kv, chunk_lo, nch, bo, ncells_p1, q * every + r);
   } else {
     const uint32_t c = nb_perm * every + (b - nb_perm * (every + 1));
@@ -643,21 +669,28 @@ __global__ __launch_bounds__(kThreads) void k_offsets_permutation(
 }
 
 // Rows {global_cell, offset_in_cell, count, batch} (sphops/utils.cuh:295-301)
-// of the blocks starting at sorted position i < n (row rowidx[i]; position i
-// starts a block when rowidx[i + 1] > rowidx[i], the scan having counted its
-// flag), zero rows r in [total, max_blocks) (thread i handles position i and
-// row i), and the block count into total_out.  Cell bounds as in
-// k_permutation.  With UNITS the flags are k_permutation's masks (`masks`,
-// 2 nw words) and the scan its per-wave counts (`scan64`, nw + 1 words, the
-// totals last; a position's row and slot are its wave's plus the starts
-// below it in the wave): the fill's units are written too, units[slot] = {k,
-// unit_len[k]}, and their number into unit_total.
-template <bool UNITS>
+// of the blocks starting at sorted position i < n, zero rows r in [total,
+// max_blocks) (thread i handles position i and row i), and the block count
+// into total_out.  Cell bounds from bin_offsets, or with bo null from the
+// sorted keys.
+// UNITS: the flags are the permutation's masks (`masks`, 2 nw words) and
+// `counts` its nw per-wave counts; a position's row and unit slot are the
+// prefix of its wave's count plus the starts below it in the wave, and the
+// fill's units are written too, units[slot] = {k, unit_len[k]}, and their
+// number into unit_total.  FOLD: the workgroup sums the counts before its
+// positions itself (at most kFoldWaves of them, a few loads a thread), so no
+// scan runs between the permutation and this kernel; else `counts` has been
+// scanned, the totals at counts[nw].  info null (particle mode): no rows.
+// Without UNITS: row rowidx32[i], i starting a block when rowidx32[i + 1] is
+// above it, the scan having counted its flag.
+constexpr uint32_t kFoldWaves = 4096;  // 2^18 particles
+
+template <bool UNITS, bool FOLD>
 __global__ __launch_bounds__(kThreads) void k_block_rows(const uint64_t* __restrict__ kv, uint32_t n,
                                                          const int32_t* __restrict__ bo,
                                                          const uint32_t* __restrict__ rowidx32,
                                                          const uint64_t* __restrict__ masks,
-                                                         const uint64_t* __restrict__ scan64, uint32_t maxp,
+                                                         const uint64_t* __restrict__ counts, uint32_t maxp,
                                                          uint32_t G, int4* __restrict__ info,
                                                          const uint32_t* __restrict__ total32, uint64_t max_blocks,
                                                          int32_t* __restrict__ total_out,
@@ -665,19 +698,55 @@ __global__ __launch_bounds__(kThreads) void k_block_rows(const uint64_t* __restr
                                                          uint2* __restrict__ units, int32_t* __restrict__ unit_total) {
   const uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
   const uint32_t nw = (n + 63) >> 6;
-  const uint32_t t = UNITS ? (uint32_t)scan64[nw] : *total32;
+  constexpr uint32_t kWaves = kThreads / kWave;
+  uint64_t base = 0, totals = 0;  // FOLD: counts of the workgroups before this one, and of all
+  if constexpr (UNITS && FOLD) {
+    __shared__ uint64_t part[2][kWaves];
+    const uint32_t w0 = min(blockIdx.x * kWaves, nw);
+    for (uint32_t u = threadIdx.x; u < nw; u += kThreads) {
+      const uint64_t c = counts[u];
+      totals += c;
+      base += u < w0 ? c : 0ull;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      base += __shfl_down(base, off, 64);
+      totals += __shfl_down(totals, off, 64);
+    }
+    if (__lane_id() == 0) {
+      part[0][threadIdx.x >> 6] = base;
+      part[1][threadIdx.x >> 6] = totals;
+    }
+    __syncthreads();
+    base = totals = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < kWaves; ++u) {
+      base += part[0][u];
+      totals += part[1][u];
+    }
+  } else if constexpr (UNITS) {
+    totals = counts[nw];
+  }
+  const uint32_t t = UNITS ? (uint32_t)totals : *total32;
   if (i == 0) {
     if (total_out) *total_out = (int32_t)t;
-    if constexpr (UNITS) *unit_total = (int32_t)(scan64[nw] >> 32);
+    if constexpr (UNITS) *unit_total = (int32_t)(totals >> 32);
   }
-  if (i < max_blocks && i >= t) info[i] = make_int4(0, 0, 0, 0);
+  if (info != nullptr && i < max_blocks && i >= t) info[i] = make_int4(0, 0, 0, 0);
   if (i >= n) return;
   const uint32_t k = (uint32_t)i;
   uint32_t row;
   if constexpr (UNITS) {
     const uint32_t w = k >> 6;
     const uint64_t below = (1ull << (k & 63u)) - 1ull;
-    const uint64_t bm = masks[2 * (uint64_t)w], um = masks[2 * (uint64_t)w + 1], sk = scan64[w];
+    const uint64_t bm = masks[2 * (uint64_t)w], um = masks[2 * (uint64_t)w + 1];
+    uint64_t sk;
+    if constexpr (FOLD) {
+      sk = base;
+      for (uint32_t u = blockIdx.x * kWaves; u < w; ++u) sk += counts[u];  // wave-uniform, below kWaves steps
+    } else {
+      sk = counts[w];
+    }
     if ((um >> (k & 63u)) & 1ull)
       units[(uint32_t)(sk >> 32) + (uint32_t)__popcll(um & below)] = make_uint2(k, (uint32_t)unit_len[k]);
     if (((bm >> (k & 63u)) & 1ull) == 0ull) return;  // not a block start
@@ -1073,45 +1142,43 @@ void run_instantiate(Grid& g, const float* pos, int32_t* perm, int32_t* bo, int3
   }
   const uint64_t* skv = g.kv[cur];
 
-  // 3. bin_offsets via per-chunk key ranges
-  const uint32_t nch = (uint32_t)g.n_chunks;
-  hipLaunchKernelGGL(k_chunk_lo, blocks_for((uint64_t)nch + 1), dim3(kThreads), 0, st, skv, n, g.chunk_lo, nch);
-  SPHOPS_LAUNCHED();
-  const uint32_t nb_bo = (nch + kChunksPerBlock - 1) / kChunksPerBlock;
-
-  // 4. permutation (destination slot of each input particle), with the
-  // block-start flags in grid mode and, when the grid has the fill's
-  // buffers, the fill's work split (unit_len, the units and their count);
-  // on large grids it takes cell bounds from the sorted keys and runs in
-  // the bin_offsets launch
-  const int32_t* cell_bo = g.n_cells >= kRunSearchMinCells ? nullptr : bo;
+  // 3. bin_offsets and the permutation (destination slot of each input
+  // particle) in one launch, with the block-start flags in grid mode and,
+  // when the grid has the fill's buffers, the fill's work split (unit_len,
+  // the units and their count)
+  const bool search = g.n_cells < kRunSearchMinCells;
+  const int32_t* cell_bo = search ? bo : nullptr;
   const bool units = g.unit_len != nullptr && g.units != nullptr && g.unit_total != nullptr;
   // the masks of the block and unit starts and their per-wave counts take
   // 3 nw + 1 words of the other sort buffer (n + 1 words, free after the sort)
   const uint32_t nw = (n + 63) / 64;
-  const bool dual = units && !g.particle_mode && n >= 64 && dual_scan_fits(g, nw);
+  const bool dual = units && n >= 64 && (nw <= kFoldWaves || dual_scan_fits(g, nw));
   uint64_t* f64 = g.kv[cur ^ 1];
-  const uint32_t nb_perm = blocks_for(n).x;
-  if (cell_bo != nullptr) {
-    hipLaunchKernelGGL(k_bin_offsets, dim3(nb_bo), dim3(kThreads), 0, st, skv, g.chunk_lo, nch, bo, ncp1);
-    SPHOPS_LAUNCHED();
-  }
+  const uint32_t nb_perm = blocks_for(n).x, nb_cells = blocks_for(ncp1).x;
+  const uint32_t nch = (uint32_t)g.n_chunks;
+  const uint32_t nb_bo = (nch + kChunksPerBlock - 1) / kChunksPerBlock;
   const uint32_t every = std::max<uint32_t>(1u, nb_bo / std::max<uint32_t>(nb_perm, 1u));
   // the interleaved launch covers nb_perm * (every + 1) workgroups, or more
   // when the chunks outnumber the permutation's (every rounds down)
   const uint32_t nb_all = std::max(nb_bo + nb_perm, nb_perm * (every + 1));
+  if (!search) {
+    hipLaunchKernelGGL(k_chunk_lo, blocks_for((uint64_t)nch + 1), dim3(kThreads), 0, st, skv, n, g.chunk_lo, nch);
+    SPHOPS_LAUNCHED();
+  }
 #define SPHOPS_PERM(BL, UN, F32, F64)                                                                              \
   do {                                                                                                              \
-    if (cell_bo != nullptr)                                                                                         \
-      hipLaunchKernelGGL((k_permutation<BL, UN>), blocks_for(n), dim3(kThreads), 0, st, skv, n, g.p.N, perm,       \
-                         cell_bo, g.p.maxp, F32, F64, UN ? g.unit_len : nullptr, inv);                              \
+    if (search)                                                                                                     \
+      hipLaunchKernelGGL((k_search_permutation<BL, UN>), dim3(nb_cells + nb_perm), dim3(kThreads), 0, st, skv, bo, \
+                         (uint32_t)ncp1, nb_cells, n, g.p.N, perm, g.p.maxp, F32, F64,                              \
+                         UN ? g.unit_len : nullptr, inv);                                                           \
     else                                                                                                            \
       hipLaunchKernelGGL((k_offsets_permutation<BL, UN>), dim3(nb_all), dim3(kThreads), 0, st, skv, g.chunk_lo,    \
                          nch, bo, ncp1, nb_bo, n, g.p.N, perm, g.p.maxp, F32, F64, UN ? g.unit_len : nullptr, inv,  \
                          nb_perm, every);                                                                           \
   } while (0)
   if (g.particle_mode) {
-    if (units) SPHOPS_PERM(false, true, g.flags, nullptr);
+    if (dual) SPHOPS_PERM(false, true, nullptr, f64);
+    else if (units) SPHOPS_PERM(false, true, g.flags, nullptr);
     else SPHOPS_PERM(false, false, nullptr, nullptr);
   } else {
     if (dual) SPHOPS_PERM(true, true, nullptr, f64);
@@ -1120,22 +1187,27 @@ void run_instantiate(Grid& g, const float* pos, int32_t* perm, int32_t* bo, int3
 #undef SPHOPS_PERM
   SPHOPS_LAUNCHED();
 
-  // 5. block table (grid mode) and the fill's units
-  if (!g.particle_mode) {
-    const dim3 rows_grid = blocks_for(std::max<uint64_t>(n, g.max_blocks));
-    if (dual) {
-      uint64_t* counts = f64 + 2 * (uint64_t)nw;
-      device_exclusive_scan64(counts, counts, nw, g.scan_tmp, counts + nw, st);
-      hipLaunchKernelGGL(k_block_rows<true>, rows_grid, dim3(kThreads), 0, st, skv, n, cell_bo, nullptr, f64, counts,
-                         g.p.maxp, g.p.G, reinterpret_cast<int4*>(block_info), nullptr, g.max_blocks, total_blocks,
-                         g.unit_len, g.units, g.unit_total);
+  // 4. block table (grid mode) and the fill's units
+  int4* rows = g.particle_mode ? nullptr : reinterpret_cast<int4*>(block_info);
+  const dim3 rows_grid = blocks_for(std::max<uint64_t>(n, rows != nullptr ? g.max_blocks : 0));
+  if (dual) {
+    uint64_t* counts = f64 + 2 * (uint64_t)nw;
+    if (nw <= kFoldWaves) {
+      hipLaunchKernelGGL((k_block_rows<true, true>), rows_grid, dim3(kThreads), 0, st, skv, n, cell_bo, nullptr, f64,
+                         counts, g.p.maxp, g.p.G, rows, nullptr, g.max_blocks, total_blocks, g.unit_len, g.units,
+                         g.unit_total);
     } else {
-      device_exclusive_scan(g.flags, g.flags, n, g.scan_tmp, g.flags + n, st);
-      hipLaunchKernelGGL(k_block_rows<false>, rows_grid, dim3(kThreads), 0, st, skv, n, cell_bo, g.flags, nullptr,
-                         nullptr,
-                         g.p.maxp, g.p.G, reinterpret_cast<int4*>(block_info), g.flags + n, g.max_blocks,
-                         total_blocks, nullptr, nullptr, nullptr);
+      device_exclusive_scan64(counts, counts, nw, g.scan_tmp, counts + nw, st);
+      hipLaunchKernelGGL((k_block_rows<true, false>), rows_grid, dim3(kThreads), 0, st, skv, n, cell_bo, nullptr, f64,
+                         counts, g.p.maxp, g.p.G, rows, nullptr, g.max_blocks, total_blocks, g.unit_len, g.units,
+                         g.unit_total);
     }
+    SPHOPS_LAUNCHED();
+  } else if (!g.particle_mode) {
+    device_exclusive_scan(g.flags, g.flags, n, g.scan_tmp, g.flags + n, st);
+    hipLaunchKernelGGL((k_block_rows<false, false>), rows_grid, dim3(kThreads), 0, st, skv, n, cell_bo, g.flags,
+                       nullptr, nullptr, g.p.maxp, g.p.G, rows, g.flags + n, g.max_blocks, total_blocks, nullptr,
+                       nullptr, nullptr);
     SPHOPS_LAUNCHED();
   } else {
     if (units) {
