@@ -294,32 +294,54 @@ __global__ __launch_bounds__(kThreads) void k_radix_colscan(uint32_t* __restrict
   if (lane == 0) tot[d] = carry;
 }
 
-// Stable scatter of one radix digit.  Wave w of the tile owns keys
-// [w*1024, (w+1)*1024) and walks them 64 at a time in index order; lanes with
-// equal digits find each other with 8 ballots, so each key's rank among the
-// equal-digit keys before it is exact and no atomics are involved.
-__global__ __launch_bounds__(kThreads) void k_radix_scatter(const uint64_t* __restrict__ kin,
-                                                            uint64_t* __restrict__ kout, uint32_t n, int shift,
-                                                            const uint32_t* __restrict__ hist_scan,
-                                                            const uint32_t* __restrict__ tot, uint32_t ntiles) {
-  static_assert(kBins == 4 * kThreads, "four digits a thread in the digit prefix");
-  __shared__ uint32_t wcnt[kThreads / 64][kBins];
+// Stable scatter of one radix digit, one workgroup of kCountThreads threads
+// per tile.  Wave w of the tile owns keys [256 w, 256 (w + 1)) and walks them
+// 64 at a time in index order; lanes with equal digits find each other with
+// ten ballots, so each key's rank among the equal-digit keys before it is
+// exact and no atomics are involved.  The walk is a serial chain of ballots
+// and counter updates: sixteen waves of four steps take 9.5 us over 65536
+// keys and 13.7 us over 2^20, where four waves of sixteen took 13.2 and 17.  Thread d also finds digit d's first slot: the totals
+// of the digits below d (a prefix over the workgroup) plus the counts of d in
+// the tiles before this one.  FOLD: hist holds the tiles' raw counts and the
+// thread sums them itself (at most kFoldTiles), so no column scan runs
+// between the counts and this kernel; else hist holds their prefix over the
+// tiles and tot the digits' totals.
+constexpr uint32_t kFoldTiles = 32;
+
+template <bool FOLD>
+__global__ __launch_bounds__(kCountThreads) void k_radix_scatter(const uint64_t* __restrict__ kin,
+                                                                 uint64_t* __restrict__ kout, uint32_t n, int shift,
+                                                                 const uint32_t* __restrict__ hist,
+                                                                 const uint32_t* __restrict__ tot, uint32_t ntiles) {
+  static_assert(kBins == kCountThreads, "one digit a thread");
+  constexpr int kWaves = kCountThreads / kWave;
+  __shared__ uint16_t wcnt[kWaves][kBins];  // a wave counts at most 256 keys, a prefix at most kTile
   __shared__ uint32_t gbase[kBins];
-  __shared__ uint32_t wsum[kThreads / 64];
+  __shared__ uint32_t wsum[kWaves];
   const int wave = threadIdx.x >> 6, lane = __lane_id();
-  for (int i = threadIdx.x; i < (kThreads / 64) * kBins; i += kThreads) (&wcnt[0][0])[i] = 0;
-  {
-    // digit d's first slot: the totals of the digits below d (exclusive
-    // prefix over the workgroup, four consecutive digits a thread) plus the
-    // counts of d in the tiles before this one
-    const int d0 = 4 * threadIdx.x;
-    uint32_t v[4], sum = 0;
+  const uint32_t base = blockIdx.x * kTile + wave * (kTile / kWaves);
+  uint64_t word[kCountItems];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      v[u] = tot[d0 + u];
-      sum += v[u];
+  for (int t = 0; t < kCountItems; ++t) {
+    const uint32_t idx = base + t * 64 + lane;
+    word[t] = idx < n ? kin[idx] : 0ull;
+  }
+  for (int i = threadIdx.x; i < kWaves * kBins / 2; i += kCountThreads) reinterpret_cast<uint32_t*>(&wcnt[0][0])[i] = 0;
+  {
+    const uint32_t* __restrict__ h = hist + (uint64_t)threadIdx.x * ntiles;
+    uint32_t mine = 0, total = 0;
+    if constexpr (FOLD) {
+#pragma unroll 8
+      for (uint32_t t = 0; t < ntiles; ++t) {
+        const uint32_t c = h[t];
+        mine += t < blockIdx.x ? c : 0u;
+        total += c;
+      }
+    } else {
+      mine = h[blockIdx.x];
+      total = tot[threadIdx.x];
     }
-    uint32_t incl = sum;
+    uint32_t incl = total;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const uint32_t y = __shfl_up(incl, off, 64);
@@ -327,25 +349,15 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(const uint64_t* __re
     }
     if (lane == 63) wsum[wave] = incl;
     __syncthreads();
-    uint32_t run = incl - sum;
-    for (int w = 0; w < wave; ++w) run += wsum[w];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      gbase[d0 + u] = run + hist_scan[(uint64_t)(d0 + u) * ntiles + blockIdx.x];
-      run += v[u];
-    }
+    uint32_t below = incl - total;
+    for (int w = 0; w < wave; ++w) below += wsum[w];
+    gbase[threadIdx.x] = below + mine;
   }
-  __syncthreads();
-
-  const uint32_t base = blockIdx.x * kTile + wave * (kTile / (kThreads / 64));
   const uint64_t below_mask = lanemask_lt();
-  uint64_t word[kItems];
-  uint32_t rank[kItems];
+  uint32_t rank[kCountItems];
 #pragma unroll
-  for (int t = 0; t < kItems; ++t) {
-    const uint32_t idx = base + t * 64 + lane;
-    const bool valid = idx < n;
-    word[t] = valid ? kin[idx] : 0ull;
+  for (int t = 0; t < kCountItems; ++t) {
+    const bool valid = base + t * 64 + lane < n;
     const uint32_t digit = (kv_key(word[t]) >> shift) & (kBins - 1);
     uint64_t peers = __ballot(valid);
 #pragma unroll
@@ -356,25 +368,23 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(const uint64_t* __re
     }
     const uint32_t before = (uint32_t)__popcll(peers & below_mask);
     const uint32_t prior = wcnt[wave][digit];
-    if (valid && before == 0) wcnt[wave][digit] = prior + (uint32_t)__popcll(peers);
+    if (valid && before == 0) wcnt[wave][digit] = (uint16_t)(prior + (uint32_t)__popcll(peers));
     rank[t] = prior + before;
   }
   __syncthreads();
-  // exclusive prefix of the per-wave counts, digit by digit
-  for (int d = threadIdx.x; d < kBins; d += kThreads) {
+  {  // exclusive prefix of the per-wave counts, digit by digit
     uint32_t run = 0;
 #pragma unroll
-    for (int w = 0; w < kThreads / 64; ++w) {
-      const uint32_t c = wcnt[w][d];
-      wcnt[w][d] = run;
+    for (int w = 0; w < kWaves; ++w) {
+      const uint32_t c = wcnt[w][threadIdx.x];
+      wcnt[w][threadIdx.x] = (uint16_t)run;
       run += c;
     }
   }
   __syncthreads();
 #pragma unroll
-  for (int t = 0; t < kItems; ++t) {
-    const uint32_t idx = base + t * 64 + lane;
-    if (idx < n) {
+  for (int t = 0; t < kCountItems; ++t) {
+    if (base + t * 64 + lane < n) {
       const uint32_t digit = (kv_key(word[t]) >> shift) & (kBins - 1);
       kout[gbase[digit] + wcnt[wave][digit] + rank[t]] = word[t];
     }
@@ -905,11 +915,8 @@ __global__ __launch_bounds__(kCountThreads) void k_class_count(const int32_t* __
   if (threadIdx.x < kNumClasses) cnt[blockIdx.x * kNumClasses + threadIdx.x] = h[threadIdx.x];
 }
 
-// Waves of a segment of c items at g lanes per item (64 / g items a wave).
-__device__ __forceinline__ uint32_t seg_waves(uint32_t c, int32_t g) {
-  const uint32_t per = (uint32_t)(kWave / g);
-  return (c + per - 1) / per;
-}
+// log2 of the items a wave holds at g lanes per item (64 / g, a power of two).
+__device__ __forceinline__ uint32_t wave_items_log2(int32_t g) { return (uint32_t)(__clz(g) - 25); }
 
 // Stable scatter of a tile's items into order, class by class, and the wave
 // descriptors of the tile's segments.  The tile first finds its segment
@@ -920,11 +927,12 @@ __device__ __forceinline__ uint32_t seg_waves(uint32_t c, int32_t g) {
 // of its segments in the descriptor table of each group-size table (the
 // waves of all earlier segments), and the last tile writes the tables' wave
 // totals.  Same tile walk as the radix scatter: wave w owns items
-// [w*1024, (w+1)*1024) in index order; three ballots identify lanes of the
+// [256 w, 256 (w + 1)) in index order (8 us for 16 tiles and 10 us for 256,
+// where four waves a tile and a serial prefix by one thread took 16 and 20); three ballots identify lanes of the
 // same class.  Descriptor {first slot in order, group size << 8 | items}:
 // one per 64-lane wave of a segment.
 template <bool CSR>
-__global__ __launch_bounds__(kThreads) void k_class_scatter(const int32_t* __restrict__ src, uint32_t n,
+__global__ __launch_bounds__(kCountThreads) void k_class_scatter(const int32_t* __restrict__ src, uint32_t n,
                                                             ClassBounds cb, const uint32_t* __restrict__ cnt,
                                                             uint32_t* __restrict__ seg,
                                                             int32_t* __restrict__ order, GroupSizes gs1,
@@ -932,20 +940,30 @@ __global__ __launch_bounds__(kThreads) void k_class_scatter(const int32_t* __res
                                                             uint2* __restrict__ waves2,
                                                             int32_t* __restrict__ total1,
                                                             int32_t* __restrict__ total2) {
-  __shared__ uint32_t wcnt[kThreads / 64][kNumClasses];
+  constexpr int kWaves = kCountThreads / kWave;
+  __shared__ uint32_t wcnt[kWaves][kNumClasses];
   __shared__ uint32_t gbase[kNumClasses], gcnt[kNumClasses];
   __shared__ uint32_t wbase[2][kNumClasses];
-  __shared__ uint32_t part[3][kThreads / 64];
+  __shared__ uint32_t part[3][kWaves];
   const int wave = threadIdx.x >> 6, lane = __lane_id();
-  if (threadIdx.x < (kThreads / 64) * kNumClasses) (&wcnt[0][0])[threadIdx.x] = 0;
+  if (threadIdx.x < kWaves * kNumClasses) (&wcnt[0][0])[threadIdx.x] = 0;
   {
-    const uint32_t before = blockIdx.x * (uint32_t)kNumClasses;
+    static_assert(kCountThreads % kNumClasses == 0, "a thread's counts are all of one class");
+    const uint32_t before = blockIdx.x * (uint32_t)kNumClasses, q = threadIdx.x % kNumClasses;
+    const uint32_t mine = cnt[before + q];  // the tile's own count of class q
+    uint32_t l1 = 0, l2 = 0;
+#pragma unroll
+    for (int u = 0; u < kNumClasses; ++u) {
+      l1 = q == (uint32_t)u ? wave_items_log2(gs1.g[u]) : l1;
+      l2 = q == (uint32_t)u ? wave_items_log2(gs2.g[u]) : l2;
+    }
+    const uint32_t r1 = (1u << l1) - 1u, r2 = (1u << l2) - 1u;
     uint32_t s = 0, w1 = 0, w2 = 0;
-    for (uint32_t i = threadIdx.x; i < before; i += kThreads) {
+    for (uint32_t i = threadIdx.x; i < before; i += kCountThreads) {
       const uint32_t c = cnt[i];
       s += c;
-      w1 += seg_waves(c, gs1.g[i % kNumClasses]);
-      if (tables == 2) w2 += seg_waves(c, gs2.g[i % kNumClasses]);
+      w1 += (c + r1) >> l1;
+      w2 += (c + r2) >> l2;
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -959,37 +977,48 @@ __global__ __launch_bounds__(kThreads) void k_class_scatter(const int32_t* __res
       part[2][wave] = w2;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      uint32_t run = 0, r1 = 0, r2 = 0;
-      for (int w = 0; w < kThreads / 64; ++w) {
-        run += part[0][w];
-        r1 += part[1][w];
-        r2 += part[2][w];
+    if (wave == 0) {
+      // totals of the earlier tiles, then the prefix over the tile's classes
+      // (lane q < kNumClasses: class q; the others repeat)
+      uint32_t b0 = part[0][lane % kWaves], b1 = part[1][lane % kWaves], b2 = part[2][lane % kWaves];
+#pragma unroll
+      for (int off = kWaves / 2; off > 0; off >>= 1) {
+        b0 += __shfl_xor(b0, off, kWaves);
+        b1 += __shfl_xor(b1, off, kWaves);
+        b2 += __shfl_xor(b2, off, kWaves);
       }
-      for (int q = 0; q < kNumClasses; ++q) {
-        const uint32_t c = cnt[before + q];
-        gbase[q] = run;
-        gcnt[q] = c;
-        seg[before + q] = run;
-        run += c;
-        wbase[0][q] = r1;
-        r1 += seg_waves(c, gs1.g[q]);
-        wbase[1][q] = r2;
-        if (tables == 2) r2 += seg_waves(c, gs2.g[q]);
+      const uint32_t m1 = (mine + r1) >> l1, m2 = (mine + r2) >> l2;
+      uint32_t p0 = mine, p1 = m1, p2 = m2;
+#pragma unroll
+      for (int off = 1; off < kNumClasses; off <<= 1) {
+        const uint32_t y0 = __shfl_up(p0, off, kNumClasses), y1 = __shfl_up(p1, off, kNumClasses),
+                       y2 = __shfl_up(p2, off, kNumClasses);
+        if ((lane & (kNumClasses - 1)) >= off) {
+          p0 += y0;
+          p1 += y1;
+          p2 += y2;
+        }
       }
-      if (blockIdx.x == gridDim.x - 1) {
-        seg[before + kNumClasses] = run;
-        *total1 = (int32_t)r1;
-        if (tables == 2) *total2 = (int32_t)r2;
+      if (lane < kNumClasses) {
+        gbase[lane] = b0 + p0 - mine;
+        gcnt[lane] = mine;
+        seg[before + lane] = b0 + p0 - mine;
+        wbase[0][lane] = b1 + p1 - m1;
+        wbase[1][lane] = b2 + p2 - m2;
+        if (lane == kNumClasses - 1 && blockIdx.x == gridDim.x - 1) {
+          seg[before + kNumClasses] = b0 + p0;
+          *total1 = (int32_t)(b1 + p1);
+          if (tables == 2) *total2 = (int32_t)(b2 + p2);
+        }
       }
     }
   }
   __syncthreads();
-  const uint32_t base = blockIdx.x * kTile + wave * (kTile / (kThreads / 64));
+  const uint32_t base = blockIdx.x * kTile + wave * (kTile / kWaves);
   const uint64_t below_mask = lanemask_lt();
-  uint32_t cls[kItems], rank[kItems];
+  uint32_t cls[kCountItems], rank[kCountItems];
 #pragma unroll
-  for (int t = 0; t < kItems; ++t) {
+  for (int t = 0; t < kCountItems; ++t) {
     const uint32_t idx = base + t * 64 + lane;
     const int32_t len = idx < n ? item_length<CSR>(src, idx) : -1;
     const bool valid = len >= 0;
@@ -1009,7 +1038,7 @@ __global__ __launch_bounds__(kThreads) void k_class_scatter(const int32_t* __res
   __syncthreads();
   if (threadIdx.x < kNumClasses) {
     uint32_t run = 0;
-    for (int w = 0; w < kThreads / 64; ++w) {
+    for (int w = 0; w < kWaves; ++w) {
       const uint32_t c = wcnt[w][threadIdx.x];
       wcnt[w][threadIdx.x] = run;
       run += c;
@@ -1017,7 +1046,7 @@ __global__ __launch_bounds__(kThreads) void k_class_scatter(const int32_t* __res
   }
   __syncthreads();
 #pragma unroll
-  for (int t = 0; t < kItems; ++t) {
+  for (int t = 0; t < kCountItems; ++t) {
     const uint32_t idx = base + t * 64 + lane;
     if (idx < n && item_length<CSR>(src, idx) >= 0) order[gbase[cls[t]] + wcnt[wave][cls[t]] + rank[t]] = (int32_t)idx;
   }
@@ -1027,11 +1056,11 @@ __global__ __launch_bounds__(kThreads) void k_class_scatter(const int32_t* __res
     uint2* __restrict__ waves = tb == 0 ? waves1 : waves2;
 #pragma unroll
     for (int q = 0; q < kNumClasses; ++q) {
-      const uint32_t lo = gbase[q], c = gcnt[q];
-      const uint32_t per = (uint32_t)(kWave / gs.g[q]);
-      const uint32_t nw = (c + per - 1) / per;
-      for (uint32_t u = threadIdx.x; u < nw; u += kThreads)
-        waves[wbase[tb][q] + u] = make_uint2(lo + u * per, ((uint32_t)gs.g[q] << 8) | min(per, c - u * per));
+      const uint32_t lo = gbase[q], c = gcnt[q], at = wbase[tb][q];
+      const uint32_t lg = wave_items_log2(gs.g[q]), per = 1u << lg;
+      const uint32_t nw = (c + per - 1) >> lg;
+      for (uint32_t u = threadIdx.x; u < nw; u += kCountThreads)
+        waves[at + u] = make_uint2(lo + u * per, ((uint32_t)gs.g[q] << 8) | min(per, c - u * per));
     }
   }
 }
@@ -1053,7 +1082,7 @@ void tiled_schedule(const Grid& g, const int32_t* src, const ClassBounds& cb, co
   SPHOPS_LAUNCHED();
   const int tables = waves2 != nullptr ? 2 : 1;  // a second table: same order, other group sizes
   const GroupSizes gsb = gs2 != nullptr ? *gs2 : gs;
-  hipLaunchKernelGGL((k_class_scatter<CSR>), dim3(ntiles), dim3(kThreads), 0, st, src, n, cb, cnt, seg, order, gs,
+  hipLaunchKernelGGL((k_class_scatter<CSR>), dim3(ntiles), dim3(kCountThreads), 0, st, src, n, cb, cnt, seg, order, gs,
                      gsb, tables, waves, tables == 2 ? waves2 : waves, wave_total,
                      tables == 2 ? wave_total2 : wave_total);
   SPHOPS_LAUNCHED();
@@ -1132,11 +1161,16 @@ void run_instantiate(Grid& g, const float* pos, int32_t* perm, int32_t* bo, int3
                          ntiles);
       SPHOPS_LAUNCHED();
     }
-    hipLaunchKernelGGL(k_radix_colscan, dim3(kBins / (kThreads / 64)), dim3(kThreads), 0, st, g.hist, ntiles,
-                       digit_totals);
-    SPHOPS_LAUNCHED();
-    hipLaunchKernelGGL(k_radix_scatter, dim3(ntiles), dim3(kThreads), 0, st, g.kv[cur], g.kv[cur ^ 1], n, shift,
-                       g.hist, digit_totals, ntiles);
+    if (ntiles <= kFoldTiles) {
+      hipLaunchKernelGGL(k_radix_scatter<true>, dim3(ntiles), dim3(kCountThreads), 0, st, g.kv[cur], g.kv[cur ^ 1], n,
+                         shift, g.hist, nullptr, ntiles);
+    } else {
+      hipLaunchKernelGGL(k_radix_colscan, dim3(kBins / (kThreads / 64)), dim3(kThreads), 0, st, g.hist, ntiles,
+                         digit_totals);
+      SPHOPS_LAUNCHED();
+      hipLaunchKernelGGL(k_radix_scatter<false>, dim3(ntiles), dim3(kCountThreads), 0, st, g.kv[cur], g.kv[cur ^ 1],
+                         n, shift, g.hist, digit_totals, ntiles);
+    }
     SPHOPS_LAUNCHED();
     cur ^= 1;
   }
