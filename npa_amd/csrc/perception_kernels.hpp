@@ -126,6 +126,29 @@ struct Walker {
 
 // ------------------------------------------------------------- row loads
 
+// N consecutive floats at any 4-byte aligned address, in loads of up to 16
+// bytes (global loads take dword-aligned addresses at every width).
+template <int N>
+__device__ __forceinline__ void load_dwords(const float* __restrict__ p, float* v) {
+  typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+  typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
+  if constexpr (N >= 4) {
+    const f4 t = *reinterpret_cast<const f4*>(p);
+    v[0] = t.x;
+    v[1] = t.y;
+    v[2] = t.z;
+    v[3] = t.w;
+    load_dwords<N - 4>(p + 4, v + 4);
+  } else if constexpr (N >= 2) {
+    const f2 t = *reinterpret_cast<const f2*>(p);
+    v[0] = t.x;
+    v[1] = t.y;
+    load_dwords<N - 2>(p + 2, v + 2);
+  } else if constexpr (N == 1) {
+    v[0] = *p;
+  }
+}
+
 template <int N, bool VEC>
 __device__ __forceinline__ void load_span(const float* __restrict__ p, float* v) {
   if constexpr (VEC) {
@@ -1217,6 +1240,25 @@ __device__ __forceinline__ const float* row_slice(const float* __restrict__ base
   return base + (uint64_t)j * stride + c0;
 }
 
+// N floats of a lane's slice of CW channels: 16-byte loads for slices that
+// are whole 16-byte vectors (the launcher checks the bases), dword-aligned
+// ones for the others (C = 12 or 20: slices of 3 or 5 floats).
+template <int CW, int N>
+__device__ __forceinline__ void load_slice(const float* __restrict__ p, float* v) {
+  if constexpr (CW % 4 == 0) load_span<N, true>(p, v);
+  else load_dwords<N>(p, v);
+}
+
+// Waves per SIMD the forward is compiled for: what its registers allow
+// without spills (the four rows a lane keeps in flight and its gradient sums
+// grow with the slice).  With the C = 16 clamped kernel's bound of 6
+// throughout, C = 32 spilled 212 bytes a lane.
+constexpr int fwd_quad_waves(int D, bool P, int CW) {
+  if (CW <= 4) return P ? (D == 3 ? 4 : 5) : 6;
+  if (CW <= 6) return D == 3 ? 4 : 5;
+  return D == 3 ? 3 : 4;
+}
+
 // PARTS: 3 for the fused pair, 1 for blur alone (upstream a.g), 2 for the
 // gradient alone (upstream a.g2); the other operator's loads and terms are
 // left out.
@@ -1224,7 +1266,7 @@ __device__ __forceinline__ const float* row_slice(const float* __restrict__ base
 // VGPRs and 4 waves per SIMD, but schedules the loop better than a bound of
 // 4: 0.871 against 0.883 ms at cfg5.
 template <int D, bool P, int CW, bool FULL, bool OFF32, int PARTS>
-__global__ __launch_bounds__(kThreads, CW == 4 ? 3 : 2) void k_blur_hybrid_bwd_quad(GridParams g, OpPtrs a) {
+__global__ __launch_bounds__(kThreads, CW <= 4 ? 3 : 2) void k_blur_hybrid_bwd_quad(GridParams g, OpPtrs a) {
   constexpr int C = 4 * CW;
   constexpr bool kB = (PARTS & 1) != 0, kG = (PARTS & 2) != 0;
   const uint32_t live = wave_limit(a.nwaves2, a.nwaves2_dev);
@@ -1257,9 +1299,9 @@ __global__ __launch_bounds__(kThreads, CW == 4 ? 3 : 2) void k_blur_hybrid_bwd_q
       const float mi = a.m[k], ri = a.rho[k];
       vi = mi / ri;
       mr2 = mi / (ri * ri);
-      if constexpr (kG) load_span<CW * D, true>(a.g2 + ((uint64_t)k * C + c0) * D, ggi);
-      if constexpr (FULL) load_span<CW, true>(a.s + (uint64_t)k * C + c0, si);
-      if constexpr (FULL && kB) load_span<CW, true>(a.g + (uint64_t)k * C + c0, gbi);
+      if constexpr (kG) load_slice<CW, CW * D>(a.g2 + ((uint64_t)k * C + c0) * D, ggi);
+      if constexpr (FULL) load_slice<CW, CW>(a.s + (uint64_t)k * C + c0, si);
+      if constexpr (FULL && kB) load_slice<CW, CW>(a.g + (uint64_t)k * C + c0, gbi);
       const int32_t* __restrict__ nidx = a.nidx;
       const Row row = Row::of(a, k);
       const int start = row.start;
@@ -1348,8 +1390,8 @@ __global__ __launch_bounds__(kThreads, CW == 4 ? 3 : 2) void k_blur_hybrid_bwd_q
             else { SPHOPS_QUAD_FETCH(3) }
     #undef SPHOPS_QUAD_FETCH
             float gbj[kB ? CW : 1], ggj[kG ? CW * D : 1];
-            if constexpr (kB) load_span<CW, true>(row_slice<OFF32>(a.g, j, C, c0), gbj);
-            if constexpr (kG) load_span<CW * D, true>(row_slice<OFF32>(a.g2, j, C * D, c0 * D), ggj);
+            if constexpr (kB) load_slice<CW, CW>(row_slice<OFF32>(a.g, j, C, c0), gbj);
+            if constexpr (kG) load_slice<CW, CW * D>(row_slice<OFF32>(a.g2, j, C * D, c0 * D), ggj);
             if constexpr (!FULL) {
     #pragma unroll
               for (int f = 0; f < CW; ++f) {
@@ -1361,7 +1403,7 @@ __global__ __launch_bounds__(kThreads, CW == 4 ? 3 : 2) void k_blur_hybrid_bwd_q
               }
             } else {
               float sj[CW];
-              load_span<CW, true>(row_slice<OFF32>(a.s, j, C, c0), sj);
+              load_slice<CW, CW>(row_slice<OFF32>(a.s, j, C, c0), sj);
               float coef = 0.0f;  // the pair's factor of rb in dL/dx
               if constexpr (kB) {
                 float A = 0.0f, Bv = 0.0f;
@@ -1458,11 +1500,12 @@ __global__ __launch_bounds__(kThreads, CW == 4 ? 3 : 2) void k_blur_hybrid_bwd_q
 // its channel slice.  The moment matrix is accumulated by the owning lane,
 // reduced over the group and handed to the four slice lanes.  PARTS: 3 for
 // the fused pair (blur into a.out0, gradient_hybrid into a.out3), 1 for blur
-// alone, 2 for gradient_hybrid alone (into a.out3).
+// alone, 2 for gradient_hybrid alone (into a.out3), 4 for the uncorrected
+// gradient alone (into a.out3; no moment matrix).
 template <int D, bool P, int CW, bool OFF32, int PARTS>
-__global__ __launch_bounds__(kThreads, 6) void k_blur_hybrid_fwd_quad(GridParams g, OpPtrs a) {
+__global__ __launch_bounds__(kThreads, fwd_quad_waves(D, P, CW)) void k_blur_hybrid_fwd_quad(GridParams g, OpPtrs a) {
   constexpr int C = 4 * CW;
-  constexpr bool kB = (PARTS & 1) != 0, kG = (PARTS & 2) != 0;
+  constexpr bool kB = (PARTS & 1) != 0, kM = (PARTS & 2) != 0, kG = (PARTS & 6) != 0;
   const uint32_t live = wave_limit(a.nwaves2, a.nwaves2_dev);
   const uint32_t stride = schedule_stride(live);
   for (uint32_t wave = schedule_wave(live); wave < live; wave += stride) {
@@ -1483,7 +1526,7 @@ __global__ __launch_bounds__(kThreads, 6) void k_blur_hybrid_fwd_quad(GridParams
     float M[D * D] = {};
     if (active) {
       unpack(xw[k], xi);
-      if constexpr (kG) load_span<CW, true>(a.s + (uint64_t)k * C + c0, si);
+      if constexpr (kG) load_slice<CW, CW>(a.s + (uint64_t)k * C + c0, si);
       const int32_t* __restrict__ nidx = a.nidx;
       const Row row = Row::of(a, k);
       const int start = row.start;
@@ -1533,10 +1576,10 @@ __global__ __launch_bounds__(kThreads, 6) void k_blur_hybrid_fwd_quad(GridParams
           // end has j = k and zero weights, so it adds nothing), and their
           // four row loads are issued before any of them is used
           float sj[4][CW];
-          load_span<CW, true>(row_slice<OFF32>(a.s, quad_get<0>(jo), C, c0), sj[0]);
-          load_span<CW, true>(row_slice<OFF32>(a.s, quad_get<1>(jo), C, c0), sj[1]);
-          load_span<CW, true>(row_slice<OFF32>(a.s, quad_get<2>(jo), C, c0), sj[2]);
-          load_span<CW, true>(row_slice<OFF32>(a.s, quad_get<3>(jo), C, c0), sj[3]);
+          load_slice<CW, CW>(row_slice<OFF32>(a.s, quad_get<0>(jo), C, c0), sj[0]);
+          load_slice<CW, CW>(row_slice<OFF32>(a.s, quad_get<1>(jo), C, c0), sj[1]);
+          load_slice<CW, CW>(row_slice<OFF32>(a.s, quad_get<2>(jo), C, c0), sj[2]);
+          load_slice<CW, CW>(row_slice<OFF32>(a.s, quad_get<3>(jo), C, c0), sj[3]);
           if (inr) {
             if constexpr (kB) wo = poly6(g.eps2, d2) * pj.w;
             if constexpr (kG) {
@@ -1544,10 +1587,12 @@ __global__ __launch_bounds__(kThreads, 6) void k_blur_hybrid_fwd_quad(GridParams
               const float to_ = spiky_mag(g.eps, d2, &d) * pj.w;
     #pragma unroll
               for (int e = 0; e < D; ++e) tro[e] = to_ * rr[e];
+              if constexpr (kM) {
     #pragma unroll
-              for (int p = 0; p < D; ++p)
+                for (int p = 0; p < D; ++p)
     #pragma unroll
-                for (int q = p; q < D; ++q) M[p * D + q] += tro[p] * rr[q];
+                  for (int q = p; q < D; ++q) M[p * D + q] += tro[p] * rr[q];
+              }
             }
           }
     #pragma unroll
@@ -1577,8 +1622,8 @@ __global__ __launch_bounds__(kThreads, 6) void k_blur_hybrid_fwd_quad(GridParams
       else walk(std::integral_constant<bool, false>{});
     }
     if constexpr (kB) grp_sum_streams(G, blur);
-    if constexpr (kG) {
-      grp_sum_streams(G, acc);
+    if constexpr (kG) grp_sum_streams(G, acc);
+    if constexpr (kM) {
       grp_sum(G, M);
   #pragma unroll
       for (int q = 0; q < D * D; ++q) M[q] = quad_get<0>(M[q]);  // the group total, to the four slice lanes
@@ -1590,12 +1635,15 @@ __global__ __launch_bounds__(kThreads, 6) void k_blur_hybrid_fwd_quad(GridParams
       }
     }
     if (kG && active && stream == 0) {
-      float Ms[D * D], L[D * D];
+      float L[D * D];
+      if constexpr (kM) {
+        float Ms[D * D];
   #pragma unroll
-      for (int p = 0; p < D; ++p)
+        for (int p = 0; p < D; ++p)
   #pragma unroll
-        for (int q = 0; q < D; ++q) Ms[p * D + q] = (q >= p ? M[p * D + q] : M[q * D + p]) * g.cs;
-      safe_inv_sym<D>(Ms, a.tol, L);
+          for (int q = 0; q < D; ++q) Ms[p * D + q] = (q >= p ? M[p * D + q] : M[q * D + p]) * g.cs;
+        safe_inv_sym<D>(Ms, a.tol, L);
+      }
   #pragma unroll
       for (int f = 0; f < CW; ++f) {
         float raw[D];
@@ -1603,9 +1651,11 @@ __global__ __launch_bounds__(kThreads, 6) void k_blur_hybrid_fwd_quad(GridParams
         for (int e = 0; e < D; ++e) raw[e] = acc[f * D + e] * g.cs;
   #pragma unroll
         for (int e = 0; e < D; ++e) {
-          float o = 0.0f;
+          float o = kM ? 0.0f : raw[e];
+          if constexpr (kM) {
   #pragma unroll
-          for (int q = 0; q < D; ++q) o += raw[q] * L[q * D + e];
+            for (int q = 0; q < D; ++q) o += raw[q] * L[q * D + e];
+          }
           a.out3[((uint64_t)k * C + c0 + f) * D + e] = o;
         }
       }
@@ -2306,57 +2356,33 @@ void launch_pairs(const Grid& g, const int32_t* bo, OpPtrs a, hipStream_t st) {
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Lane-split kernels serve rows of 16 or 32 channels read as 16-byte vectors
-// (the fused pass B, forward and backward).
-inline bool split_ok(const OpPtrs& a) {
-  return a.nidx != nullptr && a.waves2 != nullptr && (a.C == 16 || a.C == 32) && aligned16(a.s) &&
-         aligned16(a.g) && aligned16(a.g2);
-}
-
 // Byte offsets into the (B*N, C*D) gradient rows fit in 32 bits.
 inline bool row_offsets_fit_32(const Grid& g, uint32_t C) {
   return g.n_keys * (uint64_t)C * 3u * 4u <= 0xFFFFFFFFull;
 }
 
-// PARTS as for k_blur_hybrid_fwd_quad.
+// Lane-split kernels (pass B, forward and backward): a list, its split
+// schedule, and rows of 16 or 32 channels on 16-byte bases, or of 8, 12, 20
+// or 24 (read in dword-aligned pieces) with row offsets of 32 bits.
+inline bool split_ok(const Grid& g, const OpPtrs& a) {
+  if (a.nidx == nullptr || a.waves2 == nullptr) return false;
+  if (a.C == 16 || a.C == 32) return aligned16(a.s) && aligned16(a.g) && aligned16(a.g2);
+  return (a.C == 8 || a.C == 12 || a.C == 20 || a.C == 24) && row_offsets_fit_32(g, a.C);
+}
+
+// The lane-split launchers (perception_pass_b.hpp, compiled in translation
+// units of their own): over the schedule a.waves2, positions and volumes
+// already packed into a.xw; parts as the kernels' PARTS.
+template <int D, bool P>
+void pass_b_forward(const Grid& g, int parts, const OpPtrs& a, hipStream_t st);
+template <int D, bool P>
+void pass_b_backward(const Grid& g, int parts, bool full, const OpPtrs& a, hipStream_t st);
+
 template <int D, bool P, int PARTS = 3>
 void launch_blur_hybrid_fwd_quad(const Grid& g, OpPtrs a, hipStream_t st) {
   if (g.n_keys == 0) return;
-  const uint32_t wgs = schedule_groups(a.nwaves2, a.nwaves2_dev);
   pack_for<D, VolumeWeights>(g, a, st);
-  if (wgs == 0) return;
-  const bool off32 = row_offsets_fit_32(g, a.C);
-#define SPHOPS_FWD_QUAD(CW, O32) \
-  hipLaunchKernelGGL((k_blur_hybrid_fwd_quad<D, P, CW, O32, PARTS>), dim3(wgs), dim3(kThreads), 0, st, g.p, a)
-  if (a.C == 16) {
-    if (off32) SPHOPS_FWD_QUAD(4, true);
-    else SPHOPS_FWD_QUAD(4, false);
-  } else {
-    if (off32) SPHOPS_FWD_QUAD(8, true);
-    else SPHOPS_FWD_QUAD(8, false);
-  }
-#undef SPHOPS_FWD_QUAD
-  SPHOPS_LAUNCHED();
-}
-
-// The lane-split pass-B backward over the schedule a.waves2 (positions and
-// volumes already packed into a.xw); PARTS as for k_blur_hybrid_bwd_quad.
-template <int D, bool P, bool FULL, int PARTS = 3>
-void launch_blur_hybrid_bwd_quad_packed(const Grid& g, const OpPtrs& a, hipStream_t st) {
-  const uint32_t wgs = schedule_groups(a.nwaves2, a.nwaves2_dev);
-  if (wgs == 0) return;
-  const bool off32 = row_offsets_fit_32(g, a.C);
-#define SPHOPS_BWD_QUAD(CW, O32) \
-  hipLaunchKernelGGL((k_blur_hybrid_bwd_quad<D, P, CW, FULL, O32, PARTS>), dim3(wgs), dim3(kThreads), 0, st, g.p, a)
-  if (a.C == 16) {
-    if (off32) SPHOPS_BWD_QUAD(4, true);
-    else SPHOPS_BWD_QUAD(4, false);
-  } else {
-    if (off32) SPHOPS_BWD_QUAD(8, true);
-    else SPHOPS_BWD_QUAD(8, false);
-  }
-#undef SPHOPS_BWD_QUAD
-  SPHOPS_LAUNCHED();
+  pass_b_forward<D, P>(g, PARTS, a, st);
 }
 
 template <int D, bool P, bool FULL, int PARTS = 3>
@@ -2368,7 +2394,7 @@ void launch_blur_hybrid_bwd_quad(const Grid& g, OpPtrs a, hipStream_t st) {
   const bool cells = a.nown != nullptr && a.cells != nullptr && a.cell_count != nullptr && D == 3 && !P &&
                      a.C == 16 && aligned16(a.out1);
   if (!cells) a.nown = nullptr;
-  launch_blur_hybrid_bwd_quad_packed<D, P, FULL, PARTS>(g, a, st);
+  pass_b_backward<D, P>(g, PARTS, FULL, a, st);
   if constexpr (D == 3 && !P) {
     if (cells) {
       hipLaunchKernelGGL((k_cell_pairs_bwd<D, FULL, PARTS>), dim3(kCellWorkgroups), dim3(kCellThreads), 0, st, g.p,
@@ -2392,7 +2418,7 @@ void launch_blur_hybrid_bwd_tiles(const Grid& g, const int32_t* bo, OpPtrs a, hi
   b.waves2 = a.waves_sparse;
   b.nwaves2 = a.nwaves_sparse;
   b.nwaves2_dev = a.nwaves_sparse_dev;
-  launch_blur_hybrid_bwd_quad_packed<D, P, FULL>(g, b, st);
+  pass_b_backward<D, P>(g, 3, FULL, b, st);
 }
 
 // Cell tiles of a snapshot (see perception_tiled.hpp): units of up to kTileP
@@ -2447,18 +2473,24 @@ void forward_dispatch(const Grid& g, Op op, const int32_t* bo, const OpPtrs& a_i
     // blur alone stays on the grouped kernel (a row per lane), which is faster
     // for it than the lane-split kernel (0.28 against 0.30 ms at cfg5)
     case Op::Blur: return launch_channels<D, P, OpBlur>(g, bo, a, st);
-    case Op::Gradient: return launch_channels<D, P, OpGradient>(g, bo, a, st);
-    case Op::GradientHybrid: {
-      // over a neighbour list with 16 or 32 channels: the lane-split kernel
-      // with the gradient_hybrid part only (its output in out3)
+    case Op::Gradient: {
+      // over a neighbour list: the lane-split kernel without the moment matrix
       OpPtrs b = a;
       b.out3 = a.out0;
-      if (split_ok(b)) return launch_blur_hybrid_fwd_quad<D, P, 2>(g, b, st);
+      if (split_ok(g, b)) return launch_blur_hybrid_fwd_quad<D, P, 4>(g, b, st);
+      return launch_channels<D, P, OpGradient>(g, bo, a, st);
+    }
+    case Op::GradientHybrid: {
+      // over a neighbour list: the lane-split kernel with the
+      // gradient_hybrid part only (its output in out3)
+      OpPtrs b = a;
+      b.out3 = a.out0;
+      if (split_ok(g, b)) return launch_blur_hybrid_fwd_quad<D, P, 2>(g, b, st);
       return launch_channels<D, P, OpGradientHybrid>(g, bo, a, st);
     }
     case Op::DensityPair: return launch_pairs<D, P, OpDensityPair<D, P>>(g, bo, a, st);
     case Op::BlurGradientHybrid:
-      if (split_ok(a)) return launch_blur_hybrid_fwd_quad<D, P>(g, a, st);
+      if (split_ok(g, a)) return launch_blur_hybrid_fwd_quad<D, P>(g, a, st);
       return launch_channels<D, P, OpBlurGradientHybrid>(g, bo, a, st);
     case Op::NeighbourCandidates:
       if (g.n_keys) neighbour_candidates<D, P>(g, bo, a.x, st);
@@ -2485,9 +2517,8 @@ void backward_dispatch(const Grid& g, Op op, bool full, const int32_t* bo, const
     case Op::DensityGradient: return launch_pairs<D, P, OpDensityGradientBwd<D, P>>(g, bo, a, st);
     case Op::MomentMatrix: return launch_pairs<D, P, OpMomentMatrixBwd<D, P>>(g, bo, a, st);
     case Op::Blur:
-      // over a neighbour list with 16 or 32 channels: the lane-split kernel
-      // with the blur terms only
-      if (split_ok(a)) {
+      // over a neighbour list: the lane-split kernel with the blur terms only
+      if (split_ok(g, a)) {
         if (full) return launch_blur_hybrid_bwd_quad<D, P, true, 1>(g, a, st);
         return launch_blur_hybrid_bwd_quad<D, P, false, 1>(g, a, st);
       }
@@ -2499,7 +2530,7 @@ void backward_dispatch(const Grid& g, Op op, bool full, const int32_t* bo, const
       OpPtrs b = a;
       b.g2 = a.g;
       b.g = nullptr;
-      if (split_ok(b)) {
+      if (split_ok(g, b)) {
         if (full) return launch_blur_hybrid_bwd_quad<D, P, true, 2>(g, b, st);
         return launch_blur_hybrid_bwd_quad<D, P, false, 2>(g, b, st);
       }
@@ -2508,11 +2539,11 @@ void backward_dispatch(const Grid& g, Op op, bool full, const int32_t* bo, const
     }
     case Op::DensityPair: return launch_pairs<D, P, OpDensityPairBwd<D, P>>(g, bo, a, st);
     case Op::BlurGradientHybrid: {
-      if (split_ok(a) && a.C == 16 && a.tile_units != nullptr && a.waves_sparse != nullptr) {
+      if (split_ok(g, a) && a.C == 16 && a.tile_units != nullptr && a.waves_sparse != nullptr) {
         if (full) return launch_blur_hybrid_bwd_tiles<D, P, true>(g, bo, a, st);
         return launch_blur_hybrid_bwd_tiles<D, P, false>(g, bo, a, st);
       }
-      if (split_ok(a)) {
+      if (split_ok(g, a)) {
         if (full) return launch_blur_hybrid_bwd_quad<D, P, true>(g, a, st);
         return launch_blur_hybrid_bwd_quad<D, P, false>(g, a, st);
       }
