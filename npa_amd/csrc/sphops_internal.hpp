@@ -235,6 +235,28 @@ constexpr GroupSizes kListGroups{{1, 1, 2, 4, 8, 16, 32, 64}};
 // lane-split channel kernels: four lanes (channel slices) per pair stream,
 // 1, 1, 1, 1, 4, 8, 16, 16 streams per particle (about 12-48 pairs each)
 constexpr GroupSizes kSplitGroups{{4, 4, 4, 4, 16, 32, 64, 64}};
+// Groups for fewer particles, twice as wide up to kWideParticles and four
+// times up to kWidestParticles, but no wider than one step of the kernel
+// takes of a class's longest row: at the sizes above, that few particles are
+// no more than two rounds of the waves the chip holds (kWideParticles in
+// groups of 4 lanes: 8192), and the launch lasts as long as its longest
+// rows.  Pass-B backward, 1x / 2x / 4x: 108 / 87 / 88 us (65536 particles,
+// 3D, C = 32), 84 / 66 / 65 (3 x 20011, 3D periodic, C = 20), 106 / 95 / 102
+// (131072, C = 16); its forward 9.7 / 7.3 / 6.4 us at 4096 particles, but 64
+// / 74 / 88 at 250007.
+constexpr uint64_t kWideParticles = 1ull << 17;
+constexpr uint64_t kWidestParticles = 1ull << 13;
+constexpr GroupSizes kListGroupCaps{{2, 4, 8, 16, 32, 64, 64, 64}};
+constexpr GroupSizes kSplitGroupCaps{{8, 16, 32, 64, 64, 64, 64, 64}};
+inline GroupSizes group_sizes(const GroupSizes& base, const GroupSizes& caps, uint64_t particles) {
+  const int f = particles <= kWidestParticles ? 4 : particles <= kWideParticles ? 2 : 1;
+  GroupSizes r = base;
+  for (int q = 0; q < kNumClasses; ++q) {
+    const int32_t wide = base.g[q] * f < caps.g[q] ? base.g[q] * f : caps.g[q];
+    if (wide > r.g[q]) r.g[q] = wide;
+  }
+  return r;
+}
 void run_safe_inv(const float* in, float* out, uint64_t count, int dim, float tol, hipStream_t st);
 void fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st);
 // words (<= 256) from device memory to pinned host memory (its device view)
