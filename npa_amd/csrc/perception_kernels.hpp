@@ -2470,9 +2470,13 @@ void forward_dispatch(const Grid& g, Op op, const int32_t* bo, const OpPtrs& a_i
     case Op::Density: return launch_pairs<D, P, OpDensity<D, P>>(g, bo, a, st);
     case Op::DensityGradient: return launch_pairs<D, P, OpDensityGradient<D, P>>(g, bo, a, st);
     case Op::MomentMatrix: return launch_pairs<D, P, OpMomentMatrix<D, P>>(g, bo, a, st);
-    // blur alone stays on the grouped kernel (a row per lane), which is faster
-    // for it than the lane-split kernel (0.28 against 0.30 ms at cfg5)
-    case Op::Blur: return launch_channels<D, P, OpBlur>(g, bo, a, st);
+    case Op::Blur:
+      // blur alone stays on the grouped kernel (a row per lane) at 16 and 32
+      // channels, where it is faster than the lane-split kernel (0.28 against
+      // 0.30 ms at cfg5); at the other widths the lane-split kernel gives the
+      // bits of the fused pass
+      if (a.C != 16 && a.C != 32 && split_ok(g, a)) return launch_blur_hybrid_fwd_quad<D, P, 1>(g, a, st);
+      return launch_channels<D, P, OpBlur>(g, bo, a, st);
     case Op::Gradient: {
       // over a neighbour list: the lane-split kernel without the moment matrix
       OpPtrs b = a;

@@ -45,7 +45,9 @@ void pass_b_forward(const Grid& g, int parts, const OpPtrs& a, hipStream_t st) {
   hipLaunchKernelGGL((k_blur_hybrid_fwd_quad<D, P, CW, O32, PARTS>), dim3(wgs), dim3(kThreads), 0, st, g.p, a)
     if (parts == 3) SPHOPS_FWD_QUAD(3);
     else if (parts == 2) SPHOPS_FWD_QUAD(2);
-    else SPHOPS_FWD_QUAD(4);
+    else if (parts == 4) SPHOPS_FWD_QUAD(4);
+    else if constexpr (CW % 4 != 0) SPHOPS_FWD_QUAD(1);
+    else throw Error("blur alone runs on the grouped kernel at this channel count");
 #undef SPHOPS_FWD_QUAD
   });
   SPHOPS_LAUNCHED();
