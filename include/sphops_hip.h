@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define SPHOPS_ABI_VERSION 21
+#define SPHOPS_ABI_VERSION 22
 
 #define SPHOPS_CLAMPED 0
 #define SPHOPS_PERIODIC 1
@@ -501,6 +501,27 @@ int sphops_relu_linear_forward(const float* a, const float* w, const float* b, f
  * column sums of dy; the same workspace size. */
 int sphops_relu_linear_weight_grad(const float* a, const float* dy, float* dw, float* db, int64_t rows,
                                    int in_features, int out_features, void* workspace, void* stream);
+
+/*
+ * The NPA MLP y = relu(z W1^T + b1) W2^T + b2 over rows of z (rows x
+ * in_features, fp32, row-major) for hidden = 128, in_features in [4, 168] and
+ * out_features in [4, 64] (models/npa.py:63-78 of the reference).  b1 and b2
+ * may be NULL.  The forward writes y (rows x out_features) and, unless a is
+ * NULL, the pre-activations a = z W1^T + b1 (rows x hidden) for the backward.
+ * The input gradient writes dz (rows x in_features); the weight gradients
+ * write dw1, db1, dw2 and db2 (any of them may be NULL), through a workspace
+ * of sphops_mlp_weight_grad_workspace_bytes bytes (-1: shape not supported),
+ * in a fixed order of summation.  Buffers need 4-byte alignment only.
+ */
+int sphops_mlp_forward(const float* z, const float* w1, const float* b1, const float* w2, const float* b2, float* a,
+                       float* y, int64_t rows, int in_features, int hidden, int out_features, void* stream);
+int sphops_mlp_input_grad(const float* dy, const float* w1, const float* w2, const float* a, float* dz, int64_t rows,
+                          int in_features, int hidden, int out_features, void* stream);
+int64_t sphops_mlp_weight_grad_workspace_bytes(int64_t rows, int in_features, int hidden, int out_features);
+int sphops_mlp_weight_grad(const float* z, const float* a, const float* dy, const float* w2, float* dw1, float* db1,
+                           float* dw2, float* db2, int64_t rows, int in_features, int hidden, int out_features,
+                           void* workspace, void* stream);
+
 
 #ifdef __cplusplus
 }

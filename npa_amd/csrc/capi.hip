@@ -1003,6 +1003,40 @@ int sphops_relu_linear_input_grad(const float* dy, const float* w, const float* 
   });
 }
 
+int sphops_mlp_forward(const float* z, const float* w1, const float* b1, const float* w2, const float* b2, float* a,
+                       float* y, int64_t rows, int in_features, int hidden, int out_features, void* stream) {
+  return guarded([&] {
+    require(sphops::mlp_fits(rows, in_features, hidden, out_features), "MLP shape not supported");
+    require(rows == 0 || (z && w1 && w2 && y), "null buffer");
+    sphops::run_mlp_forward(z, w1, b1, w2, b2, a, y, rows, in_features, out_features, sphops::as_stream(stream));
+  });
+}
+
+int sphops_mlp_input_grad(const float* dy, const float* w1, const float* w2, const float* a, float* dz, int64_t rows,
+                          int in_features, int hidden, int out_features, void* stream) {
+  return guarded([&] {
+    require(sphops::mlp_fits(rows, in_features, hidden, out_features), "MLP shape not supported");
+    require(rows == 0 || (dy && w1 && w2 && a && dz), "null buffer");
+    sphops::run_mlp_input_grad(dy, w1, w2, a, dz, rows, in_features, out_features, sphops::as_stream(stream));
+  });
+}
+
+int64_t sphops_mlp_weight_grad_workspace_bytes(int64_t rows, int in_features, int hidden, int out_features) {
+  if (!sphops::mlp_fits(rows, in_features, hidden, out_features)) return -1;
+  return sphops::mlp_weight_grad_floats(rows, in_features, out_features) * (int64_t)sizeof(float);
+}
+
+int sphops_mlp_weight_grad(const float* z, const float* a, const float* dy, const float* w2, float* dw1, float* db1,
+                           float* dw2, float* db2, int64_t rows, int in_features, int hidden, int out_features,
+                           void* workspace, void* stream) {
+  return guarded([&] {
+    require(sphops::mlp_fits(rows, in_features, hidden, out_features), "MLP shape not supported");
+    require(rows == 0 || (z && a && dy && w2 && workspace), "null buffer");
+    sphops::run_mlp_weight_grad(z, a, dy, w2, dw1, db1, dw2, db2, rows, in_features, out_features,
+                                static_cast<float*>(workspace), sphops::as_stream(stream));
+  });
+}
+
 }  // extern "C"
 
 // ------------------------------------------------ binning without allocation

@@ -311,6 +311,20 @@ bool relu_linear_input_grad_fits(int64_t rows, int nin);
 void run_relu_linear_input_grad(const float* dy, const float* w, const float* h, float* dx, int64_t rows, int nin,
                                 int nout, hipStream_t st);
 
+// mlp_rows.hip: Linear, ReLU, Linear with kMlpHidden hidden units over many rows
+constexpr int kMlpHidden = 128;
+constexpr int kMaxMlpIn = 168;   // the first layer's operand image and a row fit LDS and registers
+constexpr int kMaxMlpOut = 64;
+constexpr int64_t kMaxMlpRows = int64_t(1) << 30;  // byte offsets in a chunk of the weight gradients below 2^31
+bool mlp_fits(int64_t rows, int nin, int hidden, int nout);
+int64_t mlp_weight_grad_floats(int64_t rows, int nin, int nout);
+void run_mlp_forward(const float* z, const float* w1, const float* b1, const float* w2, const float* b2, float* a,
+                     float* y, int64_t rows, int nin, int nout, hipStream_t st);
+void run_mlp_input_grad(const float* dy, const float* w1, const float* w2, const float* a, float* dz, int64_t rows,
+                        int nin, int nout, hipStream_t st);
+void run_mlp_weight_grad(const float* z, const float* a, const float* dy, const float* w2, float* dw1, float* db1,
+                         float* dw2, float* db2, int64_t rows, int nin, int nout, float* work, hipStream_t st);
+
 constexpr uint32_t kMaxChannels = 64;
 constexpr int kRadixBins = 1024;  // digit values per radix-sort pass (10 bits)
 // Words of the radix histograms: kRadixBins tile counts per tile of 4096

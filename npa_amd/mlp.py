@@ -9,7 +9,9 @@ torch's forward and input gradient (both large, well-shaped GEMMs) and
 replaces the weight and bias gradients by the row-chunked matrix-core kernel.
 A ReLU followed by a Linear with at most 64 outputs (NPA's last layer) runs
 as ``ReluLinear``, whose backward computes the input gradient through both in
-one kernel.  ``mlp(module, z)`` runs a module the way the module would run
+one kernel.  The whole Linear, ReLU, Linear of NPA with 128 hidden units runs
+as ``MlpRows``, one kernel forward and two backward, which keep a row's hidden
+values in registers between the two products.  ``mlp(module, z)`` runs a module the way the module would run
 itself, with its ``torch.nn.Linear`` layers through these; the parameters are
 the module's own, so optimisers and checkpoints see no difference.
 """
@@ -25,6 +27,10 @@ _lib = _native.lib
 
 def _ptr(t):
     return ctypes.c_void_p(0 if t is None else t.data_ptr())
+
+
+def _stream(t):
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(t.device.index))
 
 
 class LinearRows(torch.autograd.Function):
@@ -126,6 +132,74 @@ class ReluLinear(torch.autograd.Function):
         return da, (dw if need_w else None), (db if need_b else None)
 
 
+class MlpRows(torch.autograd.Function):
+    """y = relu(z W1^T + b1) W2^T + b2 (``torch.nn.Linear``, ``ReLU``,
+    ``Linear``) over z of shape (..., in) in one kernel
+    (``sphops_mlp_forward``); the backward keeps z and the pre-activations and
+    takes dz and the weight gradients from one kernel each."""
+
+    @staticmethod
+    def forward(ctx, z, w1, b1, w2, b2):
+        hidden, in_f = w1.shape
+        out_f = w2.shape[0]
+        z2 = z.reshape(-1, in_f).contiguous()
+        rows = z2.shape[0]
+        dense = [None if t is None else t.detach().contiguous() for t in (w1, b1, w2, b2)]
+        ctx.shape = (rows, in_f, hidden, out_f)
+        ctx.biases = (b1 is not None, b2 is not None)
+        a = torch.empty(rows, hidden, device=z.device) if any(ctx.needs_input_grad) else None
+        y = torch.empty(rows, out_f, device=z.device)
+        _native.check(_lib.sphops_mlp_forward(_ptr(z2), *(_ptr(t) for t in dense), _ptr(a), _ptr(y), rows, in_f,
+                                              hidden, out_f, _stream(z)))
+        ctx.save_for_backward(z2, a, w1, w2)
+        return y.reshape(*z.shape[:-1], out_f)
+
+    @staticmethod
+    def backward(ctx, dy):
+        z2, a, w1, w2 = ctx.saved_tensors
+        need_z, need_w1, need_b1, need_w2, need_b2 = ctx.needs_input_grad
+        rows, in_f, hidden, out_f = ctx.shape
+        dy2 = dy.reshape(-1, out_f).contiguous()
+        if dy2.dtype != torch.float32 or not dy2.is_cuda:
+            raise TypeError("the MLP kernels take float32 GPU tensors")
+        w2c, st = w2.detach().contiguous(), _stream(dy2)
+        dz = dw1 = db1 = dw2 = db2 = None
+        if need_z:
+            dz = torch.empty_like(z2)
+            _native.check(_lib.sphops_mlp_input_grad(_ptr(dy2), _ptr(w1.detach().contiguous()), _ptr(w2c), _ptr(a),
+                                                     _ptr(dz), rows, in_f, hidden, out_f, st))
+            dz = dz.reshape(dy.shape[:-1] + (in_f,))
+        if need_w1 or need_b1 or need_w2 or need_b2:
+            dev = z2.device
+            dw1 = torch.empty(hidden, in_f, device=dev) if need_w1 else None
+            db1 = torch.empty(hidden, device=dev) if need_b1 else None
+            dw2 = torch.empty(out_f, hidden, device=dev) if need_w2 else None
+            db2 = torch.empty(out_f, device=dev) if need_b2 else None
+            nbytes = _lib.sphops_mlp_weight_grad_workspace_bytes(rows, in_f, hidden, out_f)
+            work = torch.empty(max(nbytes // 4, 1), device=dev)
+            _native.check(_lib.sphops_mlp_weight_grad(_ptr(z2), _ptr(a), _ptr(dy2), _ptr(w2c), _ptr(dw1), _ptr(db1),
+                                                      _ptr(dw2), _ptr(db2), rows, in_f, hidden, out_f, _ptr(work),
+                                                      st))
+        return dz, dw1, db1, dw2, db2
+
+
+def _mlp_rows_ok(z, first, second):
+    """The shapes, types and device that ``MlpRows`` takes; anything else (and
+    autocast, under which torch's products run in 16 bits) keeps the layers'
+    own functions."""
+    w1, w2 = first.weight, second.weight
+    tensors = [t for t in (z, w1, first.bias, w2, second.bias) if t is not None]
+    return (w1.shape[0] == MLP_HIDDEN == w2.shape[1] and 4 <= w1.shape[1] <= MLP_MAX_IN
+            and 4 <= w2.shape[0] <= RELU_LINEAR_MAX_OUT and z.dim() >= 1 and z.shape[-1] == w1.shape[1]
+            and all(t.is_cuda and t.dtype == torch.float32 and t.device == z.device for t in tensors)
+            and z.numel() <= MLP_MAX_ROWS * w1.shape[1] and not torch.is_autocast_enabled())
+
+
+# MlpRows: the hidden width its kernels tile for, and the widest input whose
+# operand image fits a CU's LDS
+MLP_HIDDEN = 128
+MLP_MAX_IN = 168
+MLP_MAX_ROWS = 1 << 30
 # ReluLinear keeps W's 32-output tiles in registers (the fused forward also
 # all of a row's in_features)
 RELU_LINEAR_MAX_OUT = 64
@@ -143,8 +217,9 @@ def relu_linear(a, layer):
 
 def mlp(module, z):
     """``module(z)`` for a ``torch.nn.Linear`` or a ``torch.nn.Sequential`` of
-    layers (the shapes NPA's _get_mlp builds): a ReLU followed by a Linear of at
-    most RELU_LINEAR_MAX_OUT outputs through ``ReluLinear``, every other Linear
+    layers (the shapes NPA's _get_mlp builds): a Linear, ReLU, Linear that
+    ``MlpRows`` takes through it, a ReLU followed by a Linear of at most
+    RELU_LINEAR_MAX_OUT outputs through ``ReluLinear``, every other Linear
     through ``LinearRows``; any other module runs as it is."""
     if isinstance(module, torch.nn.Linear):
         return linear(z, module)
@@ -154,6 +229,12 @@ def mlp(module, z):
         while i < len(layers):
             layer = layers[i]
             nxt = layers[i + 1] if i + 1 < len(layers) else None
+            last = layers[i + 2] if i + 2 < len(layers) else None
+            if (type(nxt) is torch.nn.ReLU and isinstance(layer, torch.nn.Linear) and isinstance(last, torch.nn.Linear)
+                    and _mlp_rows_ok(z, layer, last)):
+                z = MlpRows.apply(z, layer.weight, layer.bias, last.weight, last.bias)
+                i += 3
+                continue
             if (type(layer) is torch.nn.ReLU and isinstance(nxt, torch.nn.Linear)
                     and nxt.out_features <= RELU_LINEAR_MAX_OUT):
                 z = relu_linear(z, nxt)

@@ -10,7 +10,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get(
     "SPHOPS_HIP_LIB", os.path.join(os.path.dirname(_HERE), "_lib", "libsphops_hip.so"))
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 if not os.path.exists(LIB_PATH):
     raise ImportError(
@@ -71,6 +71,10 @@ _SIGNATURES = {
     "sphops_relu_linear_input_grad": ([_p, _p, _p, _p, _i64, _i32, _i32, _p], _i32),
     "sphops_relu_linear_forward": ([_p, _p, _p, _p, _i64, _i32, _i32, _p], _i32),
     "sphops_relu_linear_weight_grad": ([_p, _p, _p, _p, _i64, _i32, _i32, _p, _p], _i32),
+    "sphops_mlp_forward": ([_p, _p, _p, _p, _p, _p, _p, _i64, _i32, _i32, _i32, _p], _i32),
+    "sphops_mlp_input_grad": ([_p, _p, _p, _p, _p, _i64, _i32, _i32, _i32, _p], _i32),
+    "sphops_mlp_weight_grad_workspace_bytes": ([_i64, _i32, _i32, _i32], _i64),
+    "sphops_mlp_weight_grad": ([_p, _p, _p, _p, _p, _p, _p, _p, _i64, _i32, _i32, _i32, _p, _p], _i32),
     "sphops_forward": ([_p, _i32, _p, _p], _i32),
     "sphops_backward": ([_p, _i32, _i32, _i32, _i32, _p, _p], _i32),
     "sphops_neighbor_candidates": ([_p, _p, _p, _i32, _p], _i32),
