@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define SPHOPS_ABI_VERSION 22
+#define SPHOPS_ABI_VERSION 23
 
 #define SPHOPS_CLAMPED 0
 #define SPHOPS_PERIODIC 1
@@ -522,6 +522,87 @@ int sphops_mlp_weight_grad(const float* z, const float* a, const float* dy, cons
                            float* dw2, float* db2, int64_t rows, int in_features, int hidden, int out_features,
                            void* workspace, void* stream);
 
+
+/* sphops_neighbor_candidates, _fill and _schedule in one call and two
+ * launches fewer (no reference counterpart): counts (8-byte aligned) receives
+ * the pair total and the pairs not stored (two 64-bit words) and the wave
+ * counts of the two schedules (words 4 and 5); host_counts, unless NULL, is
+ * pinned host memory that receives the same six words, to be read once the
+ * stream has passed. */
+int sphops_neighbor_list(const sphops_grid* grid, const float* x, const int32_t* bin_offsets,
+                         int split_from_initialize, int32_t* nbr_start, int32_t* nbr_index, int64_t index_capacity,
+                         int32_t* nbr_count, int32_t* nbr_order, uint32_t* nbr_waves, uint32_t* nbr_waves_split,
+                         int32_t* counts, void* host_counts, void* stream);
+
+/* NPA.perceive (models/npa.py:87-137 of the reference) with the state and
+ * density gradients on, in one call each way: instantiate, bin (unit masses:
+ * mass holds ones and is not moved), list, density + density gradient, blur +
+ * gradient_hybrid, features.  All device buffers, shaped as the calls it
+ * replaces take them; z is what sphops_perception_features_forward writes.
+ * packed_mass / packed_volume (B*N float4, 16-byte aligned, or NULL) keep the
+ * (x, weight) records for the backward. */
+typedef struct sphops_perceive {
+  const float* x;
+  const float* s;
+  const float* mass;
+  int32_t* permutation;
+  int32_t* inverse;
+  int32_t* bin_offsets;
+  int32_t* block_info;
+  int32_t* total_blocks;
+  float* x_bin;
+  float* s_bin;
+  int32_t* nbr_start;
+  int32_t* nbr_count;
+  int32_t* nbr_index;
+  int64_t index_capacity;
+  int32_t* nbr_order;
+  uint32_t* nbr_waves;
+  uint32_t* nbr_waves_split;
+  int32_t nbr_wave_count;       /* launch estimates, as in sphops_args */
+  int32_t nbr_wave_count_split;
+  int32_t* counts;              /* as sphops_neighbor_list's */
+  void* host_counts;
+  float* rho;
+  float* grad_rho;
+  float* blur;
+  float* grad_s;
+  float* packed_mass;
+  float* packed_volume;
+  float* z;
+  uint32_t feature_dim;
+  int32_t flags;
+  float tol;
+  float coef_s;
+  float coef_rho;
+  float total_mass;
+} sphops_perceive;
+
+/* Upstreams (any may be NULL: zero), scratch and outputs of the backward.
+ * positions / state: whether z's gradient flows to x / s (stopgrad_pos and
+ * stopgrad_state off).  grad_x and grad_s (input order; NULL: not wanted)
+ * receive the sums d_x_bin + ... and d_s_bin + .... */
+typedef struct sphops_perceive_grads {
+  const float* dz;
+  const float* d_x_bin;
+  const float* d_s_bin;
+  int32_t positions;
+  int32_t state;
+  float* d_s;
+  float* d_blur;
+  float* d_grad_s;
+  float* d_grad_rho;
+  float* g_s;
+  float* g_x;
+  float* g_x2;
+  float* g_rho;
+  float* grad_x;
+  float* grad_s;
+} sphops_perceive_grads;
+
+int sphops_perceive_forward(sphops_grid* grid, const sphops_perceive* p, void* stream);
+int sphops_perceive_backward(const sphops_grid* grid, const sphops_perceive* p, const sphops_perceive_grads* d,
+                             void* stream);
 
 #ifdef __cplusplus
 }

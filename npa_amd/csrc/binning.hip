@@ -813,6 +813,55 @@ __global__ __launch_bounds__(kThreads) void k_move_rows(const float* __restrict_
   }
 }
 
+// The same scatter with the rows summed from up to three sources on the way
+// (a null source counts as absent, uniformly): the gradients that meet at a
+// binned particle are added while they are moved, instead of in a pass over
+// the rows each.
+template <int P, bool VEC4>
+__global__ __launch_bounds__(kThreads) void k_unbin_sum(RowSum in, const int32_t* __restrict__ inv,
+                                                        float* __restrict__ out_pos, float* __restrict__ out_state,
+                                                        uint32_t n, uint32_t N, uint32_t C, int lanes_log2) {
+  const uint64_t gid = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
+  const uint64_t k = gid >> lanes_log2;
+  const uint32_t q = (uint32_t)(gid & ((1u << lanes_log2) - 1));
+  if (k >= n) return;
+  const uint64_t dst = (k / N) * N + (uint32_t)inv[k];
+  if (q == 0 && out_pos != nullptr) {
+    float v[P] = {};
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      if (in.x[u] == nullptr) continue;
+#pragma unroll
+      for (int e = 0; e < P; ++e) v[e] += in.x[u][k * P + e];
+    }
+#pragma unroll
+    for (int e = 0; e < P; ++e) out_pos[dst * P + e] = v[e];
+  }
+  if (out_state == nullptr) return;
+  const uint32_t lanes = 1u << lanes_log2;
+  if constexpr (VEC4) {
+    const uint32_t U = C >> 2;
+    for (uint32_t w = q; w < U; w += lanes) {
+      float4 t = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+      for (int u = 0; u < 3; ++u) {
+        if (in.s[u] == nullptr) continue;
+        const float4 a = reinterpret_cast<const float4*>(in.s[u])[k * U + w];
+        t = make_float4(t.x + a.x, t.y + a.y, t.z + a.z, t.w + a.w);
+      }
+      reinterpret_cast<float4*>(out_state)[dst * U + w] = t;
+    }
+  } else {
+    for (uint32_t w = q; w < C; w += lanes) {
+      float t = 0.0f;
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        if (in.s[u] != nullptr) t += in.s[u][k * C + w];
+      out_state[dst * C + w] = t;
+    }
+  }
+}
+
 template <int D>
 void launch_keys(const Grid& g, const float* pos, uint32_t n, hipStream_t st) {
   const uint32_t ntiles = (uint32_t)g.n_tiles;
@@ -885,11 +934,17 @@ __device__ __forceinline__ int32_t item_length(const int32_t* __restrict__ src, 
 
 // Per tile of kTile items: the number of items of each class, written to
 // cnt[tile * kNumClasses + class].
-// Items of negative length are skipped: they get no class and no slot.
+// Items of negative length are skipped: they get no class and no slot.  With
+// fill_total the first workgroup also takes the list fill's totals
+// (fill_totals), which saves the fill a launch of its own.
 template <bool CSR>
 __global__ __launch_bounds__(kCountThreads) void k_class_count(const int32_t* __restrict__ src, uint32_t n,
-                                                               ClassBounds cb, uint32_t* __restrict__ cnt) {
+                                                               ClassBounds cb, uint32_t* __restrict__ cnt,
+                                                               unsigned long long* __restrict__ fill_ctr,
+                                                               uint32_t stripes,
+                                                               unsigned long long* __restrict__ fill_total) {
   __shared__ uint32_t h[kNumClasses];
+  if (fill_total != nullptr && blockIdx.x == 0) fill_totals(fill_ctr, stripes, fill_total);
   if (threadIdx.x < kNumClasses) h[threadIdx.x] = 0;
   __syncthreads();
   const uint32_t base = blockIdx.x * kTile;
@@ -939,7 +994,9 @@ __global__ __launch_bounds__(kCountThreads) void k_class_scatter(const int32_t* 
                                                             GroupSizes gs2, int tables, uint2* __restrict__ waves1,
                                                             uint2* __restrict__ waves2,
                                                             int32_t* __restrict__ total1,
-                                                            int32_t* __restrict__ total2) {
+                                                            int32_t* __restrict__ total2,
+                                                            const uint32_t* __restrict__ fill_total,
+                                                            uint32_t* host) {
   constexpr int kWaves = kCountThreads / kWave;
   __shared__ uint32_t wcnt[kWaves][kNumClasses];
   __shared__ uint32_t gbase[kNumClasses], gcnt[kNumClasses];
@@ -1009,6 +1066,13 @@ __global__ __launch_bounds__(kCountThreads) void k_class_scatter(const int32_t* 
           seg[before + kNumClasses] = b0 + p0;
           *total1 = (int32_t)(b1 + p1);
           if (tables == 2) *total2 = (int32_t)(b2 + p2);
+          if (host != nullptr) {  // into pinned host memory, visible there once the kernel is done
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              __hip_atomic_store(host + u, fill_total[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(host + 4, b1 + p1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(host + 5, b2 + p2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          }
         }
       }
     }
@@ -1070,7 +1134,7 @@ __global__ __launch_bounds__(kCountThreads) void k_class_scatter(const int32_t* 
 template <bool CSR>
 void tiled_schedule(const Grid& g, const int32_t* src, const ClassBounds& cb, const GroupSizes& gs, int32_t* order,
                     uint2* waves, int32_t* wave_total, hipStream_t st, const GroupSizes* gs2 = nullptr,
-                    uint2* waves2 = nullptr, int32_t* wave_total2 = nullptr) {
+                    uint2* waves2 = nullptr, int32_t* wave_total2 = nullptr, const FillTail* tail = nullptr) {
   const uint32_t n = (uint32_t)g.n_keys;
   const uint32_t ntiles = (uint32_t)g.n_tiles;
   const uint32_t nseg = (uint32_t)kNumClasses * ntiles;
@@ -1078,13 +1142,15 @@ void tiled_schedule(const Grid& g, const int32_t* src, const ClassBounds& cb, co
   // offsets (nseg + 1, the last is the number of scheduled items)
   uint32_t* cnt = g.hist;
   uint32_t* seg = cnt + nseg;
-  hipLaunchKernelGGL((k_class_count<CSR>), dim3(ntiles), dim3(kCountThreads), 0, st, src, n, cb, cnt);
+  hipLaunchKernelGGL((k_class_count<CSR>), dim3(ntiles), dim3(kCountThreads), 0, st, src, n, cb, cnt,
+                     tail ? g.stripes : nullptr, tail ? tail->stripes : 0u, tail ? tail->total : nullptr);
   SPHOPS_LAUNCHED();
   const int tables = waves2 != nullptr ? 2 : 1;  // a second table: same order, other group sizes
   const GroupSizes gsb = gs2 != nullptr ? *gs2 : gs;
   hipLaunchKernelGGL((k_class_scatter<CSR>), dim3(ntiles), dim3(kCountThreads), 0, st, src, n, cb, cnt, seg, order, gs,
                      gsb, tables, waves, tables == 2 ? waves2 : waves, wave_total,
-                     tables == 2 ? wave_total2 : wave_total);
+                     tables == 2 ? wave_total2 : wave_total,
+                     tail ? reinterpret_cast<const uint32_t*>(tail->total) : nullptr, tail ? tail->host : nullptr);
   SPHOPS_LAUNCHED();
 }
 
@@ -1099,10 +1165,10 @@ void run_split_schedule(const Grid& g, const int32_t* len, int32_t* order, uint2
 }
 
 void run_neighbour_schedule(const Grid& g, const int32_t* ncnt, int32_t* order, uint2* waves, int32_t* wave_total,
-                            uint2* waves2, int32_t* wave_total2, hipStream_t st) {
+                            uint2* waves2, int32_t* wave_total2, hipStream_t st, const FillTail* tail) {
   const GroupSizes split = group_sizes(kSplitGroups, kSplitGroupCaps, g.n_keys);
   tiled_schedule<false>(g, ncnt, kListClasses, group_sizes(kListGroups, kListGroupCaps, g.n_keys), order, waves,
-                        wave_total, st, &split, waves2, wave_total2);
+                        wave_total, st, &split, waves2, wave_total2, tail);
 }
 
 namespace {
@@ -1281,6 +1347,27 @@ void run_bin_particles(const Grid& g, const float* in_pos, const float* in_state
     if (vec4) SPHOPS_MOVE(4, true); else SPHOPS_MOVE(4, false);
   }
 #undef SPHOPS_MOVE
+  SPHOPS_LAUNCHED();
+}
+
+void run_unbin_sum(const Grid& g, const RowSum& in, const int32_t* inv, float* out_pos, float* out_state, uint32_t C,
+                   hipStream_t st) {
+  const uint32_t n = (uint32_t)g.n_keys;
+  if (n == 0) return;
+  bool vec4 = C % 4 == 0 && reinterpret_cast<uintptr_t>(out_state) % 16 == 0;
+  for (const float* p : in.s) vec4 = vec4 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+  const uint32_t units = out_state == nullptr ? 1u : vec4 ? C / 4 : C;
+  int lanes_log2 = 0;
+  while ((1u << lanes_log2) < units && lanes_log2 < 4) ++lanes_log2;
+  const dim3 grid = blocks_for((uint64_t)n << lanes_log2);
+#define SPHOPS_UNBIN(P, V) \
+  hipLaunchKernelGGL((k_unbin_sum<P, V>), grid, dim3(kThreads), 0, st, in, inv, out_pos, out_state, n, g.p.N, C, lanes_log2)
+  if (g.dim == 2) {
+    if (vec4) SPHOPS_UNBIN(2, true); else SPHOPS_UNBIN(2, false);
+  } else {
+    if (vec4) SPHOPS_UNBIN(4, true); else SPHOPS_UNBIN(4, false);
+  }
+#undef SPHOPS_UNBIN
   SPHOPS_LAUNCHED();
 }
 

@@ -716,6 +716,43 @@ static int neighbor_fill(const sphops_grid* grid, const float* x, const int32_t*
   });
 }
 
+int sphops_neighbor_list(const sphops_grid* grid, const float* x, const int32_t* bo, int split_from_initialize,
+                         int32_t* nbr_start, int32_t* nbr_index, int64_t index_capacity, int32_t* nbr_count,
+                         int32_t* nbr_order, uint32_t* nbr_waves, uint32_t* nbr_waves_split, int32_t* counts,
+                         void* host_counts, void* stream) {
+  int status = sphops_neighbor_candidates(grid, x, bo, split_from_initialize, stream);
+  if (status) return status;
+  return guarded([&] {
+    require(counts != nullptr, "null buffer");
+    require(reinterpret_cast<uintptr_t>(counts) % 8 == 0, "counts must be 8-byte aligned");
+    require(index_capacity >= 0, "negative index capacity");
+    require(index_capacity <= sphops::kMaxListEntries, "index_capacity above 2^30 entries");
+    const hipStream_t st = sphops::as_stream(stream);
+    void* host = nullptr;
+    if (host_counts != nullptr) SPHOPS_HIP(hipHostGetDevicePointer(&host, host_counts, 0));
+    if (grid->n_keys == 0) {
+      sphops::fill_u32(reinterpret_cast<uint32_t*>(counts), 6, 0u, st);
+      if (host != nullptr)
+        sphops::copy_words_to_host(reinterpret_cast<const uint32_t*>(counts), static_cast<uint32_t*>(host), 6, st);
+      return;
+    }
+    require(nbr_start != nullptr && nbr_count != nullptr && (nbr_index != nullptr || index_capacity == 0) &&
+                nbr_order != nullptr && nbr_waves != nullptr && nbr_waves_split != nullptr,
+            "null buffer");
+    OpPtrs a;
+    a.x = x;
+    a.iout3 = nbr_start;
+    a.iout = nbr_index;
+    a.iout2 = nbr_count;
+    a.cap = index_capacity;
+    sphops::forward(*grid, Op::NeighbourFill, bo, a, st);
+    const sphops::FillTail tail{reinterpret_cast<unsigned long long*>(counts),
+                                sphops::fill_stripes(grid->n_keys, index_capacity), static_cast<uint32_t*>(host)};
+    sphops::run_neighbour_schedule(*grid, nbr_count, nbr_order, reinterpret_cast<uint2*>(nbr_waves), counts + 4,
+                                   reinterpret_cast<uint2*>(nbr_waves_split), counts + 5, st, &tail);
+  });
+}
+
 int sphops_neighbor_fill(const sphops_grid* grid, const float* x, const int32_t* bo, int32_t* nbr_start,
                          int32_t* nbr_index, int64_t index_capacity, int32_t* nbr_count, int64_t* nbr_total,
                          void* stream) {
@@ -872,6 +909,122 @@ int sphops_perception_features_backward(int dim, const float* dz, const float* g
             "grad_rho must not be NULL");
     sphops::run_glue_backward(dim, dz, grad_s, grad_rho, d_s, d_blur, d_grad_s, d_grad_rho, (uint64_t)particles, C,
                               coef_s, coef_rho, total_mass, flags, sphops::as_stream(stream));
+  });
+}
+
+// The list of a perception call, as the operators take it.
+static OpPtrs perceive_ptrs(const sphops_perceive* p) {
+  OpPtrs a;
+  a.x = p->x_bin;
+  a.m = p->mass;
+  a.C = p->feature_dim;
+  a.nptr = p->nbr_start;
+  a.ncnt = p->nbr_count;
+  a.nidx = p->nbr_index;
+  a.order = p->nbr_order;
+  a.waves = reinterpret_cast<const uint2*>(p->nbr_waves);
+  a.nwaves = (uint32_t)std::max(p->nbr_wave_count, 0);
+  a.waves2 = reinterpret_cast<const uint2*>(p->nbr_waves_split);
+  a.nwaves2 = (uint32_t)std::max(p->nbr_wave_count_split, 0);
+  a.nwaves_dev = p->counts + 4;
+  a.nwaves2_dev = p->counts + 5;
+  return a;
+}
+
+static int check_perceive(const sphops_grid* grid, const sphops_perceive* p) {
+  return guarded([&] {
+    require(grid != nullptr && p != nullptr, "grid and p must not be NULL");
+    require(grid->n_keys > 0, "no particles");
+    sphops::check_channels(p->feature_dim);
+    const void* need[] = {p->mass, p->bin_offsets, p->x_bin, p->s_bin, p->nbr_start, p->nbr_count, p->nbr_index,
+                          p->nbr_order, p->nbr_waves, p->nbr_waves_split, p->counts, p->rho, p->grad_s, p->grad_rho};
+    for (const void* b : need) require(b != nullptr, "null buffer");
+    require(sphops::pk::aligned16(p->packed_mass) && sphops::pk::aligned16(p->packed_volume),
+            "packed records must be 16-byte aligned");
+  });
+}
+
+int sphops_perceive_forward(sphops_grid* grid, const sphops_perceive* p, void* stream) {
+  int st = check_perceive(grid, p);
+  if (st) return st;
+  st = sphops_initialize_inverse(grid, p->x, p->permutation, p->inverse, p->bin_offsets, p->block_info,
+                                 p->total_blocks, stream);
+  if (st) return st;
+  st = sphops_bin_particles(grid, p->x, p->s, nullptr, p->permutation, p->x_bin, p->s_bin, nullptr, p->feature_dim,
+                            stream);
+  if (st) return st;
+  st = sphops_neighbor_list(grid, p->x_bin, p->bin_offsets, 1, p->nbr_start, p->nbr_index, p->index_capacity,
+                            p->nbr_count, p->nbr_order, p->nbr_waves, p->nbr_waves_split, p->counts, p->host_counts,
+                            stream);
+  if (st) return st;
+  OpPtrs a = perceive_ptrs(p);
+  a.out0 = p->rho;
+  a.out3 = p->grad_rho;
+  a.xw_buf = reinterpret_cast<float4*>(p->packed_mass);
+  st = fwd_op(grid, Op::DensityPair, p->bin_offsets, a, stream);
+  if (st) return st;
+  a = perceive_ptrs(p);
+  a.rho = p->rho;
+  a.s = p->s_bin;
+  a.out0 = p->blur;
+  a.out3 = p->grad_s;
+  a.tol = p->tol;
+  a.xw_buf = reinterpret_cast<float4*>(p->packed_volume);
+  st = fwd_op(grid, Op::BlurGradientHybrid, p->bin_offsets, a, stream);
+  if (st) return st;
+  return sphops_perception_features_forward(grid->dim, p->s_bin, p->blur, p->grad_s, p->grad_rho, p->z,
+                                            (int64_t)grid->n_keys, p->feature_dim, p->coef_s, p->coef_rho,
+                                            p->total_mass, p->flags, stream);
+}
+
+int sphops_perceive_backward(const sphops_grid* grid, const sphops_perceive* p, const sphops_perceive_grads* d,
+                             void* stream) {
+  int st = check_perceive(grid, p);
+  if (st) return st;
+  st = guarded([&] {
+    require(d != nullptr, "d must not be NULL");
+    require(p->inverse != nullptr, "null buffer");
+    require(d->dz == nullptr || !(d->positions || d->state) ||
+                (d->d_blur && d->d_grad_s && d->g_s && (!d->state || d->d_s) &&
+                 (!d->positions || (d->d_grad_rho && d->g_x && d->g_x2 && d->g_rho))),
+            "null buffer");
+  });
+  if (st) return st;
+  const bool through = d->dz != nullptr && (d->positions || d->state);
+  if (through) {
+    st = sphops_perception_features_backward(grid->dim, d->dz, p->grad_s, p->grad_rho, d->state ? d->d_s : nullptr,
+                                             d->d_blur, d->d_grad_s, d->positions ? d->d_grad_rho : nullptr,
+                                             (int64_t)grid->n_keys, p->feature_dim, p->coef_s, p->coef_rho,
+                                             p->total_mass, p->flags, stream);
+    if (st) return st;
+    OpPtrs a = perceive_ptrs(p);
+    a.rho = p->rho;
+    a.s = p->s_bin;
+    a.g = d->d_blur;
+    a.g2 = d->d_grad_s;
+    a.out0 = d->positions ? d->g_x : nullptr;
+    a.out1 = d->g_s;
+    a.out2 = d->positions ? d->g_rho : nullptr;
+    a.xw_buf = reinterpret_cast<float4*>(p->packed_volume);
+    a.xw_ready = p->packed_volume != nullptr;
+    st = bwd_op(grid, Op::BlurGradientHybrid, d->positions != 0, p->bin_offsets, a, stream);
+    if (st) return st;
+    if (d->positions) {
+      a = perceive_ptrs(p);
+      a.g = d->g_rho;
+      a.g2 = d->d_grad_rho;
+      a.out0 = d->g_x2;
+      a.xw_buf = reinterpret_cast<float4*>(p->packed_mass);
+      a.xw_ready = p->packed_mass != nullptr;
+      st = bwd_op(grid, Op::DensityPair, true, p->bin_offsets, a, stream);
+      if (st) return st;
+    }
+  }
+  return guarded([&] {
+    const bool pos = through && d->positions, state = through && d->state;
+    const sphops::RowSum rows{{d->d_x_bin, pos ? d->g_x : nullptr, pos ? d->g_x2 : nullptr},
+                              {d->d_s_bin, state ? d->d_s : nullptr, state ? d->g_s : nullptr}};
+    sphops::run_unbin_sum(*grid, rows, p->inverse, d->grad_x, d->grad_s, p->feature_dim, sphops::as_stream(stream));
   });
 }
 

@@ -2186,44 +2186,11 @@ __global__ __launch_bounds__(kThreads) void k_fill(GridParams g, const float4* _
       g, xw, bo, unit_len, units, nunits, mine, nidx, nstart, ncnt, fs, ft);
 }
 
-// total[0] = in-radius pairs (blocks written or not), total[1] = pairs of
-// the blocks not written, from the counters' words (see FillStripes); the
-// counters, and the unit queues of all kFillStripes stripes, are then reset
-// to zero for the next fill.  One workgroup of
-// kThreads >= kFillStripes.
-static_assert(kThreads >= kFillStripes, "k_fill_totals reads one counter per thread");
+static_assert(kFillStripes == 256 && kStripeWords == 32 && kUnitQueueWord == 16, "as fill_totals reads them");
 [[maybe_unused]] static __global__ __launch_bounds__(kThreads) void k_fill_totals(unsigned long long* __restrict__ ctr,
                                                                  uint32_t stripes,
                                                                  unsigned long long* __restrict__ total) {
-  __shared__ unsigned long long part[2][kThreads / kWave];
-  const uint32_t s = threadIdx.x;
-  unsigned long long a = 0, o = 0;
-  if (s < stripes) {
-    unsigned long long* c = ctr + (uint64_t)s * kStripeWords;
-    a = c[0] - c[1] + c[2];
-    o = c[2];
-    c[0] = c[1] = c[2] = 0ull;
-  }
-  if (s < kFillStripes) ctr[(uint64_t)s * kStripeWords + kUnitQueueWord] = 0ull;  // the fill's unit queues
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    a += __shfl_down(a, off, kWave);
-    o += __shfl_down(o, off, kWave);
-  }
-  if (__lane_id() == 0) {
-    part[0][s / kWave] = a;
-    part[1][s / kWave] = o;
-  }
-  __syncthreads();
-  if (s == 0) {
-    unsigned long long sa = 0, so = 0;
-    for (uint32_t w = 0; w < kThreads / kWave; ++w) {
-      sa += part[0][w];
-      so += part[1][w];
-    }
-    total[0] = sa;
-    total[1] = so;
-  }
+  fill_totals(ctr, stripes, total);
 }
 
 
@@ -2291,13 +2258,7 @@ void neighbour_fill(const Grid& g, const int32_t* bo, const float* x, int32_t* n
     SPHOPS_LAUNCHED();
     xw = g.packed;
   }
-  // S slices of at least kStripeMinEntries entries and, for n particles,
-  // about n / (kStripeMinUnits * kUnitParticles) units or more each (one
-  // slice for small buffers)
-  uint32_t S = 1;
-  while (S < kFillStripes && (int64_t)(2 * S) * kStripeMinEntries <= cap &&
-         (uint64_t)(2 * S) * kStripeMinUnits * kUnitParticles <= n)
-    S *= 2;
+  const uint32_t S = fill_stripes(n, cap);
   // the counters are zero here: zeroed at grid creation and by the totals
   // kernel of every fill
   FillStripes fs{g.stripes, S - 1, (uint64_t)(cap / S)};
@@ -2315,8 +2276,10 @@ void neighbour_fill(const Grid& g, const int32_t* bo, const float* x, int32_t* n
   }
 #undef SPHOPS_FILL
   SPHOPS_LAUNCHED();
-  hipLaunchKernelGGL(k_fill_totals, dim3(1), dim3(kThreads), 0, st, g.stripes, S, used);
-  SPHOPS_LAUNCHED();
+  if (used != nullptr) {  // else the schedule's first kernel takes them
+    hipLaunchKernelGGL(k_fill_totals, dim3(1), dim3(kThreads), 0, st, g.stripes, S, used);
+    SPHOPS_LAUNCHED();
+  }
 }
 
 // Workgroups for a schedule of `waves` waves, rounded up to a multiple of 8

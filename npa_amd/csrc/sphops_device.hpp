@@ -234,4 +234,41 @@ __device__ __forceinline__ uint32_t xcd_block_id_chunked(uint32_t nb_live) {
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
+// Totals of the list fill's row-allocation counters, by one workgroup of at
+// least 256 threads (a barrier inside): total[0] = in-radius pairs (blocks
+// written or not), total[1] = pairs of the blocks not written.  Counter words
+// (a 256-byte record of 32 64-bit words per stripe): [0] entries taken (a
+// failed attempt's block included), [1] entries of failed attempts, [2]
+// entries of blocks not written, [16] the stripe's unit queue; all are reset
+// to zero for the next fill.
+__device__ __forceinline__ void fill_totals(unsigned long long* __restrict__ ctr, uint32_t stripes,
+                                            unsigned long long* __restrict__ total) {
+  __shared__ unsigned long long part[2][4];
+  const uint32_t s = threadIdx.x;
+  if (s < 256u) {
+    unsigned long long* c = ctr + (uint64_t)s * 32u;
+    unsigned long long a = 0, o = 0;
+    if (s < stripes) {
+      a = c[0] - c[1] + c[2];
+      o = c[2];
+      c[0] = c[1] = c[2] = 0ull;
+    }
+    c[16] = 0ull;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      a += __shfl_down(a, off, 64);
+      o += __shfl_down(o, off, 64);
+    }
+    if (__lane_id() == 0) {
+      part[0][s / 64] = a;
+      part[1][s / 64] = o;
+    }
+  }
+  __syncthreads();
+  if (s == 0) {
+    total[0] = part[0][0] + part[0][1] + part[0][2] + part[0][3];
+    total[1] = part[1][0] + part[1][1] + part[1][2] + part[1][3];
+  }
+}
+
 }  // namespace sphops

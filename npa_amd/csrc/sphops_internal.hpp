@@ -72,6 +72,15 @@ void run_instantiate(Grid& g, const float* pos, int32_t* perm, int32_t* bin_offs
 void run_bin_particles(const Grid& g, const float* in_pos, const float* in_state, const float* in_mass,
                        const int32_t* perm, float* out_pos, float* out_state, float* out_mass,
                        uint32_t C, bool forward, hipStream_t st);
+// Rows back to input order, out[b, inv[b, k]] = the sum of the given rows at
+// binned slot k (up to three state and position sources; null ones are left
+// out, in this order of summation).
+struct RowSum {
+  const float* x[3];
+  const float* s[3];
+};
+void run_unbin_sum(const Grid& g, const RowSum& in, const int32_t* inv, float* out_pos, float* out_state, uint32_t C,
+                   hipStream_t st);
 // Words of partial sums a device scan of n words needs (every recursion
 // level padded to a tile of 4096).
 constexpr uint64_t kScanTile = 4096;
@@ -183,8 +192,17 @@ void run_backward(const Grid& g, Op op, bool full, const int32_t* bin_offsets, c
 // Pair-kernel schedule: per tile of 4096 binned particles, a stable partition
 // by neighbour-list length class (kListClasses / kListGroups), tiles in
 // order; one descriptor per wave {first slot in order, group size << 8 | particles}.
+// With `tail` the schedule's kernels also finish the fill before them: its
+// pair totals go to tail->total (the first kernel, see fill_totals), and,
+// with tail->host, total, wave_total and wave_total2 (words 0-3, 4 and 5) to
+// pinned host memory (the second).
+struct FillTail {
+  unsigned long long* total;
+  uint32_t stripes;
+  uint32_t* host;  // device view of the pinned words, or null
+};
 void run_neighbour_schedule(const Grid& g, const int32_t* ncnt, int32_t* order, uint2* waves, int32_t* wave_total,
-                            uint2* waves2, int32_t* wave_total2, hipStream_t st);
+                            uint2* waves2, int32_t* wave_total2, hipStream_t st, const FillTail* tail = nullptr);
 // The split-group schedule alone (kSplitGroups) over lengths `len`; items of
 // negative length are left out.
 void run_split_schedule(const Grid& g, const int32_t* len, int32_t* order, uint2* waves, int32_t* wave_total,
@@ -216,6 +234,16 @@ constexpr uint32_t kStripeWords = 32;
 constexpr uint32_t kUnitQueueWord = 16;
 constexpr int64_t kStripeMinEntries = (int64_t)1 << 15;
 constexpr uint64_t kStripeMinUnits = 64;
+// Stripes a fill of n particles into `cap` entries uses: slices of at least
+// kStripeMinEntries entries and about n / (kStripeMinUnits * kUnitParticles)
+// units or more each (one slice for small buffers).
+inline uint32_t fill_stripes(uint64_t n, int64_t cap) {
+  uint32_t S = 1;
+  while (S < kFillStripes && (int64_t)(2 * S) * kStripeMinEntries <= cap &&
+         (uint64_t)(2 * S) * kStripeMinUnits * kUnitParticles <= n)
+    S *= 2;
+  return S;
+}
 // Work classes of the list traversal: class q holds
 // the items whose length is <= t[q] (and above the previous bound), the last
 // class the rest; each class is served by groups of g[q] lanes per particle

@@ -8,7 +8,9 @@ their pass fusion applies); the features the reference then assembles with
 torch elementwise ops and ``torch.cat`` (the eps/eps0 scaling, the
 log-normalisation of models/npa.py:83-85, the density-gradient scaling by
 coef^(1+D)/N) are built by one HIP kernel, and their gradient by another
-(``sphops_perception_features_forward`` / ``_backward``).
+(``sphops_perception_features_forward`` / ``_backward``).  With the state and
+density gradients on, the whole sequence is one native call each way
+(``Perceive``).
 
 Difference from the reference: its density-gradient branch uses ``coef``,
 which it defines only in the state-gradient branch (models/npa.py:121-127), so
@@ -20,7 +22,7 @@ import ctypes
 import numpy as np
 import torch
 
-from .sphops import _native
+from .sphops import _native, sph
 from .sphops import bin_particles, blur, density, density_gradient, gradient_hybrid
 
 _lib = _native.lib
@@ -90,6 +92,127 @@ class PerceptionFeatures(torch.autograd.Function):
         return d_s, d_blur, d_gs, d_gr, None, None, None, None, None
 
 
+class Perceive(torch.autograd.Function):
+    """(z, x_bin, s_bin) of NPA.perceive with both gradients on, one native
+    call each way (``sphops_perceive_forward`` / ``_backward``): the calls of
+    the general path in its order, without the Python between them, and with
+    the gradients that meet at x and s summed as they are unbinned.  ``out``
+    receives the snapshot, whose neighbour list later operators reuse."""
+
+    @staticmethod
+    def forward(ctx, x, s, grid, args, stop_pos, stop_state, out):
+        B, N, P = x.shape
+        C, D, dev, hg = s.shape[2], grid.dim, x.device, grid.hashgrid
+        n = B * N
+        flags, coef_s, coef_rho, total_mass = args
+        # whether z's gradient flows to x and to s
+        pos = ctx.needs_input_grad[0] and not stop_pos
+        state = ctx.needs_input_grad[1] and not stop_state
+        snap = grid._new_snapshot(dev)
+        x_bin, s_bin = torch.empty_like(x), torch.empty_like(s)
+        z = torch.empty(B, N, feature_width(C, D, flags), dtype=torch.float32, device=dev)
+        # what the backward reads in one buffer of 16-byte aligned pieces: rho,
+        # both gradients and the (x, weight) records
+        pad = (n + 3) & ~3
+        grads = pos or state
+        sizes = [pad, pad * C * D, pad * D, 4 * n if grads else 0, 4 * n if pos else 0]
+        blur_s = torch.empty_like(s)
+        work = torch.empty(sum(sizes), dtype=torch.float32, device=dev)
+        at, ptrs = work.data_ptr(), []
+        for k in sizes:
+            ptrs.append(at if k else None)
+            at += 4 * k
+        mass = sph._default_mass(x, None)
+        a = _native.Perceive()
+        a.x, a.s, a.mass = x.data_ptr(), s.data_ptr(), mass.data_ptr()
+        a.permutation, a.inverse = snap.permutation.data_ptr(), snap.inverse.data_ptr()
+        a.bin_offsets, a.total_blocks = snap.bin_offsets.data_ptr(), snap.total_blocks.data_ptr()
+        a.block_info = snap.block_info.data_ptr()
+        a.x_bin, a.s_bin, a.z = x_bin.data_ptr(), s_bin.data_ptr(), z.data_ptr()
+        a.rho, a.grad_s, a.grad_rho, a.packed_volume, a.packed_mass = ptrs
+        a.blur = blur_s.data_ptr()
+        a.feature_dim, a.flags, a.tol = C, flags, 1e-3
+        a.coef_s, a.coef_rho, a.total_mass = coef_s, coef_rho, total_mass
+        plan = hg._perceive(a, x, snap.bin_offsets)
+        snap.inverse_versions = (snap.permutation._version, snap.inverse._version)
+        snap.plan = (x_bin.detach(), x_bin.data_ptr(), x_bin._version, tuple(x_bin.shape), plan)
+        out.append(snap)
+        if stop_pos and stop_state:
+            ctx.mark_non_differentiable(z)
+        ctx.set_materialize_grads(False)
+        if any(ctx.needs_input_grad):
+            if grads:
+                ctx.save_for_backward(x_bin, s_bin, mass, work)
+            ctx.snapshot, ctx.pos, ctx.state, ctx.sizes, ctx.args = snap, pos, state, sizes, args
+            ctx.shapes, ctx.device = (x.shape, s.shape), dev
+        return z, x_bin, s_bin
+
+    @staticmethod
+    def backward(ctx, dz, dx_bin, ds_bin):
+        need_x, need_s = ctx.needs_input_grad[:2]
+        snap, dev = ctx.snapshot, ctx.device
+        (B, N, P), (_, _, C) = ctx.shapes
+        through = dz is not None and (ctx.pos or ctx.state)
+        ups = [None if t is None else t.contiguous() for t in (dz if through else None, dx_bin, ds_bin)]
+        for t in ups:
+            if t is not None and (t.dtype != torch.float32 or t.device != dev):
+                raise TypeError("perceive's gradients must be float32 on the inputs' device")
+        if not through:  # only the binning was differentiated
+            dx, ds = (torch.zeros(shape, device=dev) if t is None else t for t, shape in zip(ups[1:], ctx.shapes))
+            grad_x, grad_s = torch.empty_like(dx), torch.empty_like(ds)
+            sph._unbin(snap, dx, ds, None, grad_x, grad_s, None)
+            return (grad_x if need_x else None, grad_s if need_s else None) + (None,) * 5
+        x_bin, s_bin, mass, work = ctx.saved_tensors
+        n, D = B * N, snap.dim
+        # a permutation modified since the step: rows summed in binned order,
+        # then gathered by it, as the operators' own backward does
+        binned = snap.inverse_versions != (snap.permutation._version, snap.inverse._version)
+        inverse = (torch.arange(N, dtype=torch.int32, device=dev).repeat(B, 1) if binned else snap.inverse)
+        grad_x = torch.empty_like(x_bin) if need_x or binned else None
+        grad_s = torch.empty_like(s_bin) if need_s or binned else None
+        a, d = _native.Perceive(), _native.PerceiveGrads()
+        a.mass, a.x_bin, a.s_bin = mass.data_ptr(), x_bin.data_ptr(), s_bin.data_ptr()
+        a.bin_offsets, a.inverse = snap.bin_offsets.data_ptr(), inverse.data_ptr()
+        plan = sph._plan(snap, x_bin)
+        snap.grid._set_list(a, plan)
+        flags, a.coef_s, a.coef_rho, a.total_mass = ctx.args
+        a.feature_dim, a.flags = C, flags
+        at, ptrs = work.data_ptr(), []
+        for k in ctx.sizes:
+            ptrs.append(at if k else None)
+            at += 4 * k
+        a.rho, a.grad_s, a.grad_rho, a.packed_volume, a.packed_mass = ptrs
+        d.dz, d.d_x_bin, d.d_s_bin = (None if t is None else t.data_ptr() for t in ups)
+        d.positions, d.state = int(ctx.pos), int(ctx.state)
+        pad = (n + 3) & ~3
+        sizes = [pad * C, pad * C, pad * C * D, pad * C] + ([pad * D, P * pad, P * pad, pad] if ctx.pos else [])
+        scratch = torch.empty(sum(sizes), dtype=torch.float32, device=dev)
+        at = scratch.data_ptr()
+        for name, k in zip(("d_s", "d_blur", "d_grad_s", "g_s", "d_grad_rho", "g_x", "g_x2", "g_rho"), sizes):
+            setattr(d, name, at)
+            at += 4 * k
+        d.grad_x = None if grad_x is None else grad_x.data_ptr()
+        d.grad_s = None if grad_s is None else grad_s.data_ptr()
+        _native.check(_lib.sphops_perceive_backward(snap.grid._h, ctypes.byref(a), ctypes.byref(d), _stream(x_bin)))
+        if binned:
+            out = torch.empty_like(grad_x), torch.empty_like(grad_s)
+            snap.grid.backward_bin_particles(grad_x, grad_s, None, snap.permutation, out[0], out[1], None)
+            grad_x, grad_s = out
+        return (grad_x if need_x else None, grad_s if need_s else None) + (None,) * 5
+
+
+def _native_ok(x, s, grid):
+    """What ``Perceive`` takes: dense float32 GPU tensors of the grid's shape
+    (anything else goes to the operators, which raise or handle it), the
+    default lists, and pass fusion on (``NPA_SPHOPS_FUSE``)."""
+    hg = grid.hashgrid
+    return (sph._PASS_A.enabled and sph._PASS_B.enabled and not hg.tiles_enabled and not hg._cells_wanted()
+            and isinstance(x, torch.Tensor) and x.dtype == s.dtype == torch.float32 and x.is_cuda
+            and x.device == s.device and x.dim() == s.dim() == 3 and x.is_contiguous() and s.is_contiguous()
+            and x.shape == (hg._b, hg._n, hg._pw) and s.shape[:2] == x.shape[:2] and 1 <= s.shape[2] <= 64
+            and x.numel() > 0 and x.data_ptr() % 16 == 0)
+
+
 def perceive(x, s, grid, eps0=0.1, state_grad=True, density_grad=True, log_norm_grad=True,
              log_norm_density_grad=True, stopgrad_pos=True, stopgrad_state=False):
     """NPA.perceive (models/npa.py:87-137) with the NPA constructor's flags
@@ -97,6 +220,19 @@ def perceive(x, s, grid, eps0=0.1, state_grad=True, density_grad=True, log_norm_
     Returns (z, x_bin, s_bin, snapshot), z of width 2C (+ C*D) (+ D)."""
     B, N, C = s.shape
     D = grid.dim
+    # coef = eps / eps0 and coef ** (1 + D) rounded as torch evaluates them on
+    # the model's fp32 buffer: a Python float over a tensor is the tensor's
+    # reciprocal times the float; the cube is c * c * c, other powers powf
+    e0 = buffer_value(eps0)
+    coef = np.float32(np.float32(1.0) / np.float32(e0)) * np.float32(grid.eps)
+    coef_rho = coef * coef * coef if D == 2 else np.power(coef, np.float32(1 + D))
+    if state_grad and density_grad and _native_ok(x, s, grid):
+        flags = (STATE_GRAD | (LOG_NORM_GRAD if log_norm_grad else 0)
+                 | DENSITY_GRAD | (LOG_NORM_DENSITY_GRAD if log_norm_density_grad else 0))
+        out = []
+        z, x_bin, s_bin = Perceive.apply(x, s, grid, (flags, float(coef), float(coef_rho), float(N)), stopgrad_pos,
+                                         stopgrad_state, out)
+        return z, x_bin, s_bin, out[0]
     with torch.no_grad():
         snapshot = grid.instantiate(x)
     x_bin, s_bin = bin_particles(x, s, snapshot)
@@ -104,12 +240,6 @@ def perceive(x, s, grid, eps0=0.1, state_grad=True, density_grad=True, log_norm_
     s_p = s_bin.detach() if stopgrad_state else s_bin
     rho = density(x_p, snapshot)
     blur_s = blur(x_p, rho, s_p, snapshot)
-    # coef = eps / eps0 and coef ** (1 + D) rounded as torch evaluates them on
-    # the model's fp32 buffer: a Python float over a tensor is the tensor's
-    # reciprocal times the float; the cube is c * c * c, other powers powf
-    e0 = buffer_value(eps0)
-    coef = np.float32(np.float32(1.0) / np.float32(e0)) * np.float32(grid.eps)
-    coef_rho = coef * coef * coef if D == 2 else np.power(coef, np.float32(1 + D))
     flags = 0
     grad_s = grad_rho = None
     if state_grad:

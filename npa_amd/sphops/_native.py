@@ -10,7 +10,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get(
     "SPHOPS_HIP_LIB", os.path.join(os.path.dirname(_HERE), "_lib", "libsphops_hip.so"))
-ABI_VERSION = 22
+ABI_VERSION = 23
 
 if not os.path.exists(LIB_PATH):
     raise ImportError(
@@ -79,6 +79,9 @@ _SIGNATURES = {
     "sphops_backward": ([_p, _i32, _i32, _i32, _i32, _p, _p], _i32),
     "sphops_neighbor_candidates": ([_p, _p, _p, _i32, _p], _i32),
     "sphops_copy_words_to_host": ([_p, _p, _u32, _p], _i32),
+    "sphops_neighbor_list": ([_p, _p, _p, _i32, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _p], _i32),
+    "sphops_perceive_forward": ([_p, _p, _p], _i32),
+    "sphops_perceive_backward": ([_p, _p, _p, _p], _i32),
     "sphops_neighbor_fill": ([_p, _p, _p, _p, _p, _i64, _p, _p, _p], _i32),
     "sphops_neighbor_fill_tiled": ([_p, _p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _p], _i32),
     "sphops_neighbor_cell_capacity": ([_p], _i64),
@@ -101,6 +104,25 @@ class Args(ctypes.Structure):
                 ("nbr_wave_count_sparse", ctypes.c_int32), ("nbr_wave_count_sparse_device", _p),
                 ("packed", _p), ("packed_valid", ctypes.c_int32), ("nbr_own", _p), ("cells", _p),
                 ("cell_count", _p)]
+
+
+class Perceive(ctypes.Structure):
+    """``sphops_perceive`` (include/sphops_hip.h)."""
+    _fields_ = [("x", _p), ("s", _p), ("mass", _p), ("permutation", _p), ("inverse", _p), ("bin_offsets", _p),
+                ("block_info", _p), ("total_blocks", _p), ("x_bin", _p), ("s_bin", _p), ("nbr_start", _p),
+                ("nbr_count", _p), ("nbr_index", _p), ("index_capacity", _i64), ("nbr_order", _p),
+                ("nbr_waves", _p), ("nbr_waves_split", _p), ("nbr_wave_count", ctypes.c_int32),
+                ("nbr_wave_count_split", ctypes.c_int32), ("counts", _p), ("host_counts", _p), ("rho", _p),
+                ("grad_rho", _p), ("blur", _p), ("grad_s", _p), ("packed_mass", _p), ("packed_volume", _p),
+                ("z", _p), ("feature_dim", _u32), ("flags", ctypes.c_int32), ("tol", _f32), ("coef_s", _f32),
+                ("coef_rho", _f32), ("total_mass", _f32)]
+
+
+class PerceiveGrads(ctypes.Structure):
+    """``sphops_perceive_grads`` (include/sphops_hip.h)."""
+    _fields_ = [("dz", _p), ("d_x_bin", _p), ("d_s_bin", _p), ("positions", ctypes.c_int32),
+                ("state", ctypes.c_int32), ("d_s", _p), ("d_blur", _p), ("d_grad_s", _p), ("d_grad_rho", _p),
+                ("g_s", _p), ("g_x", _p), ("g_x2", _p), ("g_rho", _p), ("grad_x", _p), ("grad_s", _p)]
 
 
 (OP_COUNT, OP_DENSITY, OP_DENSITY_GRADIENT, OP_MOMENT_MATRIX, OP_BLUR, OP_GRADIENT, OP_GRADIENT_HYBRID,

@@ -105,16 +105,22 @@ class HashGrid:
     def instantiate(self, x):
         """Bin positions ``x`` (B, N, 2|4) and return the snapshot."""
         B, N, _ = x.shape
-        dev = x.device
+        snap = self._new_snapshot(x.device, B, N)
+        self.hashgrid.initialize(x, snap.permutation, snap.bin_offsets, snap.block_info, snap.total_blocks,
+                                 inverse=snap.inverse)
+        snap.inverse_versions = (snap.permutation._version, snap.inverse._version)
+        return snap
+
+    def _new_snapshot(self, dev, B=None, N=None):
+        """A snapshot's buffers, not yet written."""
+        B, N = (self.batch_size, self.num_particles) if B is None else (B, N)
         permutation = torch.empty(B, N, dtype=torch.int32, device=dev)
         bin_offsets = torch.empty(B * self.num_cells + 1, dtype=torch.int32, device=dev)
         block_info = torch.empty(self.hashgrid.max_blocks, 4, dtype=torch.int32, device=dev)
         total_blocks = torch.empty(1, dtype=torch.int32, device=dev)
         inverse = torch.empty(B, N, dtype=torch.int32, device=dev)
-        self.hashgrid.initialize(x, permutation, bin_offsets, block_info, total_blocks, inverse=inverse)
         return HashGridSnapshot(grid=self.hashgrid, bin_offsets=bin_offsets, permutation=permutation,
-                                block_info=block_info, dim=self.dim, total_blocks=total_blocks,
-                                inverse=inverse, inverse_versions=(permutation._version, inverse._version))
+                                block_info=block_info, dim=self.dim, total_blocks=total_blocks, inverse=inverse)
 
     def set_capture_capacity(self, index_capacity):
         """Fix the buffer and launch sizes of neighbour lists so that a step

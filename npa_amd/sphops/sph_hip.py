@@ -423,6 +423,16 @@ class _HashGridNative:
         tiles = self._tile_buffers(dev, n, wcap) if self.tiles_enabled else None
         src = getattr(self, "_split_source", None)
         reuse = src is not None and src[0]() is bin_offsets and bin_offsets._version == src[1]
+        if tiles is None and not self._cells_wanted():
+            # the whole build in one call, its totals into the pinned words
+            host = None if capturing else self._readback_buffer()
+            _check(_lib.sphops_neighbor_list(
+                self._h, x, bo, 1 if reuse else 0, start.data_ptr(), index.data_ptr(), cap, count.data_ptr(),
+                order.data_ptr(), waves.data_ptr(), waves2.data_ptr(), small.data_ptr(),
+                None if host is None else host.data_ptr(), st))
+            if host is not None:
+                self._readback_started(cap, False)
+            return self._new_plan(n, start, count, index, order, waves, waves2, small, cap)
         _check(_lib.sphops_neighbor_candidates(self._h, x, bo, 1 if reuse else 0, st))
         cells = None
         if tiles is None and self._cells_wanted():
@@ -461,6 +471,47 @@ class _HashGridNative:
         self._last_plan = plan
         return plan
 
+    def _new_plan(self, n, start, count, index, order, waves, waves2, small, cap):
+        e1, e2, _ = self._wave_estimates(n)
+        plan = NeighborPlan(start, count, index, order, waves, e1, waves2, e2, small)
+        plan.capacity = cap
+        self._last_plan = plan
+        return plan
+
+    def _perceive(self, a, x, bin_offsets):
+        """``sphops_perceive_forward`` on arguments filled but for the
+        neighbour list, whose buffers are allocated here as ``neighbor_list``
+        does; returns the list."""
+        dev, n = x.device, self._b * self._n
+        capturing = torch.cuda.is_current_stream_capturing()
+        if not capturing:
+            self._consume_readback()
+        wcap = 2 * max(int(_lib.sphops_neighbor_wave_capacity(self._h)), 1)
+        cap = self._capacity(n)
+        start, count, order = (torch.empty(n, dtype=_I32, device=dev) for _ in range(3))
+        waves, waves2 = (torch.empty(wcap, dtype=_I32, device=dev) for _ in range(2))
+        small = torch.empty(9, dtype=_I32, device=dev)
+        index = torch.empty(max(cap, 1), dtype=_I32, device=dev)
+        plan = self._new_plan(n, start, count, index, order, waves, waves2, small, cap)
+        self._set_list(a, plan)
+        host = None if capturing else self._readback_buffer()
+        a.host_counts = None if host is None else host.data_ptr()
+        _check(_lib.sphops_perceive_forward(self._h, ctypes.byref(a), _stream(x)))
+        if host is not None:
+            self._readback_started(cap, False)
+        # as after initialize(): the work split of the list fill is this snapshot's
+        self._split_source = (weakref.ref(bin_offsets), bin_offsets._version)
+        return plan
+
+    @staticmethod
+    def _set_list(a, plan):
+        start, count, index, order, waves, e1, waves2, e2, small = plan
+        a.nbr_start, a.nbr_count, a.nbr_index = start.data_ptr(), count.data_ptr(), index.data_ptr()
+        a.index_capacity, a.nbr_order = plan.capacity, order.data_ptr()
+        a.nbr_waves, a.nbr_wave_count = waves.data_ptr(), e1
+        a.nbr_waves_split, a.nbr_wave_count_split = waves2.data_ptr(), e2
+        a.counts = small.data_ptr()
+
     # Largest index buffer (entries) a snapshot allocates; rows that do not
     # fit are walked on the stencil instead.  At most 2^30 (the library's
     # limit).
@@ -493,20 +544,29 @@ class _HashGridNative:
     # its buffer held the total, i.e. the fill's slices were uneven.
     _slack_shift = 3
 
-    def _start_readback(self, small, cap, tiles):
-        """Copy the device counts to pinned host memory without waiting
-        (the tile counts are valid only for a plan with tiles)."""
+    def _readback_buffer(self):
+        """Pinned words that receive a list's totals and wave counts."""
         rb = getattr(self, "_rb", None)
         if rb is None:
             self._rb = rb = torch.empty(8, dtype=_I32, pin_memory=True)
-        # a small kernel writes them into the pinned buffer (no copy-engine
-        # transfer on the stream)
-        _check(_lib.sphops_copy_words_to_host(ctypes.c_void_p(small.data_ptr()), ctypes.c_void_p(rb.data_ptr()), 8,
-                                              _stream(small)))
+        return rb
+
+    def _readback_started(self, cap, tiles):
+        """Note the read-back enqueued on the current stream (the tile counts
+        are valid only for a plan with tiles)."""
         self._rb_cap = cap
         self._rb_tiles = tiles
         self._rb_event = torch.cuda.Event()
         self._rb_event.record()
+
+    def _start_readback(self, small, cap, tiles):
+        """Copy the device counts to pinned host memory without waiting: a
+        small kernel writes them there (no copy-engine transfer on the
+        stream)."""
+        rb = self._readback_buffer()
+        _check(_lib.sphops_copy_words_to_host(ctypes.c_void_p(small.data_ptr()), ctypes.c_void_p(rb.data_ptr()), 8,
+                                              _stream(small)))
+        self._readback_started(cap, tiles)
 
     def _consume_readback(self, wait=False):
         """Take the counts of an earlier snapshot once they have arrived

@@ -1,0 +1,111 @@
+"""npa_amd.perceive's one-call path (Perceive) against the operators called one
+by one, over dimensions, boundaries, modes, channel counts, the stop-gradient
+and normalisation flags, the inputs that require a gradient and the outputs
+that receive one.  The forward runs the same kernels: bit for bit.  A gradient
+is a sum of at most three terms, which the two paths add in another order:
+within 2^-22 of the sum of their magnitudes, taken as eight times the larger of
+the value and the tensor's root mean square (their scale here)."""
+import pytest
+import torch
+
+import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+GRIDS = [(2, False, "grid", 16), (2, True, "grid", 12), (3, False, "particle", 5), (3, True, "grid", 20),
+         (3, False, "grid", 32)]
+
+
+def _grid(dim, per, mode, C, B=2, N=301):
+    import npa_amd.sphops as sp
+    c = H.random_case("p", B, N, C, dim, 8, 0.25, per, mode, seed=dim + C)
+    grid = sp.HashGrid(dim=dim, boundary="periodic" if per else "clamped", mode=mode, grid_size=list(c.grid_size),
+                       eps=c.eps, num_particles=N, batch_size=B, max_particles_per_block=c.maxp)
+    return grid, torch.from_numpy(c.x).cuda(), torch.from_numpy(c.s).cuda()
+
+
+def _both(monkeypatch, call):
+    from npa_amd import perceive as PF
+    got = call()
+    monkeypatch.setattr(PF, "_native_ok", lambda *a: False)
+    call()  # the grid learns the pass pairs: the fused kernels from here on
+    ref = call()
+    monkeypatch.undo()
+    return got, ref
+
+
+def _close(a, b):
+    if b is None:
+        assert a is None
+        return
+    rms = b.double().pow(2).mean().sqrt()
+    assert torch.all((a.double() - b.double()).abs() <= 2.0 ** -22 * 8 * (b.double().abs() + rms))
+
+
+@pytest.mark.parametrize("dim,per,mode,C", GRIDS)
+@pytest.mark.parametrize("stop_pos,stop_state", [(True, False), (False, False), (False, True), (True, True)])
+def test_perceive_matches_operators(monkeypatch, dim, per, mode, C, stop_pos, stop_state):
+    from npa_amd import perceive as PF
+    grid, x, s = _grid(dim, per, mode, C)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    W = PF.feature_width(C, dim, PF.STATE_GRAD | PF.DENSITY_GRAD)
+    ups = [torch.randn(2, 301, k, device="cuda", generator=g) for k in (W, x.shape[2], C)]
+    for which in ((0, 1, 2), (0,), (1, 2), (2,)):
+        for need in ((True, True), (False, True), (True, False)):
+            def call():
+                xr, sr = (t.clone().requires_grad_(r) for t, r in zip((x, s), need))
+                z, xb, sb, snap = PF.perceive(xr, sr, grid, 0.1, log_norm_grad=C != 12, log_norm_density_grad=C != 5,
+                                              stopgrad_pos=stop_pos, stopgrad_state=stop_state)
+                outs = (z, xb, sb)
+                live = [i for i in which if outs[i].requires_grad]
+                if live:
+                    torch.autograd.backward([outs[i] for i in live], [ups[i] for i in live])
+                return [t.detach() for t in outs], [t.requires_grad for t in outs], snap, (xr.grad, sr.grad)
+            (fo, fr, fs, fg), (ro, rr, rs, rg) = _both(monkeypatch, call)
+            assert fr == rr
+            assert all(torch.equal(a, b) for a, b in zip(fo, ro))
+            for k in ("permutation", "inverse", "bin_offsets", "block_info", "total_blocks"):
+                if k != "block_info" or mode == "grid":
+                    assert torch.equal(getattr(fs, k), getattr(rs, k)), k
+            for a, b in zip(fg, rg):
+                _close(a, b)
+
+
+def test_snapshot_and_list_serve_later_operators():
+    """The returned snapshot's list is reused by the operators; a permutation
+    modified in place makes the backward gather by it, as the operators do."""
+    import npa_amd.sphops as sp
+    from npa_amd import perceive as PF
+    grid, x, s = _grid(3, False, "grid", 16)
+    with torch.no_grad():
+        z, xb, sb, snap = PF.perceive(x, s, grid, 0.1)
+        plan = snap.plan[4]
+        rho = sp.density(xb, snap)
+        assert snap.plan[4] is plan and torch.equal(sb, z[..., :16])
+        assert torch.equal(sp.blur(xb, rho, sb, snap), sp.blur(xb, rho, sb, grid.instantiate(x)))
+    grads = []
+    for touch in (False, True):
+        sr = s.clone().requires_grad_(True)
+        z, _, _, snap = PF.perceive(x, sr, grid, 0.1)
+        if touch:
+            snap.permutation.add_(0)
+        z.square().sum().backward()
+        grads.append(sr.grad)
+    assert torch.equal(*grads)
+
+
+def test_overflowing_list_walks_the_stencil():
+    """A list without room for its rows: the same features and gradients to
+    rounding (sums of at most 70 terms, in another order)."""
+    from npa_amd import perceive as PF
+    grid, x, s = _grid(2, False, "grid", 16)
+    outs = []
+    for cap in (0, 7):
+        grid.set_capture_capacity(cap)
+        sr = s.clone().requires_grad_(True)
+        z, _, _, _ = PF.perceive(x, sr, grid, 0.1)
+        z.sum().backward()
+        outs.append((z.detach(), sr.grad))
+        assert grid.list_overflow() == (cap == 7)
+    for a, b in zip(*outs):
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-4 * b.abs().max().item())
