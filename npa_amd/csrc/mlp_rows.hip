@@ -29,7 +29,8 @@
 // traffic for each of the first two.  Measured inside a training step: 0.30 +
 // 0.28 + 0.36 ms, where the separate kernels took 0.51 (library product,
 // ReLU + second layer), 0.66 (its input gradient, library product) and 0.39;
-// forward and backward back to back 1.54 -> 0.95 ms.
+// forward and backward back to back 1.54 -> 0.91 ms (0.95 with the next row
+// tile's operands loaded under the second product only).
 #include "sphops_internal.hpp"
 #include "sphops_device.hpp"
 
@@ -170,15 +171,24 @@ __global__ __launch_bounds__(forward_threads(G), 2) void k_mlp_forward(const flo
 
   const int64_t step = (int64_t)gridDim.x * (kThreads / 64);
   int64_t tile = (int64_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kThreads / 64) + threadIdx.x / 64));
-  f32x4 zv[G];
+  // the next row tile's z is loaded while this one computes: all along, into
+  // registers of its own, where they fit (kAhead), else under the second
+  // product
+  constexpr bool kAhead = G <= 11;
+  f32x4 zv[G], zn[kAhead ? G : 1];
   const RowLoad<G> rl(nin, c, h);
-  auto load = [&](int64_t t) {
+  auto load = [&](int64_t t, f32x4 (&v)[G]) {
     const int64_t r0 = t * kT, nr = t < tiles ? min<int64_t>(kT, rows - r0) : 0;
-    rl.load(rows_rsrc(z + (nr > 0 ? r0 * nin : 0), nr * nin * 4), zv);
+    rl.load(rows_rsrc(z + (nr > 0 ? r0 * nin : 0), nr * nin * 4), v);
   };
-  load(tile);
+  load(tile, zv);
   for (; tile < tiles; tile += step) {
     rl.settle(zv);
+    if constexpr (kAhead) {
+      __builtin_amdgcn_sched_barrier(0);
+      load(tile + step, zn);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     f32x16 acc[kHT];
 #pragma unroll
     for (int t = 0; t < kHT; ++t) {
@@ -200,9 +210,11 @@ __global__ __launch_bounds__(forward_threads(G), 2) void k_mlp_forward(const flo
         for (int t = 0; t < kHT; ++t) acc[t] = mma(w[t][j], zv[g][j], acc[t]);
       }
     }
-    __builtin_amdgcn_sched_barrier(0);
-    load(tile + step);  // in flight under the second product and the stores
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!kAhead) {
+      __builtin_amdgcn_sched_barrier(0);
+      load(tile + step, zv);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     const int64_t r0 = tile * kT, nr = min<int64_t>(kT, rows - r0);
     if (a != nullptr) {
       const __amdgpu_buffer_rsrc_t ra = rows_rsrc(a + r0 * kHid, nr * kHid * 4);
@@ -234,6 +246,10 @@ __global__ __launch_bounds__(forward_threads(G), 2) void k_mlp_forward(const flo
     const __amdgpu_buffer_rsrc_t ry = rows_rsrc(y + r0 * nout, nr * nout * 4);
 #pragma unroll
     for (int o = 0; o < OT; ++o) store_row(ry, nout, kT * o, c, h, out[o]);
+    if constexpr (kAhead) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) zv[g] = zn[g];
+    }
   }
 }
 
@@ -268,13 +284,13 @@ __global__ __launch_bounds__(kMlpThreads, CT > 3 ? 1 : 2) void k_mlp_input_grad(
 
   const int64_t step = (int64_t)gridDim.x * (kThreads / 64);
   int64_t tile = (int64_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kThreads / 64) + threadIdx.x / 64));
-  f32x4 dv[GO], av[kHT][4];
+  f32x4 dv[GO], dn[GO], av[kHT][4];
   const RowLoad<GO> rl(nout, c, h);
   const uint32_t arow = (uint32_t)(c * kHid + 4 * h) * 4u;
   auto rows_of = [&](int64_t t) { return t < tiles ? min<int64_t>(kT, rows - t * kT) : (int64_t)0; };
   auto load_dy = [&](int64_t t) {
     const int64_t nr = rows_of(t);
-    rl.load(rows_rsrc(dy + (nr > 0 ? t * kT * nout : 0), nr * nout * 4), dv);
+    rl.load(rows_rsrc(dy + (nr > 0 ? t * kT * nout : 0), nr * nout * 4), dn);
   };
   auto load_a = [&](int64_t t, int u) {
     const int64_t nr = rows_of(t);
@@ -286,7 +302,12 @@ __global__ __launch_bounds__(kMlpThreads, CT > 3 ? 1 : 2) void k_mlp_input_grad(
 #pragma unroll
   for (int u = 0; u < kHT; ++u) load_a(tile, u);
   for (; tile < tiles; tile += step) {
-    rl.settle(dv);
+    rl.settle(dn);
+#pragma unroll
+    for (int g = 0; g < GO; ++g) dv[g] = dn[g];
+    __builtin_amdgcn_sched_barrier(0);
+    load_dy(tile + step);  // in flight until the next row tile
+    __builtin_amdgcn_sched_barrier(0);
     f32x16 out[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) out[ct] = f32x16{};
@@ -305,7 +326,6 @@ __global__ __launch_bounds__(kMlpThreads, CT > 3 ? 1 : 2) void k_mlp_input_grad(
       for (int r = 0; r < 16; ++r) dh[r] = av[t][r / 4][r % 4] <= 0.0f ? 0.0f : dh[r];
       __builtin_amdgcn_sched_barrier(0);
       load_a(tile + step, t);  // in flight until the next row tile
-      if (t == kHT - 1) load_dy(tile + step);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
@@ -328,6 +348,10 @@ __global__ __launch_bounds__(kMlpThreads, CT > 3 ? 1 : 2) void k_mlp_input_grad(
 
 // -------------------------------------------------------- weight gradients
 
+// Waves per SIMD of the weight gradients: as many as their sums in registers
+// leave room for.
+constexpr int weight_grad_waves(int ct, int go) { return ct > 3 ? 1 : go > 3 ? 2 : 3; }
+
 // Workgroup = one chunk of rows; wave t the hidden units 32 t .. 32 t + 31.
 // The four waves share each row tile's z and dy, staged in LDS as they lie in
 // memory (the tile's rows are one contiguous piece of each), the next tile's
@@ -336,7 +360,7 @@ __global__ __launch_bounds__(kMlpThreads, CT > 3 ? 1 : 2) void k_mlp_input_grad(
 // chunk's partial sums: dW1 (128 x nin), db1 (128), dW2 (nout x 128), db2
 // (nout), in that order.
 template <int CT, int GO>
-__global__ __launch_bounds__(kMlpThreads, CT > 3 ? 1 : 2) void k_mlp_weight_grad(
+__global__ __launch_bounds__(kMlpThreads, weight_grad_waves(CT, GO)) void k_mlp_weight_grad(
     const float* __restrict__ z, const float* __restrict__ a, const float* __restrict__ dy,
     const float* __restrict__ w2, float* __restrict__ part, int64_t rows, int nin, int nout, int64_t chunk_rows) {
   constexpr int OT = (GO + 3) / 4;
@@ -519,14 +543,16 @@ inline dim3 tile_grid(int64_t tiles, int threads) {
   return dim3((uint32_t)std::min<int64_t>(2048 / waves, (tiles + waves - 1) / waves));
 }
 
-// Rows per chunk of the weight gradients: 512 chunks (four waves each: two a
-// SIMD) for long inputs, at least two row tiles.
-int64_t weight_chunk_rows(int64_t rows) {
-  const int64_t c = (rows + 511) / 512;
+// Rows per chunk of the weight gradients: a chunk (of four waves) for every
+// workgroup the chip holds at once, at least two row tiles.
+int64_t weight_chunk_rows(int64_t rows, int nin, int nout) {
+  const int64_t want = 256 * std::max(2, weight_grad_waves((nin + kT - 1) / kT, (nout + 7) / 8));
+  const int64_t c = (rows + want - 1) / want;
   return std::max<int64_t>(64, (c + kT - 1) / kT * kT);
 }
-int64_t weight_chunks(int64_t rows) {
-  return rows > 0 ? (rows + weight_chunk_rows(rows) - 1) / weight_chunk_rows(rows) : 0;
+int64_t weight_chunks(int64_t rows, int nin, int nout) {
+  const int64_t c = weight_chunk_rows(rows, nin, nout);
+  return rows > 0 ? (rows + c - 1) / c : 0;
 }
 
 // f(integral_constant n) for a run-time 1 <= n <= N.
@@ -546,7 +572,7 @@ bool mlp_fits(int64_t rows, int nin, int hidden, int nout) {
 }
 
 int64_t mlp_weight_grad_floats(int64_t rows, int nin, int nout) {
-  return weight_chunks(rows) * ((int64_t)kHid * nin + kHid + (int64_t)nout * kHid + nout);
+  return weight_chunks(rows, nin, nout) * ((int64_t)kHid * nin + kHid + (int64_t)nout * kHid + nout);
 }
 
 void run_mlp_forward(const float* z, const float* w1, const float* b1, const float* w2, const float* b2, float* a,
@@ -590,11 +616,12 @@ void run_mlp_input_grad(const float* dy, const float* w1, const float* w2, const
 
 void run_mlp_weight_grad(const float* z, const float* a, const float* dy, const float* w2, float* dw1, float* db1,
                          float* dw2, float* db2, int64_t rows, int nin, int nout, float* work, hipStream_t st) {
-  const int64_t chunks = weight_chunks(rows);
+  const int64_t chunks = weight_chunks(rows, nin, nout);
   if (chunks > 0) {
     with_tiles(nin, nout, [&](auto ct, auto go) {
       hipLaunchKernelGGL((k_mlp_weight_grad<decltype(ct)::value, decltype(go)::value>), dim3((uint32_t)chunks),
-                         dim3(kMlpThreads), 0, st, z, a, dy, w2, work, rows, nin, nout, weight_chunk_rows(rows));
+                         dim3(kMlpThreads), 0, st, z, a, dy, w2, work, rows, nin, nout,
+                         weight_chunk_rows(rows, nin, nout));
     });
     SPHOPS_LAUNCHED();
   }
