@@ -222,13 +222,21 @@ __device__ __forceinline__ void store_pos_grad(float* __restrict__ out, uint32_t
   }
 }
 
+// p q - u v with the rounding error of u v put back (two fused multiply-adds):
+// nearly singular moment matrices cancel here.
+__device__ __forceinline__ float diff_of_products(float p, float q, float u, float v) {
+  const float w = u * v;
+  const float e = fmaf(-u, v, w);
+  return fmaf(p, q, -w) + e;
+}
+
 // Adjugate inverse of a symmetric 2x2 / 3x3 matrix read from its upper
 // triangle, identity when |det| < tol (sphops/sph_cuda.cu:3095-3179).
 template <int D>
 __device__ __forceinline__ void safe_inv_sym(const float* M, float tol, float* L) {
   if constexpr (D == 2) {
     const float a = M[0], b = M[1], d = M[3];
-    const float det = a * d - b * b;
+    const float det = diff_of_products(a, d, b, b);
     if (fabsf(det) < tol) {
       L[0] = 1.0f; L[1] = 0.0f; L[2] = 0.0f; L[3] = 1.0f;
       return;
@@ -237,18 +245,19 @@ __device__ __forceinline__ void safe_inv_sym(const float* M, float tol, float* L
     L[0] = d * id; L[1] = -b * id; L[2] = -b * id; L[3] = a * id;
   } else {
     const float a = M[0], b = M[1], c = M[2], d = M[4], e = M[5], f = M[8];
-    const float t1 = d * f - e * e, t2 = c * e - b * f, t3 = b * e - c * d;
-    const float det = a * t1 + b * t2 + c * t3;
+    const float t1 = diff_of_products(d, f, e, e), t2 = diff_of_products(c, e, b, f),
+                t3 = diff_of_products(b, e, c, d);
+    const float det = fmaf(a, t1, diff_of_products(b, t2, -c, t3));
     if (fabsf(det) < tol) {
 #pragma unroll
       for (int q = 0; q < 9; ++q) L[q] = (q % 4 == 0) ? 1.0f : 0.0f;
       return;
     }
     const float id = 1.0f / det;
-    const float u = (b * c - a * e) * id;
+    const float u = diff_of_products(b, c, a, e) * id;
     L[0] = t1 * id; L[1] = t2 * id; L[2] = t3 * id;
-    L[3] = t2 * id; L[4] = (a * f - c * c) * id; L[5] = u;
-    L[6] = t3 * id; L[7] = u; L[8] = (a * d - b * b) * id;
+    L[3] = t2 * id; L[4] = diff_of_products(a, f, c, c) * id; L[5] = u;
+    L[6] = t3 * id; L[7] = u; L[8] = diff_of_products(a, d, b, b) * id;
   }
 }
 
