@@ -1771,6 +1771,12 @@ __device__ __forceinline__ void store_entry(int32_t* __restrict__ nidx, uint32_t
 // Rounds of 64 candidates whose hit bytes a unit keeps in LDS for its write
 // pass (later rounds are tested again).
 constexpr int kFillRounds = 48;
+// Rounds whose candidates it keeps there too (4 bytes each), so that the write
+// pass need not map them again: a mapping is two instructions a stencil range
+// and candidate, as much as testing a small unit.  With the units' counter
+// asked ahead (fill_items): 250 000 particles in particle mode 266 -> 243-257
+// us, 10^6 in a clamped grid 280 -> 272-281.
+constexpr int kFillKept = 8;
 
 // Rows of the unit i0 .. i0 + ni - 1 (ni <= kUnitParticles particles of one
 // cell, or one lone particle), one wave.  Lane r < R fetches stencil range r
@@ -1778,7 +1784,7 @@ constexpr int kFillRounds = 48;
 // concatenated ranges, lane l taking position 64q + l, against every
 // particle of the unit (wave-uniform positions).  Pass one counts the hits
 // per particle and keeps, per lane and round, the byte of the unit's
-// particles its candidate hit (`hits`, this wave's kFillRounds * 64 bytes of
+// particles its candidate hit (`hits`, the first kFillRounds * 64 bytes of this wave's
 // LDS); the unit takes one block of the index buffer; pass two writes each
 // particle's row, ranking the hits of a round with mbcnt.
 template <int D, bool P, int R, bool OT>
@@ -1789,6 +1795,7 @@ __device__ __forceinline__ void unit_rows(const GridParams& g, const float4* __r
                                           int32_t* __restrict__ ncnt, const FillStripes& fs,
                                           const FillTiles& ft) {
   const uint32_t lane = (uint32_t)__lane_id();
+  uint32_t* __restrict__ kept_j = reinterpret_cast<uint32_t*>(hits + kFillRounds * kWave);
   const float4 pt = xw[i0 + min(lane, ni - 1u)];
   float xs[kUnitParticles][3];
 #pragma unroll
@@ -1796,6 +1803,30 @@ __device__ __forceinline__ void unit_rows(const GridParams& g, const float4* __r
     xs[t][0] = lane_float(pt.x, t);
     xs[t][1] = lane_float(pt.y, t);
     xs[t][2] = lane_float(pt.z, t);
+  }
+  // periodic: a candidate within near_lo .. near_hi lies less than half a box
+  // from every particle of the unit on every axis (0.95 of that, for the
+  // rounding), so no pair with it wraps; off the borders of a grid of five or
+  // more cells an axis, that is every candidate of the stencil.  The fill is
+  // bound by vector instructions and this test has a third fewer (3 x 20011
+  // particles: 123 -> 110 us)
+  float near_lo[3], near_hi[3];
+  bool inner = P;
+  if constexpr (P) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      float lo = xs[0][d], hi = xs[0][d];
+#pragma unroll
+      for (int t = 1; t < kUnitParticles; ++t) {
+        if (t < (int)ni) {
+          lo = fminf(lo, xs[t][d]);
+          hi = fmaxf(hi, xs[t][d]);
+        }
+      }
+      inner = inner && g.L[d] > 0.0f && lo >= -4.0f * g.L[d] && hi <= 4.0f * g.L[d];
+      near_lo[d] = hi - 0.95f * g.half_L[d];
+      near_hi[d] = lo + 0.95f * g.half_L[d];
+    }
   }
   // stencil range `lane` of the cell: start and length
   uint32_t lo = 0, len = 0;
@@ -1911,23 +1942,36 @@ __device__ __forceinline__ void unit_rows(const GridParams& g, const float4* __r
     unpack(nx, xj);
     if (p >= ncand) xj[0] = __int_as_float(0x7FC00000);  // NaN: never in radius
     const bool own = OT && tiled && jn >= cs && jn < ce;
+    if (rd < (uint32_t)kFillKept) kept_j[rd * kWave + lane] = jn;
     if (rd + 1 < rounds) {
       jn = candidate(p + kWave);
       nx = xw[jn];
     }
     uint32_t bits = 0;
+    auto test = [&](auto near) {
 #pragma unroll
-    for (int t = 0; t < kUnitParticles; ++t) {
-      if (t < (int)ni) {
-        float r[3];
-        const bool in = displacement<D, P>(g, xs[t], xj, r) < g.eps2;
-        cnt[t] += (uint32_t)__popcll(__ballot(in));
-        if constexpr (OT) {
-          if (tiled && rd * kWave < po1 && rd * kWave + kWave > po0)
-            cown[t] += (uint32_t)__popcll(__ballot(in && own));
+      for (int t = 0; t < kUnitParticles; ++t) {
+        if (t < (int)ni) {
+          float r[3];
+          const float d2 = decltype(near)::value ? near_displacement<D>(g, xs[t], xj) : displacement<D, P>(g, xs[t], xj, r);
+          const bool in = d2 < g.eps2;
+          cnt[t] += (uint32_t)__popcll(__ballot(in));
+          if constexpr (OT) {
+            if (tiled && rd * kWave < po1 && rd * kWave + kWave > po0)
+              cown[t] += (uint32_t)__popcll(__ballot(in && own));
+          }
+          bits |= (in ? 1u : 0u) << t;
         }
-        bits |= (in ? 1u : 0u) << t;
       }
+    };
+    if constexpr (P) {
+      bool outside = false;
+#pragma unroll
+      for (int d = 0; d < D; ++d) outside = outside || xj[d] < near_lo[d] || xj[d] > near_hi[d];
+      if (inner && __ballot(outside) == 0) test(std::integral_constant<bool, true>{});
+      else test(std::integral_constant<bool, false>{});
+    } else {
+      test(std::integral_constant<bool, false>{});
     }
     if (rd < (uint32_t)kFillRounds) hits[rd * kWave + lane] = (uint8_t)bits;
   }
@@ -1965,7 +2009,7 @@ __device__ __forceinline__ void unit_rows(const GridParams& g, const float4* __r
   // pass two: write the rows
   for (uint32_t rd = 0; rd < rounds; ++rd) {
     const uint32_t p = rd * kWave + lane;
-    const uint32_t j = candidate(p);
+    const uint32_t j = rd < (uint32_t)kFillKept ? kept_j[rd * kWave + lane] : candidate(p);
     uint32_t bits;
     if (rd < (uint32_t)kFillRounds) {
       bits = hits[rd * kWave + lane];
@@ -2016,6 +2060,12 @@ __device__ __forceinline__ void unit_rows(const GridParams& g, const float4* __r
   }
 }
 
+// Periodic boxes: a lone particle of up to kLoneLight candidates is walked by
+// its lane, one of up to 64 too where more than kLoneFew of the wave's lanes
+// have such a one (they walk at the same time).
+constexpr uint32_t kLoneLight = 24;
+constexpr int kLoneFew = 3;
+
 // Lone particles of the chunk of 64 particles starting at k0, one lane each:
 // a first walk over the stencil counts the candidates and marks the in-radius
 // ones among the first 64 (a 64-bit mask, the first four also kept in
@@ -2023,6 +2073,13 @@ __device__ __forceinline__ void unit_rows(const GridParams& g, const float4* __r
 // written from the registers or, for more than four hits, by a second walk.
 // A lone particle with more than 64 candidates is served afterwards by the
 // whole wave (unit_rows, ni = 1).
+// In a periodic box, whose density is about even, the few lone particles lie
+// among full cells and their walks, which wait for each load in turn, end
+// last: there the ranges' lengths are added up first and the heavy ones go to
+// the whole wave unwalked (3 x 20011 particles in 3D, 8 a cell: 110 -> 83 us,
+// 4 x 16384 in 2D 40 -> 34).  In the clouds of clamped grids the lone
+// particles are the many of the sparse outskirts, where adding up first only
+// costs (10^6 particles: 272 -> 310 us).
 template <int D, bool P, int R, bool OT>
 __device__ __forceinline__ void lone_rows(const GridParams& g, const float4* __restrict__ xw,
                                           const int32_t* __restrict__ bo, const int32_t* __restrict__ unit_len,
@@ -2050,6 +2107,21 @@ __device__ __forceinline__ void lone_rows(const GridParams& g, const float4* __r
   if (lone) {
     unpack(xw[k], xi);
     w.init(g, xi, k);
+  }
+  bool walk = lone;
+  if constexpr (P) {
+    uint32_t total = 0;
+    if (lone) {
+#pragma unroll 1
+      for (int r = 0; r < R; ++r) {
+        w.fetch(g, bo, r);
+        total += w.jend - w.j;
+      }
+    }
+    const uint64_t mid = __ballot(lone && total > kLoneLight && total <= (uint32_t)kWave);
+    walk = lone && total <= (__popcll(mid) > kLoneFew ? (uint32_t)kWave : kLoneLight);
+  }
+  if (walk) {
 #pragma unroll 1
     for (int r0 = 0; r0 < R; r0 += kFetch) {
       uint32_t rlo[kFetch], rhi[kFetch];
@@ -2088,7 +2160,7 @@ __device__ __forceinline__ void lone_rows(const GridParams& g, const float4* __r
       }
     }
   }
-  const bool light = lone && cand <= (uint32_t)kWave;
+  const bool light = walk && cand <= (uint32_t)kWave;
   const uint32_t cnt = light ? c : 0u;
   if constexpr (OT) {
     if (lone) ft.own[k] = 0;  // a lone particle's cell is never a tile
@@ -2139,7 +2211,9 @@ __device__ __forceinline__ void lone_rows(const GridParams& g, const float4* __r
 // queue q holds the units u = q, q + kFillStripes, ... (a sample of the whole
 // cloud, so the queues carry about equal work), its counter at word
 // kUnitQueueWord of stripe q, and the waves w = q mod kFillStripes take its
-// units one at a time until it is empty.  A unit's cost runs from one round
+// units one at a time until it is empty: each its own first (number w /
+// kFillStripes), then the next one the counter gives, asked for while the
+// current unit is served.  A unit's cost runs from one round
 // to dozens (crowded cells sit together), so a fixed share per wave leaves
 // the waves that drew crowded cells running long after the others.  Even
 // waves take their chunks first, odd waves their units first, so that the
@@ -2164,15 +2238,16 @@ __device__ __forceinline__ void fill_items(const GridParams& g, const float4* __
     } else {
       const uint32_t q = wave & (kFillStripes - 1u);
       const uint32_t in_queue = q < nunits ? (nunits - q + kFillStripes - 1u) / kFillStripes : 0u;
+      const uint32_t sharers = nwaves / kFillStripes;
       unsigned long long* __restrict__ next = fs.ctr + (uint64_t)q * kStripeWords + kUnitQueueWord;
-      for (;;) {
-        uint32_t i = 0;
-        if (__lane_id() == 0) i = (uint32_t)atomicAdd(next, 1ull);
-        i = (uint32_t)__builtin_amdgcn_readfirstlane((int)__shfl((int)i, 0, kWave));
-        if (i >= in_queue) break;
+      for (uint32_t i = wave / kFillStripes; i < in_queue;) {
+        uint32_t taken = 0;
+        if (in_queue > sharers && __lane_id() == 0) taken = (uint32_t)atomicAdd(next, 1ull);
         const uint2 ud = units[i * kFillStripes + q];
         unit_rows<D, P, R, OT>(g, xw, bo, __builtin_amdgcn_readfirstlane(ud.x),
                                __builtin_amdgcn_readfirstlane(ud.y), wave, hits, nidx, nstart, ncnt, fs, ft);
+        if (in_queue <= sharers) break;
+        i = sharers + (uint32_t)__builtin_amdgcn_readfirstlane((int)taken);
       }
     }
   }
@@ -2188,7 +2263,7 @@ __global__ __launch_bounds__(kThreads) void k_fill(GridParams g, const float4* _
                                                    const int32_t* __restrict__ unit_total,
                                                    int32_t* __restrict__ nidx, int32_t* __restrict__ nstart,
                                                    int32_t* __restrict__ ncnt, FillStripes fs, FillTiles ft) {
-  __shared__ __align__(16) uint8_t hits[kThreads / kWave][kFillRounds * kWave];
+  __shared__ __align__(16) uint8_t hits[kThreads / kWave][(kFillRounds + 4 * kFillKept) * kWave];
   uint8_t* mine = hits[threadIdx.x >> 6];
   const uint32_t nunits = (uint32_t)*unit_total;
   fill_items<D, P, M ? Walker<D, P>::kCellRanges : Walker<D, P>::kRowRanges, OT>(
@@ -2239,6 +2314,14 @@ constexpr uint32_t kPersistentWorkgroups = 2048;
 // beats 2048, 3072, 6144 and 8192).
 constexpr uint32_t kFillWorkgroups = 4096;
 static_assert(kFillWorkgroups * (kThreads / kWave) >= kFillStripes, "every unit queue of the fill has a wave");
+// For n particles: a wave for each of the at most n / 2 units they form, in
+// whole rounds of the unit queues.
+inline uint32_t fill_workgroups(uint64_t n) {
+  constexpr uint64_t per = kThreads / kWave, queues = kFillStripes / per;
+  const uint64_t w = (n / 2 + per - 1) / per;
+  return (uint32_t)std::min<uint64_t>(kFillWorkgroups, std::max<uint64_t>(1, (w + queues - 1) / queues) * queues);
+}
+static_assert(kFillWorkgroups % (kFillStripes / (kThreads / kWave)) == 0, "whole rounds of the unit queues");
 
 // Work split of the list fill (unit table and lone marks, in the grid's
 // scratch), read by neighbour_fill.
@@ -2274,7 +2357,7 @@ void neighbour_fill(const Grid& g, const int32_t* bo, const float* x, int32_t* n
   const bool ot = ft.own != nullptr;
   if (ot) fill_u32(reinterpret_cast<uint32_t*>(ft.count), 1, 0u, st);
 #define SPHOPS_FILL(M, OT)                                                                                      \
-  hipLaunchKernelGGL((k_fill<D, P, M, OT>), dim3(kFillWorkgroups), dim3(kThreads), 0, st, g.p, xw, bo, g.unit_len, \
+  hipLaunchKernelGGL((k_fill<D, P, M, OT>), dim3(fill_workgroups(n)), dim3(kThreads), 0, st, g.p, xw, bo, g.unit_len, \
                      g.units, g.unit_total, nidx, nstart, ncnt, fs, ft)
   if (g.particle_mode) {
     if (ot) SPHOPS_FILL(true, true);

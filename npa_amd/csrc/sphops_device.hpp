@@ -149,6 +149,21 @@ __device__ __forceinline__ float displacement(const GridParams& g, const float* 
   return acc;
 }
 
+// |r|^2 of a periodic pair that does not wrap (0 <= to - from + L / 2 < L on
+// every axis): what displacement gives, bit for bit, in a third of the
+// instructions.
+template <int D>
+__device__ __forceinline__ float near_displacement(const GridParams& g, const float* from, const float* to) {
+#pragma clang fp contract(off)
+  float acc = 0.0f;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const float v = ((to[d] - from[d]) + g.half_L[d]) - g.half_L[d];
+    acc = d == 0 ? v * v : acc + v * v;
+  }
+  return acc;
+}
+
 // -------------------------------------------------------------- kernels
 
 __device__ __forceinline__ float poly6(float eps2, float d2) {
