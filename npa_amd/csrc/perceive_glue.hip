@@ -65,7 +65,15 @@ __host__ __device__ inline uint32_t feature_width(uint32_t C, int D, int flags) 
          ((flags & SPHOPS_GLUE_DENSITY_GRAD) ? (uint32_t)D : 0u);
 }
 
-inline uint32_t tile_particles(uint32_t W) { return std::min<uint32_t>(64u, kTileFloats / W); }
+constexpr uint64_t kGlueTiles = 512;  // two a CU
+
+// Particles per tile: what the LDS holds, at most 64, and few enough that the
+// tiles fill the chip (tiles of 64 of 4096 particles run on one CU in four:
+// 11 us forward; tiles of 8: 5 us).
+inline uint32_t tile_particles(uint32_t W, uint64_t n) {
+  const uint32_t most = std::min<uint32_t>(64u, kTileFloats / W);
+  return (uint32_t)std::max<uint64_t>(std::min<uint64_t>(most, 8u), std::min<uint64_t>(most, n / kGlueTiles));
+}
 
 // i / d and i % d for i < 2^24: a float quotient, then one correction step
 __device__ __forceinline__ uint32_t div_small(uint32_t i, uint32_t d, float inv_d, uint32_t& r) {
@@ -376,7 +384,7 @@ void run_glue_forward(int dim, const float* s, const float* blur, const float* g
                       float* z, uint64_t n, uint32_t C, float coef_s, float coef_rho, float total_mass, int flags,
                       hipStream_t st) {
   if (n == 0) return;
-  const uint32_t T = tile_particles(feature_width(C, dim, flags));
+  const uint32_t T = tile_particles(feature_width(C, dim, flags), n);
   const dim3 grid((uint32_t)((n + T - 1) / T));
   if (dim == 2) {
     hipLaunchKernelGGL(k_glue_forward<2>, grid, dim3(kThreads), 0, st, s, blur, grad_s, grad_rho, z, n, C, T, coef_s,
@@ -392,7 +400,7 @@ void run_glue_backward(int dim, const float* dz, const float* grad_s, const floa
                        float* d_blur, float* d_grad_s, float* d_grad_rho, uint64_t n, uint32_t C, float coef_s,
                        float coef_rho, float total_mass, int flags, hipStream_t st) {
   if (n == 0) return;
-  const uint32_t T = tile_particles(feature_width(C, dim, flags));
+  const uint32_t T = tile_particles(feature_width(C, dim, flags), n);
   const dim3 grid((uint32_t)((n + T - 1) / T));
   if (dim == 2) {
     hipLaunchKernelGGL(k_glue_backward<2>, grid, dim3(kThreads), 0, st, dz, grad_s, grad_rho, d_s, d_blur, d_grad_s,
