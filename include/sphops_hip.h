@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define SPHOPS_ABI_VERSION 23
+#define SPHOPS_ABI_VERSION 24
 
 #define SPHOPS_CLAMPED 0
 #define SPHOPS_PERIODIC 1
@@ -420,6 +420,16 @@ int sphops_euler_update_forward(int dim, int P, const float* y, const float* x_b
                                 const float* mask, const float* noise, float* x_out, float* s_out, float* dx_norm,
                                 int64_t particles, uint32_t C, float alpha, float eps, float dt, float noise_std,
                                 float sqrt_dt, void* stream);
+
+/* The same update with row k of cloud b (clouds of `cloud` particles) written
+ * to row inverse[b][k], i.e. in input order (step_euler_trace,
+ * models/npa.py:207-241), and dx (particles, P; zero padding) and ds
+ * (particles, C) beside it, unless NULL. */
+int sphops_euler_update_trace(int dim, int P, const float* y, const float* x_bin, const float* s_bin,
+                              const float* mask, const float* noise, const int32_t* inverse, float* x_out,
+                              float* s_out, float* dx_out, float* ds_out, int64_t particles, uint32_t cloud,
+                              uint32_t C, float alpha, float eps, float dt, float noise_std, float sqrt_dt,
+                              void* stream);
 
 /* Backward of sphops_euler_update_forward with respect to y: from dL/dx_out
  * (particles, P), dL/ds_out (particles, C) and dL/d dx_norm (particles), any

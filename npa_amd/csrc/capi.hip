@@ -1043,6 +1043,23 @@ int sphops_euler_update_forward(int dim, int P, const float* y, const float* x_b
   });
 }
 
+int sphops_euler_update_trace(int dim, int P, const float* y, const float* x_bin, const float* s_bin,
+                              const float* mask, const float* noise, const int32_t* inverse, float* x_out,
+                              float* s_out, float* dx_out, float* ds_out, int64_t particles, uint32_t cloud,
+                              uint32_t C, float alpha, float eps, float dt, float noise_std, float sqrt_dt,
+                              void* stream) {
+  return guarded([&] {
+    require(dim == 2 || dim == 3, "dim must be 2 or 3");
+    require(P == (dim == 2 ? 2 : 4), "P must be 2 in 2D and 4 in 3D");
+    require(particles >= 0 && (particles == 0 || cloud > 0), "particles must be >= 0, in clouds of at least one");
+    sphops::check_channels(C);
+    require(particles == 0 || (y && x_bin && s_bin && inverse && x_out && s_out), "null buffer");
+    sphops::run_euler_trace(dim, y, x_bin, s_bin, mask, noise, inverse, x_out, s_out, dx_out, ds_out,
+                            (uint64_t)particles, cloud, C, alpha, eps, dt, noise_std, sqrt_dt,
+                            sphops::as_stream(stream));
+  });
+}
+
 int sphops_euler_update_backward(int dim, int P, const float* y, const float* mask, const float* d_x_out,
                                  const float* d_s_out, const float* d_dx_norm, float* d_y, int64_t particles,
                                  uint32_t C, float alpha, float eps, float dt, void* stream) {

@@ -302,6 +302,10 @@ void run_euler_forward(int dim, const float* y, const float* x_bin, const float*
 void run_euler_backward(int dim, const float* y, const float* mask, const float* d_x_out, const float* d_s_out,
                         const float* d_dx_norm, float* d_y, uint64_t n, uint32_t C, uint32_t P, float alpha,
                         float eps, float dt, hipStream_t st);
+void run_euler_trace(int dim, const float* y, const float* x_bin, const float* s_bin, const float* mask,
+                     const float* noise, const int32_t* inv, float* x_out, float* s_out, float* dx_out, float* ds_out,
+                     uint64_t n, uint32_t N, uint32_t C, float alpha, float eps, float dt, float noise_std,
+                     float sqrt_dt, hipStream_t st);
 // splatting.hip: 2D Gaussian splatting (utils/splatting.py:6-117)
 struct SplatParams {
   int H;             // image side (img_size)
@@ -319,7 +323,7 @@ constexpr int kMaxSplatRadius = 255;
 void run_splat_forward(const SplatParams& sp, const float* x, const float* color, const int32_t* starts, int images,
                        int64_t n, float4* rec, float* out, hipStream_t st);
 void run_splat_backward(const SplatParams& sp, const float* x, const float* color, const int32_t* starts, int images,
-                        int64_t n, const float* d_img, float* d_x, float* d_color, hipStream_t st);
+                        int64_t n, const float* d_img, float* d_x, float* d_color, void* work, hipStream_t st);
 
 // linear_grad.hip: weight / bias gradients of a linear layer over many rows
 constexpr int64_t kMaxChunkRows = 8192;

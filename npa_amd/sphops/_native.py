@@ -10,7 +10,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get(
     "SPHOPS_HIP_LIB", os.path.join(os.path.dirname(_HERE), "_lib", "libsphops_hip.so"))
-ABI_VERSION = 23
+ABI_VERSION = 24
 
 if not os.path.exists(LIB_PATH):
     raise ImportError(
@@ -60,6 +60,8 @@ _SIGNATURES = {
                                              _p], _i32),
     "sphops_euler_update_forward": ([_i32, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _u32, _f32, _f32, _f32,
                                      _f32, _f32, _p], _i32),
+    "sphops_euler_update_trace": ([_i32, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _u32, _u32, _f32, _f32,
+                                   _f32, _f32, _f32, _p], _i32),
     "sphops_euler_update_backward": ([_i32, _i32, _p, _p, _p, _p, _p, _p, _i64, _u32, _f32, _f32, _f32, _p], _i32),
     "sphops_splat_forward": ([_p, _p, _p, _i64, _i64, _i32, _i32, _f64, _f64, _f64, _i32, _i32, _f64, _p, _p, _p],
                              _i32),

@@ -119,14 +119,44 @@ def step_euler(model, x, s, grid, dt=1.0, update_prob=0.5, intermediate=False, n
     return x_new, s_new, stats
 
 
+def _trace_ok(y, x_bin, s_bin, mask, noise, dim, snapshot):
+    """What ``sphops_euler_update_trace`` takes: dense float32 rows of the
+    update's shapes, and the inverse permutation that the step left."""
+    B, N, P = x_bin.shape
+    C = s_bin.shape[-1]
+    dense = [(y, (B, N, dim + C)), (x_bin, (B, N, 2 if dim == 2 else 4)), (s_bin, (B, N, C))]
+    dense += [(mask, (B, N, 1))] if mask is not None else []
+    dense += [(noise, (B, N, P))] if noise is not None else []
+    inv = snapshot.inverse
+    return (dim in (2, 3) and N > 0 and all(t.shape == shape and t.dtype == torch.float32 and t.is_contiguous()
+                                            and t.is_cuda for t, shape in dense)
+            and inv is not None and snapshot.inverse_versions == (snapshot.permutation._version, inv._version))
+
+
 def step_euler_trace(model, x, s, grid, dt=1.0, update_prob=0.5, noise_std=0.0, return_aux=False):
     """step_euler_trace (models/npa.py:207-241): the updated particles in the
     input order; with return_aux also dx and ds of NPA.forward, unbinned."""
-    x_new, s_new, _, y, alpha = _step(model, x, s, grid, dt, update_prob, noise_std)
+    z, x_bin, s_bin, snapshot = _perceive(model, x, s, grid)
+    model.last_snapshot = snapshot
+    y = mlp(model.model, z).contiguous()
+    mask, noise = _draws(x, update_prob, noise_std)
+    alpha, D = buffer_value(model.alpha), model.spatial_dims
+    inv = snapshot.inverse
+    if _trace_ok(y, x_bin, s_bin, mask, noise, D, snapshot):
+        (B, N, P), C = x_bin.shape, s_bin.shape[-1]
+        out = [torch.empty_like(x_bin), torch.empty_like(s_bin)]
+        aux = [torch.empty_like(x_bin), torch.empty_like(s_bin)] if return_aux else [None, None]
+        st = ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(y.device.index))
+        _native.check(_lib.sphops_euler_update_trace(
+            D, P, _ptr(y), _ptr(x_bin), _ptr(s_bin), _ptr(mask), _ptr(noise), _ptr(inv), *(_ptr(t) for t in out),
+            *(_ptr(t) for t in aux), B * N, N, C, alpha, float(grid.eps), float(dt), float(noise_std),
+            math.sqrt(dt), st))
+        return (*out, *aux) if return_aux else tuple(out)
+    x_new, s_new, _ = EulerUpdate.apply(y, x_bin.contiguous(), s_bin.contiguous(), mask, noise, D, alpha,
+                                        float(grid.eps), float(dt), float(noise_std))
     x_trace, s_trace = unbin_particles(x_new, s_new, model.last_snapshot)
     if not return_aux:
         return x_trace, s_trace
-    D = model.spatial_dims
     a = y[..., :D]
     dx_bin = alpha * a * float(grid.eps) / (1.0 + a.norm(dim=-1, keepdim=True))
     if dx_bin.shape[-1] != x.shape[-1]:

@@ -192,3 +192,34 @@ def test_step_euler_static_matches_torch_assembly():
     _close("s", sf, sr, rtol=1e-4, atol=1e-5)
     _close("dL/ds", gf, gr, rtol=1e-4, atol=1e-5)
     _close("dL/dW", wf, wr, rtol=1e-3, atol=1e-4)
+
+
+@pytest.mark.parametrize("dim,N,C", [(2, 400, 8), (3, 333, 16), (3, 1, 3), (2, 5, 64)])
+@pytest.mark.parametrize("noise_std", [0.0, 0.02])
+@pytest.mark.parametrize("prob", [0.5, 1.0])
+def test_step_euler_trace_routes_agree(monkeypatch, dim, N, C, noise_std, prob):
+    # rows written in input order by the update against the update followed
+    # by unbin_particles; dx, whose scale the two paths round apart (squares,
+    # sums, root, sum, product and quotient: at most 8 roundings each), within
+    # 16 roundings of 2^-24
+    import npa_amd.sphops as sp
+    from npa_amd import step as S
+    c = H.random_case("t", 2, N, C, dim, 12, 0.15, False, "grid", sigma=0.8, seed=N)
+    torch.manual_seed(0)
+    model = _Model(dim, C).cuda()
+    x, s = torch.from_numpy(c.x).cuda(), torch.from_numpy(c.s).cuda()
+    results = []
+    for general in (False, True):
+        if general:
+            monkeypatch.setattr(S, "_trace_ok", lambda *a: False)
+        grid = sp.HashGrid(dim=dim, boundary="clamped", mode="grid", grid_size=list(c.grid_size), eps=c.eps,
+                           num_particles=N, batch_size=2, max_particles_per_block=c.maxp)
+        torch.manual_seed(5)
+        with torch.no_grad():
+            results.append(S.step_euler_trace(model, x, s, grid, 0.5, prob, noise_std, return_aux=True))
+            torch.manual_seed(5)
+            for a, b in zip(S.step_euler_trace(model, x, s, grid, 0.5, prob, noise_std), results[-1]):
+                assert torch.equal(a, b)
+    (x0, s0, dx0, ds0), (x1, s1, dx1, ds1) = results
+    assert torch.equal(x0, x1) and torch.equal(s0, s1) and torch.equal(ds0, ds1)
+    assert torch.all((dx0 - dx1).abs() <= 16 * 2.0 ** -24 * dx1.abs())
