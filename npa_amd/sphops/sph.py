@@ -228,12 +228,12 @@ def bin_particles(x, s, snapshot, mass=None):
 def unbin_particles(x_bin, s_bin, snapshot, mass_bin=None):
     x = torch.empty_like(x_bin)
     s = torch.empty_like(s_bin)
-    mass_is_none = mass_bin is None
+    if mass_bin is None:  # unit masses: nothing to move
+        _unbin(snapshot, _c(x_bin), _c(s_bin), None, x, s, None)
+        return x, s
     mass_bin = _default_mass(x_bin, mass_bin)
     mass = torch.empty_like(mass_bin)
     _unbin(snapshot, _c(x_bin), _c(s_bin), _c(mass_bin), x, s, mass)
-    if mass_is_none:
-        return x, s
     return x, s, mass
 
 
