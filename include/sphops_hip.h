@@ -450,7 +450,7 @@ int sphops_euler_update_backward(int dim, int P, const float* y, const float* ma
  * weight at the pixel over a (2r+1)^2 patch around floor(pos),
  * pos = (x - lo) / (hi - lo) * (img_size - 1) (y flipped with y_up), all as
  * the reference's splat_particles with the same arguments computes them.
- * Sums run in ascending particle order (deterministic).  workspace holds
+ * Sums run in a fixed order (deterministic).  workspace holds
  * sphops_splat_workspace_bytes(particles) bytes of per-particle records. */
 int sphops_splat_forward(const float* x, const float* color, const int32_t* starts, int64_t images,
                          int64_t particles, int ncolor, int img_size, double sigma, double lo, double hi,
@@ -468,6 +468,16 @@ int sphops_splat_backward(const float* x, const float* color, const int32_t* sta
                           int64_t particles, int ncolor, int img_size, double sigma, double lo, double hi,
                           int normalize_color, int y_up, double pixel_size, const float* d_out, float* d_x,
                           float* d_color, void* stream);
+
+/* The same, tile by tile where sphops_splat_backward_workspace_bytes of these
+ * arguments is not 0: workspace holds that many bytes, 16-byte aligned (NULL:
+ * as sphops_splat_backward). */
+int sphops_splat_backward_tiled(const float* x, const float* color, const int32_t* starts, int64_t images,
+                                int64_t particles, int ncolor, int img_size, double sigma, double lo, double hi,
+                                int normalize_color, int y_up, double pixel_size, const float* d_out, float* d_x,
+                                float* d_color, void* workspace, void* stream);
+int64_t sphops_splat_backward_workspace_bytes(int64_t particles, int img_size, double sigma, double lo, double hi,
+                                              int normalize_color, double pixel_size);
 
 /* Weight and bias gradients of a linear layer y = x W^T + b over `rows` rows
  * (no counterpart in the reference's native module: the NPA MLP is

@@ -1084,25 +1084,44 @@ int sphops_splat_forward(const float* x, const float* color, const int32_t* star
     require(images == 0 || (starts && out), "null buffer");
     require(particles == 0 || (x && color && workspace), "null buffer");
     require(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, "workspace must be 16-byte aligned");
-    sphops::run_splat_forward(sp, x, color, starts, (int)images, particles, static_cast<float4*>(workspace), out,
+    sphops::run_splat_forward(sp, x, color, starts, (int)images, particles, workspace, out,
                               sphops::as_stream(stream));
   });
 }
 
 int64_t sphops_splat_workspace_bytes(int64_t particles) { return particles > 0 ? 32 * particles : 0; }
 
-int sphops_splat_backward(const float* x, const float* color, const int32_t* starts, int64_t images,
-                          int64_t particles, int ncolor, int img_size, double sigma, double lo, double hi,
-                          int normalize_color, int y_up, double pixel_size, const float* d_out, float* d_x,
-                          float* d_color, void* stream) {
+int64_t sphops_splat_backward_workspace_bytes(int64_t particles, int img_size, double sigma, double lo, double hi,
+                                              int normalize_color, double pixel_size) {
+  int64_t bytes = 0;
+  guarded([&] {
+    bytes = sphops::splat_tiles_bytes(
+        sphops::splat_params(1, particles, 3, img_size, sigma, lo, hi, normalize_color, 0, pixel_size), particles);
+  });
+  return bytes;
+}
+
+int sphops_splat_backward_tiled(const float* x, const float* color, const int32_t* starts, int64_t images,
+                                int64_t particles, int ncolor, int img_size, double sigma, double lo, double hi,
+                                int normalize_color, int y_up, double pixel_size, const float* d_out, float* d_x,
+                                float* d_color, void* workspace, void* stream) {
   return guarded([&] {
     const sphops::SplatParams sp = sphops::splat_params(images, particles, ncolor, img_size, sigma, lo, hi,
                                                         normalize_color, y_up, pixel_size);
     require(particles == 0 || (x && color && starts && d_out && d_x && d_color), "null buffer");
     require(particles == 0 || images >= 1, "particles need at least one image");
-    sphops::run_splat_backward(sp, x, color, starts, (int)images, particles, d_out, d_x, d_color,
+    require(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, "workspace must be 16-byte aligned");
+    sphops::run_splat_backward(sp, x, color, starts, (int)images, particles, d_out, d_x, d_color, workspace,
                                sphops::as_stream(stream));
   });
+}
+
+int sphops_splat_backward(const float* x, const float* color, const int32_t* starts, int64_t images,
+                          int64_t particles, int ncolor, int img_size, double sigma, double lo, double hi,
+                          int normalize_color, int y_up, double pixel_size, const float* d_out, float* d_x,
+                          float* d_color, void* stream) {
+  return sphops_splat_backward_tiled(x, color, starts, images, particles, ncolor, img_size, sigma, lo, hi,
+                                     normalize_color, y_up, pixel_size, d_out, d_x, d_color, nullptr, stream);
 }
 
 int64_t sphops_linear_weight_grad_workspace_bytes(int64_t rows, int in_features, int out_features) {

@@ -321,7 +321,9 @@ struct SplatParams {
 };
 constexpr int kMaxSplatRadius = 255;
 void run_splat_forward(const SplatParams& sp, const float* x, const float* color, const int32_t* starts, int images,
-                       int64_t n, float4* rec, float* out, hipStream_t st);
+                       int64_t n, void* work, float* out, hipStream_t st);
+// Bytes of the workspace of the tile by tile backward, 0 where it is not used.
+int64_t splat_tiles_bytes(const SplatParams& sp, int64_t n);
 void run_splat_backward(const SplatParams& sp, const float* x, const float* color, const int32_t* starts, int images,
                         int64_t n, const float* d_img, float* d_x, float* d_color, void* work, hipStream_t st);
 

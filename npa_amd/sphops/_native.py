@@ -66,6 +66,9 @@ _SIGNATURES = {
     "sphops_splat_forward": ([_p, _p, _p, _i64, _i64, _i32, _i32, _f64, _f64, _f64, _i32, _i32, _f64, _p, _p, _p],
                              _i32),
     "sphops_splat_workspace_bytes": ([_i64], _i64),
+    "sphops_splat_backward_tiled": ([_p, _p, _p, _i64, _i64, _i32, _i32, _f64, _f64, _f64, _i32, _i32, _f64, _p, _p,
+                                     _p, _p, _p], _i32),
+    "sphops_splat_backward_workspace_bytes": ([_i64, _i32, _f64, _f64, _f64, _i32, _f64], _i64),
     "sphops_splat_backward": ([_p, _p, _p, _i64, _i64, _i32, _i32, _f64, _f64, _f64, _i32, _i32, _f64, _p, _p, _p,
                                _p], _i32),
     "sphops_linear_weight_grad": ([_p, _p, _p, _p, _i64, _i32, _i32, _p, _p], _i32),

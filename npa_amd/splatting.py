@@ -52,8 +52,12 @@ class Splat(torch.autograd.Function):
         d_x = torch.empty_like(x)
         d_color = torch.empty_like(color)
         st = ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(x.device.index))
-        _native.check(_lib.sphops_splat_backward(_ptr(x), _ptr(color), _ptr(starts), starts.numel() - 1, *ctx.args,
-                                                 _ptr(d_out), _ptr(d_x), _ptr(d_color), st))
+        n, _, img_size, sigma, lo, hi, normalize, _, pixel_size = ctx.args
+        size = _lib.sphops_splat_backward_workspace_bytes(n, img_size, sigma, lo, hi, normalize, pixel_size)
+        work = torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
+        _native.check(_lib.sphops_splat_backward_tiled(
+            _ptr(x), _ptr(color), _ptr(starts), starts.numel() - 1, *ctx.args, _ptr(d_out), _ptr(d_x), _ptr(d_color),
+            _ptr(work), st))
         return d_x, d_color, None, None, None, None, None, None, None, None
 
 

@@ -100,3 +100,37 @@ def test_deterministic_and_empty():
     far = torch.full((10, 2), 50.0, device="cuda")  # every patch off the image
     assert torch.count_nonzero(SP.splat_particles(far, cg[:10], **kw)) == 0
     assert torch.count_nonzero(SP.splat_particles(far[:0], cg[:0], **kw)) == 0
+
+
+@pytest.mark.parametrize("img_size,sigma,B,N,spread", [
+    (64, 0.8, 8, 60000, 1.1), (33, 1.0, 2, 140000, 1.3), (256, 4.0, 8, 2500, 0.01), (128, 4.0, 1, 21000, 0.7),
+    (250, 6.3, 3, 2700, 1.2)])
+@pytest.mark.parametrize("odd", [None, "pixel", "color"])
+def test_tiled_backward_matches_patches(monkeypatch, img_size, sigma, B, N, spread, odd):
+    # the two routes of the gradient, radii 4 to 32, lists that overflow (2500
+    # and more particles in a few tiles) and images cut by their edge; sums of the same
+    # terms in another order, at most (2 r + 1)^2 of them, each a product of at
+    # most six roundings: within 2^-24 (6 + 66) of the sum of magnitudes, taken
+    # as 30 times the gradient's largest element
+    from npa_amd import splatting as SP
+    lib = SP._lib
+    kw = dict(img_size=img_size, sigma=sigma, normalize_color=False)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = (torch.rand(B, N, 2, device="cuda", generator=g) * 2 - 1) * spread
+    c = torch.rand(B, N, 5, device="cuda", generator=g)
+    up = torch.randn(B, img_size, img_size, 4, device="cuda", generator=g)
+    if odd == "pixel":
+        up[0, img_size // 2, img_size // 2, 1] = float("inf")
+    if odd == "color":
+        c[0, N // 2, 3] = float("nan")
+    assert lib.sphops_splat_backward_workspace_bytes(B * N, img_size, sigma, -1.0, 1.0, 0, 2.0 / 128) > 0
+    res = []
+    for tiled in (True, False):
+        if not tiled:
+            monkeypatch.setattr(lib, "sphops_splat_backward_workspace_bytes", lambda *a: 0)
+        xr, cr = x.clone().requires_grad_(True), c.clone().requires_grad_(True)
+        res.append(torch.autograd.grad(SP.splat_particles_batch(xr, cr, **kw), (xr, cr), up))
+    for a, b in zip(*res):
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b))
+        ok = torch.isfinite(b)
+        assert torch.all((a - b)[ok].abs() <= 72 * 2.0 ** -24 * 30 * (b[ok].abs().max() if ok.any() else 0))
