@@ -2430,9 +2430,11 @@ __global__ __launch_bounds__(kThreads) void k_count_grouped(GridParams g, const 
   if (k < n && sub == 0) a.out0[k] = (float)count;
 }
 
-// Particles up to which the count is grouped: 16 lanes of each fill the chip
-// many times over from there on, and a lane each runs without their idle ones.
-constexpr uint64_t kCountGroupedParticles = 1ull << 19;
+// Particles up to which the count is grouped; beyond, a lane each fills the
+// chip.  At 2^17, grouped and by lanes, us: 85 and 101 in a periodic 3D box, 57
+// and 49 in a clamped one, 35 and 32 in 2D; at 2^19 300 and 204, 217 and 92,
+// 116 and 60.
+constexpr uint64_t kCountGroupedParticles = 1ull << 16;
 
 template <int D, bool P>
 void launch_count(const Grid& g, const int32_t* bo, OpPtrs a, hipStream_t st) {

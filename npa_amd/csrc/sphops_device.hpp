@@ -120,8 +120,8 @@ __device__ __forceinline__ void load_pos(const float* __restrict__ X, uint32_t k
 // positions inside the box never reach further; the general fmodf serves the
 // rest (NaN included).  The test runs for every candidate pair of a periodic
 // grid: with fmodf throughout, 3 x 20011 particles in a 3D box took 138 us
-// for the list fill, 125 us for the count and 77 us for the gradient; so they
-// take 123, 93 and 76 us.
+// for the list fill, 125 us for a lane per particle's count and 77 us for the
+// gradient; without, 123, 93 and 76 us.
 __device__ __forceinline__ float wrap_periodic(float d, float L, float half_L) {
 #pragma clang fp contract(off)
   if (L <= 0.0f) return d;
