@@ -89,7 +89,7 @@ def pair_kernel(name, D, periodic, C):
     """rocprofv3 kernel-name fragment of the pair kernel an operator call of
     the step launches (the call also launches a packing kernel), or None."""
     p = "true" if periodic else "false"
-    split = C in (16, 32)  # blur + gradient_hybrid on the lane-split kernels
+    split = C in (8, 12, 16, 20, 24, 32)  # blur + gradient_hybrid on the lane-split kernels
     names = {
         "pass_a_fwd": f"OpDensityPair<{D}, {p}>",
         "pass_a_bwd": f"OpDensityPairBwd<{D}, {p}>",
