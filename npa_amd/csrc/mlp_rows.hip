@@ -350,7 +350,7 @@ __global__ __launch_bounds__(kMlpThreads, CT > 3 ? 1 : 2) void k_mlp_input_grad(
 
 // Waves per SIMD of the weight gradients: as many as their sums in registers
 // leave room for.
-constexpr int weight_grad_waves(int ct, int go) { return ct > 3 ? 1 : go > 3 ? 2 : 3; }
+constexpr int weight_grad_waves(int ct, int go) { return ct > 3 ? 1 : ct > 2 || go > 3 ? 2 : 3; }
 
 // Workgroup = one chunk of rows; wave t the hidden units 32 t .. 32 t + 31.
 // The four waves share each row tile's z and dy, staged in LDS as they lie in
@@ -371,6 +371,17 @@ __global__ __launch_bounds__(kMlpThreads, weight_grad_waves(CT, GO)) void k_mlp_
   // operand reads of columns past a row's end fall into the next row, and for
   // the last row into the padding: their results are not kept
   __shared__ f32x4 zs[2][kZ4 + kT / 4], ds[2][kD4 + OT * kT / 4];
+  // dW2, whose rows relu(a) >= 0 do not cancel: every kFold tiles its sums
+  // move to LDS (each thread its own words), so that no chain of roundings is
+  // longer than kFold * kT rows (10^6 rows, 83 -> 128 -> 19: error against
+  // 64 bits 4.8e-7 with a chain a chunk, 3.8e-7 so)
+  constexpr int kFold = 8;
+  __shared__ float fold[OT][16][kMlpThreads];
+#pragma unroll
+  for (int o = 0; o < OT; ++o) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) fold[o][r][threadIdx.x] = 0.0f;
+  }
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
   const int band = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64) * kT;
   const int64_t r0 = (int64_t)blockIdx.x * chunk_rows, nr = min<int64_t>(chunk_rows, rows - r0);
@@ -417,6 +428,14 @@ __global__ __launch_bounds__(kMlpThreads, weight_grad_waves(CT, GO)) void k_mlp_
   load(0);
   int buf = 0;
   for (int64_t t0 = 0; t0 < nr; t0 += kT, buf ^= 1) {
+    if (t0 > 0 && t0 % (kFold * kT) == 0) {
+#pragma unroll
+      for (int o = 0; o < OT; ++o) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) fold[o][r][threadIdx.x] += acc2[o][r];
+        acc2[o] = f32x16{};
+      }
+    }
 #pragma unroll
     for (int u = 0; u < kLZ; ++u) {
       const int i = u * kMlpThreads + (int)threadIdx.x;
@@ -486,7 +505,7 @@ __global__ __launch_bounds__(kMlpThreads, weight_grad_waves(CT, GO)) void k_mlp_
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int m = kT * o + 8 * (r / 4) + 4 * h + r % 4;
-      if (m < nout) p[n1 + kHid + (int64_t)m * kHid + band + c] = acc2[o][r];
+      if (m < nout) p[n1 + kHid + (int64_t)m * kHid + band + c] = fold[o][r][threadIdx.x] + acc2[o][r];
     }
     const float s = sb2[o] + __shfl_xor(sb2[o], 32);
     if (band == 0 && h == 0 && kT * o + c < nout) p[n1 + kHid + n2 + kT * o + c] = s;
@@ -544,9 +563,11 @@ inline dim3 tile_grid(int64_t tiles, int threads) {
 }
 
 // Rows per chunk of the weight gradients: a chunk (of four waves) for every
-// workgroup the chip holds at once, at least two row tiles.
+// workgroup the chip holds at once, two where that is two a CU (shorter chains
+// of roundings: dW1), at least two row tiles.
 int64_t weight_chunk_rows(int64_t rows, int nin, int nout) {
-  const int64_t want = 256 * std::max(2, weight_grad_waves((nin + kT - 1) / kT, (nout + 7) / 8));
+  const int waves = weight_grad_waves((nin + kT - 1) / kT, (nout + 7) / 8);
+  const int64_t want = 256 * (waves == 2 ? 4 : std::max(2, waves));
   const int64_t c = (rows + want - 1) / want;
   return std::max<int64_t>(64, (c + kT - 1) / kT * kT);
 }
