@@ -29,8 +29,9 @@
 // traffic for each of the first two.  Measured inside a training step: 0.30 +
 // 0.28 + 0.36 ms, where the separate kernels took 0.51 (library product,
 // ReLU + second layer), 0.66 (its input gradient, library product) and 0.39;
-// forward and backward back to back 1.54 -> 0.91 ms (0.95 with the next row
-// tile's operands loaded under the second product only).
+// forward and backward back to back 1.54 -> 0.94 ms (0.95 with the next row
+// tile's operands loaded under the second product only, before the weight
+// gradients' shorter sums, which cost 0.03).
 #include "sphops_internal.hpp"
 #include "sphops_device.hpp"
 
