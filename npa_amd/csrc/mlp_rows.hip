@@ -565,12 +565,14 @@ inline dim3 tile_grid(int64_t tiles, int threads) {
 
 // Rows per chunk of the weight gradients: a chunk (of four waves) for every
 // workgroup the chip holds at once, two where that is two a CU (shorter chains
-// of roundings: dW1), at least two row tiles.
+// of roundings: dW1), at least two row tiles and at most kMaxChunkRows, which
+// bounds the chains of dW1 and db1 for any number of rows (from 4.2 or 8.4
+// million rows on).
 int64_t weight_chunk_rows(int64_t rows, int nin, int nout) {
   const int waves = weight_grad_waves((nin + kT - 1) / kT, (nout + 7) / 8);
   const int64_t want = 256 * (waves == 2 ? 4 : std::max(2, waves));
   const int64_t c = (rows + want - 1) / want;
-  return std::max<int64_t>(64, (c + kT - 1) / kT * kT);
+  return std::min<int64_t>(kMaxChunkRows, std::max<int64_t>(64, (c + kT - 1) / kT * kT));
 }
 int64_t weight_chunks(int64_t rows, int nin, int nout) {
   const int64_t c = weight_chunk_rows(rows, nin, nout);

@@ -349,7 +349,7 @@ void run_relu_linear_input_grad(const float* dy, const float* w, const float* h,
 constexpr int kMlpHidden = 128;
 constexpr int kMaxMlpIn = 168;   // the first layer's operand image and a row fit LDS and registers
 constexpr int kMaxMlpOut = 64;
-constexpr int64_t kMaxMlpRows = int64_t(1) << 30;  // byte offsets in a chunk of the weight gradients below 2^31
+constexpr int64_t kMaxMlpRows = int64_t(1) << 30;
 bool mlp_fits(int64_t rows, int nin, int hidden, int nout);
 int64_t mlp_weight_grad_floats(int64_t rows, int nin, int nout);
 void run_mlp_forward(const float* z, const float* w1, const float* b1, const float* w2, const float* b2, float* a,

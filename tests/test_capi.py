@@ -78,3 +78,14 @@ def test_header_is_plain_c(tmp_path):
     r = subprocess.run([gcc, "-std=c99", "-Wall", "-Wextra", "-pedantic", "-Werror", "-I", os.path.dirname(HEADER),
                         "-c", str(src), "-o", str(tmp_path / "abi.o")], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def test_mlp_weight_gradient_chunks_are_bounded():
+    """No chunk of the weight gradients, each one chain of sums in 32 bits,
+    is longer than 8192 rows: the workspace holds a partial sum per chunk."""
+    from npa_amd.sphops import _native
+    for nin, nout in ((4, 4), (83, 19), (163, 35)):
+        partial = 4 * (128 * nin + 128 + 128 * nout + nout)
+        for rows in (1, 65, 1 << 20, 1 << 23, (1 << 25) + 1, 1 << 30):
+            size = _native.lib.sphops_mlp_weight_grad_workspace_bytes(rows, nin, 128, nout)
+            assert size % partial == 0 and size // partial >= -(-rows // 8192)
