@@ -136,10 +136,13 @@ class MlpRows(torch.autograd.Function):
     """y = relu(z W1^T + b1) W2^T + b2 (``torch.nn.Linear``, ``ReLU``,
     ``Linear``) over z of shape (..., in) in one kernel
     (``sphops_mlp_forward``); the backward keeps z and the pre-activations and
-    takes dz and the weight gradients from one kernel each."""
+    takes dz and the weight gradients from one kernel each.  Without ``keep``
+    no backward follows and no pre-activations are written (inside ``forward``
+    grad mode is off and ``needs_input_grad`` set for every parameter, so the
+    caller says)."""
 
     @staticmethod
-    def forward(ctx, z, w1, b1, w2, b2):
+    def forward(ctx, z, w1, b1, w2, b2, keep):
         hidden, in_f = w1.shape
         out_f = w2.shape[0]
         z2 = z.reshape(-1, in_f).contiguous()
@@ -147,17 +150,18 @@ class MlpRows(torch.autograd.Function):
         dense = [None if t is None else t.detach().contiguous() for t in (w1, b1, w2, b2)]
         ctx.shape = (rows, in_f, hidden, out_f)
         ctx.biases = (b1 is not None, b2 is not None)
-        a = torch.empty(rows, hidden, device=z.device) if any(ctx.needs_input_grad) else None
+        a = torch.empty(rows, hidden, device=z.device) if keep else None
         y = torch.empty(rows, out_f, device=z.device)
         _native.check(_lib.sphops_mlp_forward(_ptr(z2), *(_ptr(t) for t in dense), _ptr(a), _ptr(y), rows, in_f,
                                               hidden, out_f, _stream(z)))
-        ctx.save_for_backward(z2, a, w1, w2)
+        if keep:
+            ctx.save_for_backward(z2, a, w1, w2)
         return y.reshape(*z.shape[:-1], out_f)
 
     @staticmethod
     def backward(ctx, dy):
         z2, a, w1, w2 = ctx.saved_tensors
-        need_z, need_w1, need_b1, need_w2, need_b2 = ctx.needs_input_grad
+        need_z, need_w1, need_b1, need_w2, need_b2, _ = ctx.needs_input_grad
         rows, in_f, hidden, out_f = ctx.shape
         dy2 = dy.reshape(-1, out_f).contiguous()
         if dy2.dtype != torch.float32 or not dy2.is_cuda:
@@ -180,7 +184,7 @@ class MlpRows(torch.autograd.Function):
             _native.check(_lib.sphops_mlp_weight_grad(_ptr(z2), _ptr(a), _ptr(dy2), _ptr(w2c), _ptr(dw1), _ptr(db1),
                                                       _ptr(dw2), _ptr(db2), rows, in_f, hidden, out_f, _ptr(work),
                                                       st))
-        return dz, dw1, db1, dw2, db2
+        return dz, dw1, db1, dw2, db2, None
 
 
 def _mlp_rows_ok(z, first, second):
@@ -232,7 +236,9 @@ def mlp(module, z):
             last = layers[i + 2] if i + 2 < len(layers) else None
             if (type(nxt) is torch.nn.ReLU and isinstance(layer, torch.nn.Linear) and isinstance(last, torch.nn.Linear)
                     and _mlp_rows_ok(z, layer, last)):
-                z = MlpRows.apply(z, layer.weight, layer.bias, last.weight, last.bias)
+                inputs = (z, layer.weight, layer.bias, last.weight, last.bias)
+                keep = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in inputs)
+                z = MlpRows.apply(*inputs, keep)
                 i += 3
                 continue
             if (type(layer) is torch.nn.ReLU and isinstance(nxt, torch.nn.Linear)

@@ -97,7 +97,7 @@ def test_mlp_rows_is_deterministic_and_optional():
         M.mlp(net, zr).backward(up)
         grads.append([zr.grad, *(p.grad.clone() for p in net.parameters())])
     assert all(torch.equal(a, b) for a, b in zip(*grads))
-    with torch.no_grad():  # no pre-activations kept
+    with torch.no_grad():
         y = M.mlp(net, z)
     assert not y.requires_grad and torch.allclose(y, net(z), rtol=1e-5, atol=1e-5)
     net[0].weight.requires_grad_(False)  # each gradient alone
@@ -109,3 +109,21 @@ def test_mlp_rows_is_deterministic_and_optional():
         other = other.cuda()  # shapes the kernels do not take: the layers' own functions
         v = torch.randn(50, other[0].in_features, device="cuda")
         assert torch.allclose(M.mlp(other, v), other(v), rtol=1e-5, atol=1e-5)
+
+
+def test_pre_activations_only_for_a_backward(monkeypatch):
+    """The 512 bytes a row that only the backward reads are written where one
+    can follow: not under no_grad, and not without an input that needs a
+    gradient."""
+    from npa_amd import mlp as M
+    net, z, _ = _case(200, 83, 19, True, 7)
+    kept, call = [], M._lib.sphops_mlp_forward
+    monkeypatch.setattr(M._lib, "sphops_mlp_forward", lambda *a: kept.append(bool(a[5].value)) or call(*a))
+    with torch.no_grad():
+        y = M.mlp(net, z)
+        M.mlp(net, z.clone().requires_grad_(True))
+    ref = M.mlp(net, z)
+    for p in net.parameters():
+        p.requires_grad_(False)
+    M.mlp(net, z)
+    assert kept == [False, False, True, False] and torch.equal(y, ref)
