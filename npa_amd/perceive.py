@@ -27,6 +27,9 @@ from .sphops import bin_particles, blur, density, density_gradient, gradient_hyb
 
 _lib = _native.lib
 
+_NATIVE_GRIDS = frozenset(sph.get_hashgrid_cls(d, b, m) for d in (2, 3) for b in ("periodic", "clamped")
+                          for m in ("grid", "particle"))
+
 STATE_GRAD, LOG_NORM_GRAD, DENSITY_GRAD, LOG_NORM_DENSITY_GRAD = 1, 2, 4, 8
 
 
@@ -202,10 +205,15 @@ class Perceive(torch.autograd.Function):
 
 
 def _native_ok(x, s, grid):
-    """What ``Perceive`` takes: dense float32 GPU tensors of the grid's shape
-    (anything else goes to the operators, which raise or handle it), the
-    default lists, and pass fusion on (``NPA_SPHOPS_FUSE``)."""
-    hg = grid.hashgrid
+    """What ``Perceive`` takes: a grid that instantiates as ``HashGrid`` and
+    its native class do (a subclass, an instance attribute or another object
+    may not), dense float32 GPU tensors of the grid's shape (anything else
+    goes to the operators, which raise or handle it), the default lists, and
+    pass fusion on (``NPA_SPHOPS_FUSE``)."""
+    hg = getattr(grid, "hashgrid", None)
+    if (getattr(type(grid), "instantiate", None) is not sph.HashGrid.instantiate or "instantiate" in vars(grid)
+            or type(hg) not in _NATIVE_GRIDS):
+        return False
     return (sph._PASS_A.enabled and sph._PASS_B.enabled and not hg.tiles_enabled and not hg._cells_wanted()
             and isinstance(x, torch.Tensor) and x.dtype == s.dtype == torch.float32 and x.is_cuda
             and x.device == s.device and x.dim() == s.dim() == 3 and x.is_contiguous() and s.is_contiguous()

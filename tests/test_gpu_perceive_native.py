@@ -109,3 +109,36 @@ def test_overflowing_list_walks_the_stencil():
         assert grid.list_overflow() == (cap == 7)
     for a, b in zip(*outs):
         assert torch.allclose(a, b, rtol=1e-4, atol=1e-4 * b.abs().max().item())
+
+
+def test_other_grids_keep_their_own_instantiate():
+    """A grid that instantiates in its own way, as a subclass, on the instance
+    or without a native grid of its own, is asked for its snapshot."""
+    import npa_amd.sphops as sp
+    from npa_amd import perceive as PF
+    grid, x, s = _grid(2, False, "grid", 16)
+    with torch.no_grad():
+        ref = PF.perceive(x, s, grid, 0.1)
+        asked = []
+
+        class Own(sp.HashGrid):
+            def instantiate(self, x):
+                asked.append("subclass")
+                return super().instantiate(x)
+
+        class Wrapped:
+            dim, eps = grid.dim, grid.eps
+
+            def instantiate(self, x):
+                asked.append("wrapped")
+                return grid.instantiate(x)
+
+        own = Own(dim=2, boundary="clamped", mode="grid", grid_size=grid.grid_size, eps=grid.eps, num_particles=301,
+                  batch_size=2, max_particles_per_block=grid.max_particles_per_block)
+        patched = _grid(2, False, "grid", 16)[0]
+        patched.instantiate = lambda x: asked.append("instance") or grid.instantiate(x)
+        for other in (own, Wrapped(), patched):
+            got = PF.perceive(x, s, other, 0.1)
+            assert all(torch.equal(a, b) for a, b in zip(got[1:3], ref[1:3]))
+            assert torch.allclose(got[0], ref[0], rtol=1e-4, atol=1e-5)
+    assert asked == ["subclass", "wrapped", "instance"]
