@@ -100,17 +100,20 @@ class Perceive(torch.autograd.Function):
     call each way (``sphops_perceive_forward`` / ``_backward``): the calls of
     the general path in its order, without the Python between them, and with
     the gradients that meet at x and s summed as they are unbinned.  ``out``
-    receives the snapshot, whose neighbour list later operators reuse."""
+    receives the snapshot, whose neighbour list later operators reuse.
+    Without ``keep`` no backward follows and nothing is kept for it (inside
+    ``forward`` grad mode is off and ``needs_input_grad`` set for every input
+    that requires a gradient, so the caller says)."""
 
     @staticmethod
-    def forward(ctx, x, s, grid, args, stop_pos, stop_state, out):
+    def forward(ctx, x, s, grid, args, stop_pos, stop_state, out, keep):
         B, N, P = x.shape
         C, D, dev, hg = s.shape[2], grid.dim, x.device, grid.hashgrid
         n = B * N
         flags, coef_s, coef_rho, total_mass = args
         # whether z's gradient flows to x and to s
-        pos = ctx.needs_input_grad[0] and not stop_pos
-        state = ctx.needs_input_grad[1] and not stop_state
+        pos = keep and ctx.needs_input_grad[0] and not stop_pos
+        state = keep and ctx.needs_input_grad[1] and not stop_state
         snap = grid._new_snapshot(dev)
         x_bin, s_bin = torch.empty_like(x), torch.empty_like(s)
         z = torch.empty(B, N, feature_width(C, D, flags), dtype=torch.float32, device=dev)
@@ -143,7 +146,7 @@ class Perceive(torch.autograd.Function):
         if stop_pos and stop_state:
             ctx.mark_non_differentiable(z)
         ctx.set_materialize_grads(False)
-        if any(ctx.needs_input_grad):
+        if keep:
             if grads:
                 ctx.save_for_backward(x_bin, s_bin, mass, work)
             ctx.snapshot, ctx.pos, ctx.state, ctx.sizes, ctx.args = snap, pos, state, sizes, args
@@ -164,7 +167,7 @@ class Perceive(torch.autograd.Function):
             dx, ds = (torch.zeros(shape, device=dev) if t is None else t for t, shape in zip(ups[1:], ctx.shapes))
             grad_x, grad_s = torch.empty_like(dx), torch.empty_like(ds)
             sph._unbin(snap, dx, ds, None, grad_x, grad_s, None)
-            return (grad_x if need_x else None, grad_s if need_s else None) + (None,) * 5
+            return (grad_x if need_x else None, grad_s if need_s else None) + (None,) * 6
         x_bin, s_bin, mass, work = ctx.saved_tensors
         n, D = B * N, snap.dim
         # a permutation modified since the step: rows summed in binned order,
@@ -201,7 +204,7 @@ class Perceive(torch.autograd.Function):
             out = torch.empty_like(grad_x), torch.empty_like(grad_s)
             snap.grid.backward_bin_particles(grad_x, grad_s, None, snap.permutation, out[0], out[1], None)
             grad_x, grad_s = out
-        return (grad_x if need_x else None, grad_s if need_s else None) + (None,) * 5
+        return (grad_x if need_x else None, grad_s if need_s else None) + (None,) * 6
 
 
 def _native_ok(x, s, grid):
@@ -238,8 +241,9 @@ def perceive(x, s, grid, eps0=0.1, state_grad=True, density_grad=True, log_norm_
         flags = (STATE_GRAD | (LOG_NORM_GRAD if log_norm_grad else 0)
                  | DENSITY_GRAD | (LOG_NORM_DENSITY_GRAD if log_norm_density_grad else 0))
         out = []
+        keep = torch.is_grad_enabled() and (x.requires_grad or s.requires_grad)
         z, x_bin, s_bin = Perceive.apply(x, s, grid, (flags, float(coef), float(coef_rho), float(N)), stopgrad_pos,
-                                         stopgrad_state, out)
+                                         stopgrad_state, out, keep)
         return z, x_bin, s_bin, out[0]
     with torch.no_grad():
         snapshot = grid.instantiate(x)

@@ -142,3 +142,24 @@ def test_other_grids_keep_their_own_instantiate():
             assert all(torch.equal(a, b) for a, b in zip(got[1:3], ref[1:3]))
             assert torch.allclose(got[0], ref[0], rtol=1e-4, atol=1e-5)
     assert asked == ["subclass", "wrapped", "instance"]
+
+
+def test_records_only_for_a_backward(monkeypatch):
+    """The (x, weight) records that only the backward reads are kept where one
+    can follow: not under no_grad, whatever the inputs require."""
+    from npa_amd import perceive as PF
+    grid, x, s = _grid(2, False, "grid", 16)
+    kept, call = [], PF._lib.sphops_perceive_forward
+
+    def spy(h, a, stream):
+        kept.append((bool(a._obj.packed_mass), bool(a._obj.packed_volume)))
+        return call(h, a, stream)
+
+    monkeypatch.setattr(PF._lib, "sphops_perceive_forward", spy)
+    xr, sr = x.clone().requires_grad_(True), s.clone().requires_grad_(True)
+    outs = []
+    with torch.no_grad():
+        outs.append(PF.perceive(xr, sr, grid, 0.1, stopgrad_pos=False))
+    outs.append(PF.perceive(xr, sr, grid, 0.1, stopgrad_pos=False))
+    assert kept == [(False, False), (True, True)]
+    assert not outs[0][0].requires_grad and all(torch.equal(a, b) for a, b in zip(outs[0][:3], outs[1][:3]))
