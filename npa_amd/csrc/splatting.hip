@@ -516,9 +516,10 @@ __global__ __launch_bounds__(kTileThreads, 4) void k_splat_backward_tiles(SplatP
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int qx = tx0 + 4 * kq + v - at.x;
+        // not a zero weight: a column outside the patch may overflow
+        if (qx < -r || qx > r) continue;
         const float ax = (float)qx - f.x;
-        const float w = gauss(ax, 0.0f, sp.inv_two_s2);
-        const float gx = qx >= -r && qx <= r ? w : 0.0f;
+        const float gx = gauss(ax, 0.0f, sp.inv_two_s2);
         const float U = c.x * T[0][v] + c.y * T[1][v] + c.z * T[2][v] + T[3][v];
         const float V = c.x * Y[0][v] + c.y * Y[1][v] + c.z * Y[2][v] + Y[3][v];
         t.dr += gx * T[0][v];

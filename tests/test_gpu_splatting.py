@@ -134,3 +134,29 @@ def test_tiled_backward_matches_patches(monkeypatch, img_size, sigma, B, N, spre
         assert torch.equal(torch.isfinite(a), torch.isfinite(b))
         ok = torch.isfinite(b)
         assert torch.all((a - b)[ok].abs() <= 72 * 2.0 ** -24 * 30 * (b[ok].abs().max() if ok.any() else 0))
+
+
+def test_large_pixels_outside_a_patch_add_nothing(monkeypatch):
+    """Finite upstreams so large that a column's sum times a colour passes the
+    largest float, in the rows but not in the columns of some patches: those
+    particles' gradients are the same as on the wave per particle's route,
+    which never reads such pixels (bound as above)."""
+    from npa_amd import splatting as SP
+    lib = SP._lib
+    kw = dict(img_size=64, sigma=0.8, normalize_color=False)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = (torch.rand(8, 60000, 2, device="cuda", generator=g) * 2 - 1) * 1.1
+    c = torch.rand(8, 60000, 3, device="cuda", generator=g) * 30
+    up = torch.randn(8, 64, 64, 4, device="cuda", generator=g)
+    up[:, :, 20, 1] = 3e38
+    assert lib.sphops_splat_backward_workspace_bytes(480000, 64, 0.8, -1.0, 1.0, 0, 2.0 / 128) > 0
+    res = []
+    for tiled in (True, False):
+        if not tiled:
+            monkeypatch.setattr(lib, "sphops_splat_backward_workspace_bytes", lambda *a: 0)
+        xr, cr = x.clone().requires_grad_(True), c.clone().requires_grad_(True)
+        res.append(torch.autograd.grad(SP.splat_particles_batch(xr, cr, **kw), (xr, cr), up))
+    for a, b in zip(*res):
+        far = torch.isfinite(b).all(-1) & (b.abs().amax(-1) < 1e30)  # the patch does not reach column 20
+        assert 0.5 < far.float().mean() < 1.0 and torch.isfinite(a[far]).all()
+        assert torch.all((a - b)[far].abs() <= 72 * 2.0 ** -24 * 30 * b[far].abs().max())
