@@ -387,10 +387,12 @@ __global__ __launch_bounds__(64 * kBwdWaves) void k_splat_backward(SplatParams s
   t.gg = wave_sum(t.gg);
   t.ggx = wave_sum(t.ggx);
   t.ggy = wave_sum(t.ggy);
-  a.sx = wave_sum(a.sx);
-  a.sy = wave_sum(a.sy);
-  a.sxa = wave_sum(a.sxa);
-  a.sya = wave_sum(a.sya);
+  if (live && sp.normalize) {  // wave-uniform
+    a.sx = wave_sum(a.sx);
+    a.sy = wave_sum(a.sy);
+    a.sxa = wave_sum(a.sxa);
+    a.sya = wave_sum(a.sya);
+  }
   store_gradients(sp, i, live, t, a, lane, 64, d_x, d_color);
 }
 
