@@ -78,6 +78,15 @@ __device__ __forceinline__ f32x16 mma(float a, float b, f32x16 c) {
 // relu as torch computes it: NaN stays NaN
 __device__ __forceinline__ float relu(float v) { return v <= 0.0f ? 0.0f : v; }
 
+// Four columns loaded `shift` before their place, moved up and zero-filled
+// (4 or more: none of them exist).
+__device__ __forceinline__ f32x4 move_up(f32x4 t, int shift) {
+  if (shift & 1) t = f32x4{t[1], t[2], t[3], 0.0f};
+  if (shift & 2) t = f32x4{t[2], t[3], 0.0f, 0.0f};
+  if (shift >= 4) t = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  return t;
+}
+
 // A lane's share of row c of a row tile of `width` >= 4 columns, G = ceil(width
 // / 8): columns 8 g + 4 h .. + 3 (h the lane's half) for each group g, in
 // 16-byte loads (dword-aligned).  The last group's load is moved back to end
@@ -99,13 +108,7 @@ struct RowLoad {
     v[G - 1] = load4(r, off_last);
   }
   // after the loads, before the first use
-  __device__ __forceinline__ void settle(f32x4 (&v)[G]) const {
-    f32x4 t = v[G - 1];
-    if (shift & 1) t = f32x4{t[1], t[2], t[3], 0.0f};
-    if (shift & 2) t = f32x4{t[2], t[3], 0.0f, 0.0f};
-    if (shift >= 4) t = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    v[G - 1] = t;
-  }
+  __device__ __forceinline__ void settle(f32x4 (&v)[G]) const { v[G - 1] = move_up(v[G - 1], shift); }
 };
 
 // Result columns of a transposed tile back to row c: registers 4 q .. 4 q + 3
@@ -125,45 +128,59 @@ __device__ __forceinline__ void store_row(__amdgpu_buffer_rsrc_t r, int width, i
   }
 }
 
+// Fills an operand image of N entries (entry i = load(i)) by T threads, kBatch
+// entries a thread in flight: a workgroup builds its images before its first
+// row tile, and one entry at a time that took longer than the tiles of few
+// rows (see k_mlp_forward and k_mlp_input_grad).
+template <int N, int T, class Load>
+__device__ __forceinline__ void build_image(f32x4* image, Load load) {
+  constexpr int kBatch = 8;
+#pragma unroll 1
+  for (int i0 = 0; i0 < N; i0 += kBatch * T) {
+    f32x4 v[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) v[u] = load(min(i0 + u * T + (int)threadIdx.x, N - 1));
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int i = i0 + u * T + (int)threadIdx.x;
+      if (i < N) image[i] = v[u];
+    }
+  }
+}
+
 // ---------------------------------------------------------------- forward
 
-// Threads a workgroup: the operand images of wide rows leave room for one
-// workgroup per CU, which then gets two waves a SIMD by itself.
-constexpr int forward_threads(int g) { return g > 13 ? 512 : 256; }
+// Threads a workgroup: the operand images of wide rows (G > 13) leave room for
+// one workgroup per CU, which then gets two waves a SIMD by itself, unless the
+// row tiles are no more than a wave each for the chip's SIMDs: two waves on a
+// SIMD take turns at the matrix core (300 rows of 163 columns: 33 us with 512
+// threads a workgroup, 21 with 256).
+constexpr int forward_threads(int g, int64_t tiles) { return g > 13 && tiles > 1024 ? 512 : 256; }
 
 // G: groups of 8 input columns; OT: output tiles.  a (rows x 128), the
 // pre-activations for the backward, may be null.
-template <int G, int OT>
-__global__ __launch_bounds__(forward_threads(G), 2) void k_mlp_forward(const float* __restrict__ z,
+template <int G, int OT, int kThreads>
+__global__ __launch_bounds__(kThreads, G > 13 ? kThreads / 256 : 2) void k_mlp_forward(const float* __restrict__ z,
                                                                 const float* __restrict__ w1,
                                                                 const float* __restrict__ b1,
                                                                 const float* __restrict__ w2,
                                                                 const float* __restrict__ b2, float* __restrict__ a,
                                                                 float* __restrict__ y, int64_t rows, int nin,
                                                                 int nout, int64_t tiles) {
-  constexpr int kThreads = forward_threads(G);
   __shared__ f32x4 w1img[G][kHT][64];        // lane l: W1[32 t + l % 32][8 g + 4 (l / 32) ..]
   __shared__ f32x4 w2img[kHT * 4][OT][64];   // lane l: W2[32 o + l % 32][8 p + 4 (l / 32) ..]
   __shared__ f32x4 b1s[kHid / 4];
   __shared__ f32x4 b2s[OT * kT / 4];
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
-  for (int i = threadIdx.x; i < G * kHT * 64; i += kThreads) {
-    const int l = i & 63, t = (i >> 6) % kHT, g = (i >> 6) / kHT, k = 8 * g + 4 * (l >> 5);
-    const float* __restrict__ p = w1 + (int64_t)(kT * t + (l & 31)) * nin + k;
-    f32x4 v;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = k + j < nin ? p[j] : 0.0f;
-    w1img[g][t][l] = v;
-  }
-  for (int i = threadIdx.x; i < kHT * 4 * OT * 64; i += kThreads) {
+  const __amdgpu_buffer_rsrc_t rw1 = rows_rsrc(w1, kHid * nin * 4), rw2 = rows_rsrc(w2, nout * kHid * 4);
+  build_image<G * kHT * 64, kThreads>(&w1img[0][0][0], [&](int i) {
+    const int l = i & 63, t = (i >> 6) % kHT, g = (i >> 6) / kHT, k = 8 * g + 4 * (l >> 5), at = min(k, nin - 4);
+    return move_up(load4(rw1, (uint32_t)((kT * t + (l & 31)) * nin + at) * 4u), k - at);
+  });
+  build_image<kHT * 4 * OT * 64, kThreads>(&w2img[0][0][0], [&](int i) {
     const int l = i & 63, o = (i >> 6) % OT, p = (i >> 6) / OT, n = kT * o + (l & 31);
-    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (n < nout) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = w2[(int64_t)n * kHid + 8 * p + 4 * (l >> 5) + j];
-    }
-    w2img[p][o][l] = v;
-  }
+    return load4(rw2, n < nout ? (uint32_t)(n * kHid + 8 * p + 4 * (l >> 5)) * 4u : kPast);
+  });
   if (threadIdx.x < kHid) reinterpret_cast<float*>(b1s)[threadIdx.x] = b1 != nullptr ? b1[threadIdx.x] : 0.0f;
   if (threadIdx.x < OT * kT)
     reinterpret_cast<float*>(b2s)[threadIdx.x] =
@@ -265,22 +282,23 @@ __global__ __launch_bounds__(kMlpThreads, CT > 3 ? 1 : 2) void k_mlp_input_grad(
   __shared__ f32x4 w1img[kHT * 4][CT][64];  // lane l: W1[8 p + 4 (l / 32) + j][32 ct + l % 32], j = 0..3
   __shared__ f32x4 w2img[GO][kHT][64];      // lane l: W2[8 g + 4 (l / 32) + j][32 t + l % 32]
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
-  for (int i = threadIdx.x; i < kHT * 4 * CT * 64; i += kThreads) {
+  const __amdgpu_buffer_rsrc_t rw1 = rows_rsrc(w1, kHid * nin * 4), rw2 = rows_rsrc(w2, nout * kHid * 4);
+  build_image<kHT * 4 * CT * 64, kThreads>(&w1img[0][0][0], [&](int i) {
     const int l = i & 63, ct = (i >> 6) % CT, p = (i >> 6) / CT, n = kT * ct + (l & 31);
-    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (n < nin) {
+    f32x4 v;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = w1[(int64_t)(8 * p + 4 * (l >> 5) + j) * nin + n];
-    }
-    w1img[p][ct][l] = v;
-  }
-  for (int i = threadIdx.x; i < GO * kHT * 64; i += kThreads) {
+    for (int j = 0; j < 4; ++j)
+      v[j] = load1(rw1, n < nin ? (uint32_t)((8 * p + 4 * (l >> 5) + j) * nin + n) * 4u : kPast);
+    return v;
+  });
+  build_image<GO * kHT * 64, kThreads>(&w2img[0][0][0], [&](int i) {
     const int l = i & 63, t = (i >> 6) % kHT, g = (i >> 6) / kHT, k = 8 * g + 4 * (l >> 5);
     f32x4 v;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = k + j < nout ? w2[(int64_t)(k + j) * kHid + kT * t + (l & 31)] : 0.0f;
-    w2img[g][t][l] = v;
-  }
+    for (int j = 0; j < 4; ++j)
+      v[j] = load1(rw2, k + j < nout ? (uint32_t)((k + j) * kHid + kT * t + (l & 31)) * 4u : kPast);
+    return v;
+  });
   __syncthreads();
 
   const int64_t step = (int64_t)gridDim.x * (kThreads / 64);
@@ -604,13 +622,18 @@ void run_mlp_forward(const float* z, const float* w1, const float* b1, const flo
   if (rows == 0) return;
   const int64_t tiles = (rows + kT - 1) / kT;
   with_groups<kMaxMlpIn / 8>((nin + 7) / 8, [&](auto gc) {
-    constexpr int G = decltype(gc)::value, T = forward_threads(G);
-    if (nout <= kT)
-      hipLaunchKernelGGL((k_mlp_forward<G, 1>), tile_grid(tiles, T), dim3(T), 0, st, z, w1, b1, w2, b2, a, y, rows,
-                         nin, nout, tiles);
-    else
-      hipLaunchKernelGGL((k_mlp_forward<G, 2>), tile_grid(tiles, T), dim3(T), 0, st, z, w1, b1, w2, b2, a, y, rows,
-                         nin, nout, tiles);
+    constexpr int G = decltype(gc)::value;
+    auto launch = [&](auto ot, auto threads) {
+      constexpr int T = decltype(threads)::value;
+      hipLaunchKernelGGL((k_mlp_forward<G, decltype(ot)::value, T>), tile_grid(tiles, T), dim3(T), 0, st, z, w1, b1,
+                         w2, b2, a, y, rows, nin, nout, tiles);
+    };
+    with_groups<2>(nout <= kT ? 1 : 2, [&](auto ot) {
+      if constexpr (forward_threads(G, kMaxMlpRows) == 512) {
+        if (forward_threads(G, tiles) == 512) return launch(ot, std::integral_constant<int, 512>{});
+      }
+      launch(ot, std::integral_constant<int, 256>{});
+    });
   });
   SPHOPS_LAUNCHED();
 }

@@ -127,3 +127,34 @@ def test_pre_activations_only_for_a_backward(monkeypatch):
         p.requires_grad_(False)
     M.mlp(net, z)
     assert kept == [False, False, True, False] and torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("rows,shape", [(300001, (83, 19)), (300001, (100, 16)), (300001, (163, 40)), (32769, (163, 40)),
+                                        (32800, (130, 32))])
+def test_many_rows_match_float64(rows, shape):
+    """Every wave's second and later row tiles, the moves of the second
+    layer's sums to LDS, ragged last chunks, and both sides of the forward's
+    two workgroup sizes.  The sums' 2-norms are within 4e-6, ten times what
+    their roundings measure; a row tile left out or read twice is off by
+    (32 / rows)^(1/2), 1e-2."""
+    from npa_amd import mlp as M
+    nin, nout = shape
+    net, z, up = _case(rows, nin, nout, True, nin)
+    w1, b1, w2, b2 = (t.detach().double() for t in (net[0].weight, net[0].bias, net[2].weight, net[2].bias))
+    zd = z.double()
+    a = zd @ w1.T + b1
+    up[(a.abs() < 1e-5).any(1)] = 0
+    zr = z.clone().requires_grad_(True)
+    y = M.mlp(net, zr)
+    y.backward(up)
+    with torch.no_grad():
+        assert torch.equal(M.mlp(net, z), y)
+    h, ud = a.clamp_min(0), up.double()
+    da = (ud @ w2) * (a > 0)
+    for name, got, ref in (("y", y, h @ w2.T + b2), ("dz", zr.grad, da @ w1), ("dW1", net[0].weight.grad, da.T @ zd),
+                           ("db1", net[0].bias.grad, da.sum(0)), ("dW2", net[2].weight.grad, ud.T @ h),
+                           ("db2", net[2].bias.grad, ud.sum(0))):
+        assert ((got.double() - ref).norm() <= 4e-6 * ref.norm()).item(), name
+    last = rows - rows % 32  # the ragged last row tile, row by row
+    for got, ref in ((y, h @ w2.T + b2), (zr.grad, da @ w1)):
+        assert torch.all((got[last - 32:].double() - ref[last - 32:]).abs() <= 1e-5 * ref.abs().max())
