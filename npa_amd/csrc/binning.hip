@@ -906,7 +906,7 @@ void fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st) {
 //
 // Stable partition of the binned particles into kNumClasses classes by
 // neighbour-list length (kListClasses), which the pair kernels serve with
-// groups of kListGroups (or kSplitGroups) lanes per particle.  The partition
+// groups of lanes per particle (kListTable, split_table).  The partition
 // is done per tile of 4096 binned particles and the tiles stay in order
 // (tile-major: every class of a region of space is processed together, so
 // neighbour rows shared between classes are reused from the same L2).
@@ -973,6 +973,25 @@ __global__ __launch_bounds__(kCountThreads) void k_class_count(const int32_t* __
 // log2 of the items a wave holds at g lanes per item (64 / g, a power of two).
 __device__ __forceinline__ uint32_t wave_items_log2(int32_t g) { return (uint32_t)(__clz(g) - 25); }
 
+// Lanes a particle for a class at `factor` times its base size.
+__device__ __forceinline__ int32_t wide_group(const GroupTable& gt, int q, int32_t factor) {
+  const int32_t cap = q == 0 && factor < 4 ? gt.short_cap : gt.cap.g[q];
+  return max(gt.base.g[q], min(gt.base.g[q] * factor, cap));
+}
+
+// How much wider a table's groups are, from the items of the thread's class
+// (class threadIdx.x % kNumClasses) in all tiles; the same in every thread.
+__device__ __forceinline__ int32_t group_factor(const GroupTable& gt, uint32_t items) {
+  const uint32_t q = threadIdx.x % kNumClasses;
+  uint32_t lanes = 0;
+#pragma unroll
+  for (int u = 0; u < kNumClasses; ++u) lanes = q == (uint32_t)u ? items * (uint32_t)gt.base.g[u] : lanes;
+#pragma unroll
+  for (int off = 1; off < kNumClasses; off <<= 1) lanes += __shfl_xor(lanes, off, kNumClasses);
+  const uint32_t w = lanes / kWave;
+  return w < gt.widest ? 4 : w < gt.wide ? 2 : 1;
+}
+
 // Stable scatter of a tile's items into order, class by class, and the wave
 // descriptors of the tile's segments.  The tile first finds its segment
 // offsets (segment s = tile * kNumClasses + class, in tile-major order): the
@@ -990,8 +1009,8 @@ template <bool CSR>
 __global__ __launch_bounds__(kCountThreads) void k_class_scatter(const int32_t* __restrict__ src, uint32_t n,
                                                             ClassBounds cb, const uint32_t* __restrict__ cnt,
                                                             uint32_t* __restrict__ seg,
-                                                            int32_t* __restrict__ order, GroupSizes gs1,
-                                                            GroupSizes gs2, int tables, uint2* __restrict__ waves1,
+                                                            int32_t* __restrict__ order, GroupTable gt1,
+                                                            GroupTable gt2, int tables, uint2* __restrict__ waves1,
                                                             uint2* __restrict__ waves2,
                                                             int32_t* __restrict__ total1,
                                                             int32_t* __restrict__ total2,
@@ -1003,16 +1022,31 @@ __global__ __launch_bounds__(kCountThreads) void k_class_scatter(const int32_t* 
   __shared__ uint32_t wbase[2][kNumClasses];
   __shared__ uint32_t part[3][kWaves];
   const int wave = threadIdx.x >> 6, lane = __lane_id();
-  if (threadIdx.x < kWaves * kNumClasses) (&wcnt[0][0])[threadIdx.x] = 0;
+  int32_t f1 = 1, f2 = 1;  // how much wider than their base the tables' groups are
   {
     static_assert(kCountThreads % kNumClasses == 0, "a thread's counts are all of one class");
     const uint32_t before = blockIdx.x * (uint32_t)kNumClasses, q = threadIdx.x % kNumClasses;
     const uint32_t mine = cnt[before + q];  // the tile's own count of class q
+    if (n <= kWideParticles) {
+      static_assert(kWideParticles / kTile * kNumClasses <= kCountThreads, "one count a thread");
+      uint32_t c = threadIdx.x < gridDim.x * kNumClasses ? cnt[threadIdx.x] : 0u;
+#pragma unroll
+      for (int off = kNumClasses; off < kWave; off <<= 1) c += __shfl_xor(c, off, kWave);
+      if (lane < kNumClasses) wcnt[wave][lane] = c;
+      __syncthreads();
+      uint32_t items = 0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) items += wcnt[w][q];
+      f1 = group_factor(gt1, items);
+      f2 = group_factor(gt2, items);
+      __syncthreads();
+    }
+    if (threadIdx.x < kWaves * kNumClasses) (&wcnt[0][0])[threadIdx.x] = 0;
     uint32_t l1 = 0, l2 = 0;
 #pragma unroll
     for (int u = 0; u < kNumClasses; ++u) {
-      l1 = q == (uint32_t)u ? wave_items_log2(gs1.g[u]) : l1;
-      l2 = q == (uint32_t)u ? wave_items_log2(gs2.g[u]) : l2;
+      l1 = q == (uint32_t)u ? wave_items_log2(wide_group(gt1, u, f1)) : l1;
+      l2 = q == (uint32_t)u ? wave_items_log2(wide_group(gt2, u, f2)) : l2;
     }
     const uint32_t r1 = (1u << l1) - 1u, r2 = (1u << l2) - 1u;
     uint32_t s = 0, w1 = 0, w2 = 0;
@@ -1116,15 +1150,17 @@ __global__ __launch_bounds__(kCountThreads) void k_class_scatter(const int32_t* 
   }
   // the descriptors of the tile's segments, table by table
   for (int tb = 0; tb < tables; ++tb) {
-    const GroupSizes& gs = tb == 0 ? gs1 : gs2;
+    const GroupTable& gt = tb == 0 ? gt1 : gt2;
+    const int32_t f = tb == 0 ? f1 : f2;
     uint2* __restrict__ waves = tb == 0 ? waves1 : waves2;
 #pragma unroll
     for (int q = 0; q < kNumClasses; ++q) {
       const uint32_t lo = gbase[q], c = gcnt[q], at = wbase[tb][q];
-      const uint32_t lg = wave_items_log2(gs.g[q]), per = 1u << lg;
+      const int32_t wide = wide_group(gt, q, f);
+      const uint32_t lg = wave_items_log2(wide), per = 1u << lg;
       const uint32_t nw = (c + per - 1) >> lg;
       for (uint32_t u = threadIdx.x; u < nw; u += kCountThreads)
-        waves[at + u] = make_uint2(lo + u * per, ((uint32_t)gs.g[q] << 8) | min(per, c - u * per));
+        waves[at + u] = make_uint2(lo + u * per, ((uint32_t)wide << 8) | min(per, c - u * per));
     }
   }
 }
@@ -1132,8 +1168,8 @@ __global__ __launch_bounds__(kCountThreads) void k_class_scatter(const int32_t* 
 // Tile-major schedule: per tile of 4096 binned particles a stable partition
 // by length class, tiles in order, plus one descriptor per 64-lane wave.
 template <bool CSR>
-void tiled_schedule(const Grid& g, const int32_t* src, const ClassBounds& cb, const GroupSizes& gs, int32_t* order,
-                    uint2* waves, int32_t* wave_total, hipStream_t st, const GroupSizes* gs2 = nullptr,
+void tiled_schedule(const Grid& g, const int32_t* src, const ClassBounds& cb, const GroupTable& gt, int32_t* order,
+                    uint2* waves, int32_t* wave_total, hipStream_t st, const GroupTable* gt2 = nullptr,
                     uint2* waves2 = nullptr, int32_t* wave_total2 = nullptr, const FillTail* tail = nullptr) {
   const uint32_t n = (uint32_t)g.n_keys;
   const uint32_t ntiles = (uint32_t)g.n_tiles;
@@ -1146,9 +1182,8 @@ void tiled_schedule(const Grid& g, const int32_t* src, const ClassBounds& cb, co
                      tail ? g.stripes : nullptr, tail ? tail->stripes : 0u, tail ? tail->total : nullptr);
   SPHOPS_LAUNCHED();
   const int tables = waves2 != nullptr ? 2 : 1;  // a second table: same order, other group sizes
-  const GroupSizes gsb = gs2 != nullptr ? *gs2 : gs;
-  hipLaunchKernelGGL((k_class_scatter<CSR>), dim3(ntiles), dim3(kCountThreads), 0, st, src, n, cb, cnt, seg, order, gs,
-                     gsb, tables, waves, tables == 2 ? waves2 : waves, wave_total,
+  hipLaunchKernelGGL((k_class_scatter<CSR>), dim3(ntiles), dim3(kCountThreads), 0, st, src, n, cb, cnt, seg, order, gt,
+                     gt2 != nullptr ? *gt2 : gt, tables, waves, tables == 2 ? waves2 : waves, wave_total,
                      tables == 2 ? wave_total2 : wave_total,
                      tail ? reinterpret_cast<const uint32_t*>(tail->total) : nullptr, tail ? tail->host : nullptr);
   SPHOPS_LAUNCHED();
@@ -1160,15 +1195,14 @@ uint64_t neighbour_wave_capacity(const Grid& g) { return g.n_keys + (uint64_t)kN
 
 void run_split_schedule(const Grid& g, const int32_t* len, int32_t* order, uint2* waves, int32_t* wave_total,
                         hipStream_t st) {
-  tiled_schedule<false>(g, len, kListClasses, group_sizes(kSplitGroups, kSplitGroupCaps, g.n_keys), order, waves,
-                        wave_total, st);
+  tiled_schedule<false>(g, len, kListClasses, split_table(g.dim), order, waves, wave_total, st);
 }
 
 void run_neighbour_schedule(const Grid& g, const int32_t* ncnt, int32_t* order, uint2* waves, int32_t* wave_total,
                             uint2* waves2, int32_t* wave_total2, hipStream_t st, const FillTail* tail) {
-  const GroupSizes split = group_sizes(kSplitGroups, kSplitGroupCaps, g.n_keys);
-  tiled_schedule<false>(g, ncnt, kListClasses, group_sizes(kListGroups, kListGroupCaps, g.n_keys), order, waves,
-                        wave_total, st, &split, waves2, wave_total2, tail);
+  const GroupTable split = split_table(g.dim);
+  tiled_schedule<false>(g, ncnt, kListClasses, kListTable, order, waves, wave_total, st, &split, waves2, wave_total2,
+                        tail);
 }
 
 namespace {

@@ -161,7 +161,7 @@ struct OpPtrs {
   const int32_t* order = nullptr; // particles in schedule order (optional, list traversal)
   const uint2* waves = nullptr;   // per-wave descriptors {first slot in order, group size << 8 | particles}
   uint32_t nwaves = 0;
-  const uint2* waves2 = nullptr;  // descriptors for lane-split channel kernels (group sizes kSplitGroups)
+  const uint2* waves2 = nullptr;  // descriptors for lane-split channel kernels (split_table)
   uint32_t nwaves2 = 0;
   // optional device copies of the wave counts; when set the kernels read them
   // and nwaves / nwaves2 only size the launch (an upper bound)
@@ -190,7 +190,7 @@ void run_forward(const Grid& g, Op op, const int32_t* bin_offsets, const OpPtrs&
 void run_backward(const Grid& g, Op op, bool full, const int32_t* bin_offsets, const OpPtrs& a,
                   hipStream_t st);
 // Pair-kernel schedule: per tile of 4096 binned particles, a stable partition
-// by neighbour-list length class (kListClasses / kListGroups), tiles in
+// by neighbour-list length class (kListClasses), tiles in
 // order; one descriptor per wave {first slot in order, group size << 8 | particles}.
 // With `tail` the schedule's kernels also finish the fill before them: its
 // pair totals go to tail->total (the first kernel, see fill_totals), and,
@@ -203,7 +203,7 @@ struct FillTail {
 };
 void run_neighbour_schedule(const Grid& g, const int32_t* ncnt, int32_t* order, uint2* waves, int32_t* wave_total,
                             uint2* waves2, int32_t* wave_total2, hipStream_t st, const FillTail* tail = nullptr);
-// The split-group schedule alone (kSplitGroups) over lengths `len`; items of
+// The split-group schedule alone (split_table) over lengths `len`; items of
 // negative length are left out.
 void run_split_schedule(const Grid& g, const int32_t* len, int32_t* order, uint2* waves, int32_t* wave_total,
                         hipStream_t st);
@@ -263,27 +263,36 @@ constexpr GroupSizes kListGroups{{1, 1, 2, 4, 8, 16, 32, 64}};
 // lane-split channel kernels: four lanes (channel slices) per pair stream,
 // 1, 1, 1, 1, 4, 8, 16, 16 streams per particle (about 12-48 pairs each)
 constexpr GroupSizes kSplitGroups{{4, 4, 4, 4, 16, 32, 64, 64}};
-// Groups for fewer particles, twice as wide up to kWideParticles and four
-// times up to kWidestParticles, but no wider than one step of the kernel
-// takes of a class's longest row: at the sizes above, that few particles are
-// no more than two rounds of the waves the chip holds (kWideParticles in
-// groups of 4 lanes: 8192), and the launch lasts as long as its longest
-// rows.  Pass-B backward, 1x / 2x / 4x: 108 / 87 / 88 us (65536 particles,
-// 3D, C = 32), 84 / 66 / 65 (3 x 20011, 3D periodic, C = 20), 106 / 95 / 102
-// (131072, C = 16); its forward 9.7 / 7.3 / 6.4 us at 4096 particles, but 64
-// / 74 / 88 at 250007.
+// Few waves leave the chip idle and the launch as long as its longest rows:
+// groups then are two or four times as wide, but no wider than one step of the
+// kernel takes of a class's longest row (short_cap: class 0's at twice).
+// Whether they are depends on the waves W that the sizes above give, known
+// where the schedule is made (whole table, in 64 lanes): four times below W =
+// widest, twice below wide.  Times of the operators in groups 2x and 4x as
+// wide, as a share of 1x, geometric mean over 8 to 32 channels, forward and
+// backward, periodic, clamped and Gaussian clouds of 20 to 90 neighbours, and
+// the largest:
+//   split table, W 250: .69, .85 (4x .56, .77); 1050: .81, 1.02 (4x .75, .97);
+//   2070: .88, 1.11 (4x .92, 1.19); 2D 2780: .98, 1.18; 3150: 1.02, 1.18;
+//   4050: 1.05, 1.22; 5050: 1.0, 1.16; 6300: .95, 1.09; 8200: .97, 1.11; 3D
+//   2780: .93, 1.15; 4050: .95, 1.19; 5050: .91, 1.1; 6300: .88, 1.08; 8200:
+//   .88, 1.06; 90 neighbours 8080: .96, 1.14, 8550: 1.08, 1.24, 20000 and
+//   more: 1.03-1.2, 1.36.
+//   list table, densities, W 250: .78-.87 (4x .68-.78); 1000: .82-.9; 3800:
+//   .9-1; 4300-5100: 1.05-1.1; 20000: 1.2.  But its widest kernels (48
+//   channels), W 260: .63, .73 (4x .5, .71); 320: .64, .75 (4x .77, 1.14);
+//   515: .67, .85; 620: 1.06, 1.31; 1900: 1.1, 1.4, and they take twenty times
+//   as long: the list's limits are theirs.
+// Above kWideParticles W is past every limit.
 constexpr uint64_t kWideParticles = 1ull << 17;
-constexpr uint64_t kWidestParticles = 1ull << 13;
-constexpr GroupSizes kListGroupCaps{{2, 4, 8, 16, 32, 64, 64, 64}};
-constexpr GroupSizes kSplitGroupCaps{{8, 16, 32, 64, 64, 64, 64, 64}};
-inline GroupSizes group_sizes(const GroupSizes& base, const GroupSizes& caps, uint64_t particles) {
-  const int f = particles <= kWidestParticles ? 4 : particles <= kWideParticles ? 2 : 1;
-  GroupSizes r = base;
-  for (int q = 0; q < kNumClasses; ++q) {
-    const int32_t wide = base.g[q] * f < caps.g[q] ? base.g[q] * f : caps.g[q];
-    if (wide > r.g[q]) r.g[q] = wide;
-  }
-  return r;
+struct GroupTable {
+  GroupSizes base, cap;
+  int32_t short_cap;
+  uint32_t widest, wide;
+};
+constexpr GroupTable kListTable{kListGroups, {{2, 4, 8, 16, 32, 64, 64, 64}}, 2, 288, 576};
+constexpr GroupTable split_table(int dim) {
+  return {kSplitGroups, {{8, 16, 32, 64, 64, 64, 64, 64}}, 4, 1536, dim == 2 ? 2560u : 8448u};
 }
 void run_safe_inv(const float* in, float* out, uint64_t count, int dim, float tol, hipStream_t st);
 void fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t st);
