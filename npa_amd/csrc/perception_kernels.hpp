@@ -2485,6 +2485,24 @@ inline bool split_ok(const Grid& g, const OpPtrs& a) {
   return (a.C == 8 || a.C == 12 || a.C == 20 || a.C == 24) && row_offsets_fit_32(g, a.C);
 }
 
+// Rows of 12 channels on 16-byte bases, three vectors a row, that blur alone
+// and the backward of a single operator read faster with a row per lane (the
+// grouped kernels) above this many particles.  Lane-split as a share of
+// grouped at 4096, 16384, 65536 and 524288 particles, 2D and 3D, periodic,
+// clamped and Gaussian clouds of 30 neighbours, then of 90 (at 4096, 16384 and
+// 524288): blur .58-.73, .68-.87, .81-.96, .84-1.07; .69-.9, up to 1.1,
+// 1.03-1.29; its backward .62-.72, .72-.87, .82-1.0, .83-1.08; .68-.88,
+// 1.08-1.4, 1.03-1.27, to the states only .69-.83, .74-.98, 1.02-1.23,
+// 1.14-1.61; .71-.99, 1.07-1.67, 1.5-1.99; the gradient's backward .59-.7,
+// .72-.97, .86-1.05, 1.01-1.17; .68-.87, up to 1.34, 1.04-1.21, to the states
+// only .63-.72, .75-.91, .79-.99, 1.01-1.16; .67-.92, up to 1.39, 1.07-1.27.
+// The gradients' forward (.56-1.0; up to 1.15) and the fused pass (.35-1.1)
+// stay.
+constexpr uint64_t kGrouped12Particles = 1ull << 12;
+inline bool grouped_rows(const Grid& g, const OpPtrs& a) {
+  return a.C == 12 && g.n_keys > kGrouped12Particles && aligned16(a.s) && aligned16(a.g) && aligned16(a.g2);
+}
+
 // The lane-split launchers (perception_pass_b.hpp, compiled in translation
 // units of their own): over the schedule a.waves2, positions and volumes
 // already packed into a.xw; parts as the kernels' PARTS.
@@ -2592,7 +2610,8 @@ void forward_dispatch(const Grid& g, Op op, const int32_t* bo, const OpPtrs& a_i
       // channels, where it is faster than the lane-split kernel (0.28 against
       // 0.30 ms at cfg5); at the other widths the lane-split kernel gives the
       // bits of the fused pass
-      if (a.C != 16 && a.C != 32 && split_ok(g, a)) return launch_blur_hybrid_fwd_quad<D, P, 1>(g, a, st);
+      if (a.C != 16 && a.C != 32 && split_ok(g, a) && !grouped_rows(g, a))
+        return launch_blur_hybrid_fwd_quad<D, P, 1>(g, a, st);
       return launch_channels<D, P, OpBlur>(g, bo, a, st);
     case Op::Gradient: {
       // over a neighbour list: the lane-split kernel without the moment matrix
@@ -2639,7 +2658,7 @@ void backward_dispatch(const Grid& g, Op op, bool full, const int32_t* bo, const
     case Op::MomentMatrix: return launch_pairs<D, P, OpMomentMatrixBwd<D, P>>(g, bo, a, st);
     case Op::Blur:
       // over a neighbour list: the lane-split kernel with the blur terms only
-      if (split_ok(g, a)) {
+      if (split_ok(g, a) && !grouped_rows(g, a)) {
         if (full) return launch_blur_hybrid_bwd_quad<D, P, true, 1>(g, a, st);
         return launch_blur_hybrid_bwd_quad<D, P, false, 1>(g, a, st);
       }
@@ -2651,7 +2670,7 @@ void backward_dispatch(const Grid& g, Op op, bool full, const int32_t* bo, const
       OpPtrs b = a;
       b.g2 = a.g;
       b.g = nullptr;
-      if (split_ok(g, b)) {
+      if (split_ok(g, b) && !grouped_rows(g, b)) {
         if (full) return launch_blur_hybrid_bwd_quad<D, P, true, 2>(g, b, st);
         return launch_blur_hybrid_bwd_quad<D, P, false, 2>(g, b, st);
       }
