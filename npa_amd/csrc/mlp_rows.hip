@@ -23,9 +23,9 @@
 //
 // Forward and input gradient keep their weights in LDS as operand images (one
 // 16-byte read a lane feeds four matrix instructions) and walk row tiles of
-// 32, one per wave at a time.  Bounds: 232 matrix instructions of 64 cycles a
-// tile forward, 240 for the input gradient, 304 for the weight gradients: 0.2
-// + 0.2 + 0.26 ms for 2^20 rows of 83 -> 128 -> 19, beside 0.19 ms of memory
+// 32, one per wave at a time.  Bounds: 240 matrix instructions of 64 cycles a
+// tile forward (padding included), 240 for the input gradient, 304 for the
+// weight gradients: 0.2 + 0.2 + 0.26 ms for 2^20 rows of 83 -> 128 -> 19, beside 0.19 ms of memory
 // traffic for each of the first two.  Measured inside a training step: 0.30 +
 // 0.28 + 0.36 ms, where the separate kernels took 0.51 (library product,
 // ReLU + second layer), 0.66 (its input gradient, library product) and 0.39;

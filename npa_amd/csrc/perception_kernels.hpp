@@ -2335,7 +2335,7 @@ void neighbour_candidates(const Grid& g, const int32_t* bo, const float* x, hipS
 
 // Fill the rows (compact, allocated from the striped counters) with the work
 // split neighbour_candidates left in the grid; used[0..1] receive the pair
-// totals (k_fill_totals).
+// totals (fill_totals).
 // With ft.own set, the rows keep the own-cell entries of the tiles last
 // (FillTiles); ft.count is cleared here.
 template <int D, bool P>
@@ -2351,8 +2351,8 @@ void neighbour_fill(const Grid& g, const int32_t* bo, const float* x, int32_t* n
     xw = g.packed;
   }
   const uint32_t S = fill_stripes(n, cap);
-  // the counters are zero here: zeroed at grid creation and by the totals
-  // kernel of every fill
+  // the counters are zero here: zeroed at grid creation and where the totals
+  // of every fill are taken (fill_totals)
   FillStripes fs{g.stripes, S - 1, (uint64_t)(cap / S)};
   const bool ot = ft.own != nullptr;
   if (ot) fill_u32(reinterpret_cast<uint32_t*>(ft.count), 1, 0u, st);

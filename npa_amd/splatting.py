@@ -4,9 +4,10 @@ reference) on the HIP kernels of libsphops_hip.so.
 ``splat_particles``, ``splat_particles_batch`` and ``splat_particles_sections``
 take the reference's arguments and return its images ((H, W, 4) or
 (images, H, W, 4), channels [r, g, b, density]).  All images of a call are
-one launch.  The forward gathers per 16 x 16 tile in ascending particle order
-and the backward sums per particle, so results are deterministic (the
-reference's scatter_add_ is not).  Positions and colours are float32 on the
+one launch.  The forward gathers per 16 x 16 tile, each of four waves its share
+of the particles in ascending order, and adds the four in a fixed order; the
+backward sums per particle, so results are deterministic (the reference's
+scatter_add_ is not).  Positions and colours are float32 on the
 GPU; only the last three colour channels receive a gradient, as in the
 reference.
 """
