@@ -471,7 +471,8 @@ int sphops_splat_backward(const float* x, const float* color, const int32_t* sta
 
 /* The same, tile by tile where sphops_splat_backward_workspace_bytes of these
  * arguments is not 0: workspace holds that many bytes, 16-byte aligned (NULL:
- * as sphops_splat_backward). */
+ * as sphops_splat_backward).  Images whose particles crowd in few tiles are
+ * found on the device and served as there. */
 int sphops_splat_backward_tiled(const float* x, const float* color, const int32_t* starts, int64_t images,
                                 int64_t particles, int ncolor, int img_size, double sigma, double lo, double hi,
                                 int normalize_color, int y_up, double pixel_size, const float* d_out, float* d_x,

@@ -85,6 +85,10 @@ __device__ __forceinline__ T wave_sum(T v) {
 // reads 8 bytes of each.
 constexpr int kNoPatch = -(1 << 30);
 
+// Share of an image's tiles that have to do the work for the tile by tile
+// backward (measurements with its other limits, below).
+constexpr float kTilesMinShare = 0.5f;
+
 struct SplatRecords {
   float4* __restrict__ col;
   int2* __restrict__ centre;
@@ -94,10 +98,9 @@ struct SplatRecords {
         frac(reinterpret_cast<float2*>(centre + n)) {}
 };
 
-__global__ __launch_bounds__(256) void k_splat_prep(SplatParams sp, const float* __restrict__ x,
-                                                    const float* __restrict__ color, int64_t n, SplatRecords rec) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
+__device__ __forceinline__ void prepare_particle(const SplatParams& sp, const float* __restrict__ x,
+                                                 const float* __restrict__ color, int64_t i,
+                                                 const SplatRecords& rec) {
   int bx = 0, by = 0;
   float fx = 0.0f, fy = 0.0f;
   const bool live = particle_setup(sp, x[2 * i], x[2 * i + 1], bx, by, fx, fy);
@@ -114,6 +117,12 @@ __global__ __launch_bounds__(256) void k_splat_prep(SplatParams sp, const float*
   rec.centre[i] = make_int2(live ? bx : kNoPatch, by);
   rec.frac[i] = make_float2(fx, fy);
   rec.col[i] = make_float4(c[0] * k, c[1] * k, c[2] * k, k);
+}
+
+__global__ __launch_bounds__(256) void k_splat_prep(SplatParams sp, const float* __restrict__ x,
+                                                    const float* __restrict__ color, int64_t n, SplatRecords rec) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) prepare_particle(sp, x, color, i, rec);
 }
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -343,6 +352,36 @@ __device__ __forceinline__ void store_gradients(const SplatParams& sp, int64_t i
   }
 }
 
+// A particle's sums over its patch, by a whole wave.
+__device__ __forceinline__ PatchSums sweep_patch(const SplatParams& sp, int bx, int by, float fx, float fy, float cr,
+                                                 float cg, float cb, const float4* __restrict__ dimg, int lane) {
+  const int r = sp.r, P = 2 * r + 1, H = sp.H;
+  PatchSums t;
+  for (int q = lane; q < P * P; q += 64) {
+    const int qy = q / P, qx = q - qy * P;
+    const int ix = bx + qx - r, iy = by + qy - r;
+    if (ix >= 0 && ix < H && iy >= 0 && iy < H) {
+      const float ax = (float)(qx - r) - fx, ay = (float)(qy - r) - fy;
+      const float g = gauss(ax, ay, sp.inv_two_s2);
+      const float4 d = dimg[(int64_t)iy * H + ix];
+      const float G = cr * d.x + cg * d.y + cb * d.z + d.w;
+      t.dr += g * d.x;
+      t.dg += g * d.y;
+      t.db += g * d.z;
+      t.gg += G * g;
+      t.ggx += G * g * ax;
+      t.ggy += G * g * ay;
+    }
+  }
+  t.dr = wave_sum(t.dr);
+  t.dg = wave_sum(t.dg);
+  t.db = wave_sum(t.db);
+  t.gg = wave_sum(t.gg);
+  t.ggx = wave_sum(t.ggx);
+  t.ggy = wave_sum(t.ggy);
+  return t;
+}
+
 __global__ __launch_bounds__(64 * kBwdWaves) void k_splat_backward(SplatParams sp, const float* __restrict__ x,
                                                                    const float* __restrict__ color,
                                                                    const int32_t* __restrict__ starts, int images,
@@ -356,37 +395,14 @@ __global__ __launch_bounds__(64 * kBwdWaves) void k_splat_backward(SplatParams s
   float fx = 0.0f, fy = 0.0f;
   const bool live = particle_setup(sp, x[2 * i], x[2 * i + 1], bx, by, fx, fy);
   const float* c = color + i * sp.ncolor + (sp.ncolor - 3);
-  const float cr = c[0], cg = c[1], cb = c[2];
-  const int r = sp.r, P = 2 * r + 1, H = sp.H;
   PatchSums t;
   AxisSums a;
-  if (live) {
+  if (live) {  // wave-uniform
     const int b = image_of(starts, images, (int)i);
-    const float4* dimg = reinterpret_cast<const float4*>(d_img) + (int64_t)b * H * H;
-    for (int q = lane; q < P * P; q += 64) {
-      const int qy = q / P, qx = q - qy * P;
-      const int ix = bx + qx - r, iy = by + qy - r;
-      if (ix >= 0 && ix < H && iy >= 0 && iy < H) {
-        const float ax = (float)(qx - r) - fx, ay = (float)(qy - r) - fy;
-        const float g = gauss(ax, ay, sp.inv_two_s2);
-        const float4 d = dimg[(int64_t)iy * H + ix];
-        const float G = cr * d.x + cg * d.y + cb * d.z + d.w;
-        t.dr += g * d.x;
-        t.dg += g * d.y;
-        t.db += g * d.z;
-        t.gg += G * g;
-        t.ggx += G * g * ax;
-        t.ggy += G * g * ay;
-      }
-    }
+    t = sweep_patch(sp, bx, by, fx, fy, c[0], c[1], c[2],
+                    reinterpret_cast<const float4*>(d_img) + (int64_t)b * sp.H * sp.H, lane);
     if (sp.normalize) a = axis_sums(sp, fx, fy, lane, 64);
   }
-  t.dr = wave_sum(t.dr);
-  t.dg = wave_sum(t.dg);
-  t.db = wave_sum(t.db);
-  t.gg = wave_sum(t.gg);
-  t.ggx = wave_sum(t.ggx);
-  t.ggy = wave_sum(t.ggy);
   if (live && sp.normalize) {  // wave-uniform
     a.sx = wave_sum(a.sx);
     a.sy = wave_sum(a.sy);
@@ -394,6 +410,64 @@ __global__ __launch_bounds__(64 * kBwdWaves) void k_splat_backward(SplatParams s
     a.sya = wave_sum(a.sya);
   }
   store_gradients(sp, i, live, t, a, lane, 64, d_x, d_color);
+}
+
+__device__ __forceinline__ int first_tile(int c, int r) { return max(0, c - r) / kTile; }
+__device__ __forceinline__ int last_tile(int c, int r, int H) { return c + r < 0 ? -1 : min(H - 1, c + r) / kTile; }
+
+// The records for the backward, and for each image whether its particles
+// crowd in few tiles (crowded[its first particle]; the first `images`
+// workgroups).  With h_t the particles that reach tile t, (sum h)^2 / sum h^2
+// is the number of tiles that do the work; sum h is a mean over particles of
+// the tiles that one reaches, sum h^2 one over pairs of the tiles that both
+// reach, taken here from 256 particles, evenly spaced in the image's order,
+// and 32 partners each.
+constexpr int kLookPairs = 32;
+
+__global__ __launch_bounds__(256) void k_splat_backward_prep(SplatParams sp, const float* __restrict__ x,
+                                                             const float* __restrict__ color,
+                                                             const int32_t* __restrict__ starts, int images,
+                                                             int64_t n, SplatRecords rec, int* __restrict__ crowded) {
+  if ((int)blockIdx.x >= images) {
+    const int64_t i = (int64_t)(blockIdx.x - images) * 256 + threadIdx.x;
+    if (i < n) prepare_particle(sp, x, color, i, rec);
+    return;
+  }
+  __shared__ int4 reach[256];  // first and last tile, x and y
+  __shared__ int sums[2][4];
+  const int p0 = starts[blockIdx.x], size = starts[blockIdx.x + 1] - p0, m = min(size, 256), t = threadIdx.x;
+  if (m <= 0) return;
+  auto shared_tiles = [](int4 u, int4 v) {
+    return max(0, min(u.y, v.y) - max(u.x, v.x) + 1) * max(0, min(u.w, v.w) - max(u.z, v.z) + 1);
+  };
+  int4 mine = make_int4(1, 0, 1, 0);
+  if (t < m) {
+    const int64_t i = p0 + (int64_t)t * size / m;
+    int bx, by;
+    float fx, fy;
+    if (particle_setup(sp, x[2 * i], x[2 * i + 1], bx, by, fx, fy))
+      mine = make_int4(first_tile(bx, sp.r), last_tile(bx, sp.r, sp.H), first_tile(by, sp.r),
+                       last_tile(by, sp.r, sp.H));
+    reach[t] = mine;
+  }
+  __syncthreads();
+  int one = shared_tiles(mine, mine), both = 0;
+  if (t < m && m > 1) {
+    for (int j = 0; j < kLookPairs; ++j) both += shared_tiles(mine, reach[(t + 1 + j * (m - 1) / kLookPairs) % m]);
+  }
+  one = wave_sum(one);
+  both = wave_sum(both);
+  if (t % 64 == 0) {
+    sums[0][t / 64] = one;
+    sums[1][t / 64] = both;
+  }
+  __syncthreads();
+  if (t == 0) {
+    const float k = (float)(sums[0][0] + sums[0][1] + sums[0][2] + sums[0][3]) / (float)m;
+    const float k2 = (float)(sums[1][0] + sums[1][1] + sums[1][2] + sums[1][3]) / (float)(m * kLookPairs);
+    const float tiles = (float)((sp.H + kTile - 1) / kTile);
+    crowded[p0] = k * k < kTilesMinShare * tiles * tiles * k2 ? 1 : 0;
+  }
 }
 
 // The same sums tile by tile.  With d_c the tile's 16 x 16 pixels of channel c
@@ -408,19 +482,19 @@ __global__ __launch_bounds__(64 * kBwdWaves) void k_splat_backward(SplatParams s
 // the side * side that its patch can reach.  A wave takes every `waves`-th
 // turn of 64 of the image's particles; blockIdx.z is the image and the part
 // of the waves.  Non-finite colours or pixels, which zero weights do not
-// silence, are summed pixel by pixel.  8 images of 256^2, 4096 particles of
+// silence, are summed pixel by pixel; crowded images are left out.  8 images of 256^2, 4096 particles of
 // radius 20 px: 83 us a wave per particle (880 MB of pixels from the L2), 54
 // so and 11 for the records and their sum; storing a group's sums a group
 // later changes nothing.
-__device__ __forceinline__ int first_tile(int c, int r) { return max(0, c - r) / kTile; }
-
 __global__ __launch_bounds__(kTileThreads, 4) void k_splat_backward_tiles(SplatParams sp, SplatRecords rec,
                                                                           const int32_t* __restrict__ starts,
                                                                           int parts, int side,
                                                                           const float* __restrict__ d_img,
+                                                                          const int* __restrict__ crowded,
                                                                           float4* __restrict__ slots) {
   __shared__ int lists[kWavesPerTile][kListSlots];
   const int b = blockIdx.z / parts, part = blockIdx.z % parts;
+  if (starts[b] == starts[b + 1] || crowded[starts[b]]) return;
   const int tx0 = blockIdx.x * kTile, ty0 = blockIdx.y * kTile;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, kq = lane >> 4, ij = lane & 15;
   int* list = lists[wave];
@@ -546,24 +620,30 @@ __global__ __launch_bounds__(kTileThreads, 4) void k_splat_backward_tiles(SplatP
                      list, multiply);
 }
 
-// Adds a particle's records (16 lanes a particle, lane l the slots l, l + 16,
-// ... of the tiles its patch reaches) and turns them into gradients.
-__global__ __launch_bounds__(256) void k_splat_backward_sum(SplatParams sp, const float* __restrict__ x, int64_t n,
-                                                            int side, const float4* __restrict__ slots,
+// Adds a particle's records (L lanes a particle, lane l the slots l, l + L,
+// ... of the tiles its patch reaches) and turns them into gradients.  In
+// crowded images, which the tiles left out, the wave sweeps the patches of its
+// 64 / L particles instead, one after the other.
+template <int L>
+__global__ __launch_bounds__(256) void k_splat_backward_sum(SplatParams sp, SplatRecords rec,
+                                                            const int32_t* __restrict__ starts, int images, int64_t n,
+                                                            int side, const float* __restrict__ d_img,
+                                                            const int* __restrict__ crowded,
+                                                            const float4* __restrict__ slots,
                                                             float* __restrict__ d_x, float* __restrict__ d_color) {
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) / 16;
-  const int lane = threadIdx.x % 16;
-  if (i >= n) return;
-  int bx = 0, by = 0;
-  float fx = 0.0f, fy = 0.0f;
-  const bool live = particle_setup(sp, x[2 * i], x[2 * i + 1], bx, by, fx, fy);
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) / L;
+  const int lane = threadIdx.x % L, group = threadIdx.x % 64 / L;
+  const int2 at = i < n ? rec.centre[i] : make_int2(kNoPatch, 0);
+  const float2 f = i < n ? rec.frac[i] : make_float2(0.0f, 0.0f);
+  const bool live = at.x != kNoPatch;
+  const int image = live ? image_of(starts, images, (int)i) : 0;
+  const bool sweep = live && crowded[starts[image]] != 0;
   PatchSums t;
   AxisSums a;
-  if (live) {
-    const int last = (sp.H - 1) / kTile;
-    const int nx = bx + sp.r < 0 ? 0 : min(last, (bx + sp.r) / kTile) - first_tile(bx, sp.r) + 1;
-    const int ny = by + sp.r < 0 ? 0 : min(last, (by + sp.r) / kTile) - first_tile(by, sp.r) + 1;
-    for (int k = lane; k < side * side; k += 16) {
+  if (live && !sweep) {
+    const int fx = first_tile(at.x, sp.r), fy = first_tile(at.y, sp.r);
+    const int nx = last_tile(at.x, sp.r, sp.H) - fx + 1, ny = last_tile(at.y, sp.r, sp.H) - fy + 1;
+    for (int k = lane; k < side * side; k += L) {
       if (k % side < nx && k / side < ny) {
         const float4* o = slots + (i * side * side + k) * 2;
         const float4 u = o[0], v = o[1];
@@ -575,15 +655,28 @@ __global__ __launch_bounds__(256) void k_splat_backward_sum(SplatParams sp, cons
         t.ggy += v.y;
       }
     }
-    if (sp.normalize) a = axis_sums(sp, fx, fy, lane, 16);
+  }
+  if (live && sp.normalize) a = axis_sums(sp, f.x, f.y, lane, L);
+  const uint64_t sweeps = __ballot(sweep);
+  for (int u = 0; u < 64 / L; ++u) {
+    if (((sweeps >> (L * u)) & 1ull) == 0) continue;  // wave-uniform
+    const int64_t iu = i - group + u;
+    const int2 au = rec.centre[iu];
+    const float2 fu = rec.frac[iu];
+    const float4 cu = rec.col[iu];
+    const int bu = __shfl(image, L * u, 64);
+    const PatchSums w = sweep_patch(sp, au.x, au.y, fu.x, fu.y, cu.x, cu.y, cu.z,
+                                    reinterpret_cast<const float4*>(d_img) + (int64_t)bu * sp.H * sp.H,
+                                    threadIdx.x % 64);
+    if (group == u && lane == 0) t = w;  // the group adds its lanes' below
   }
   float* s[10] = {&t.dr, &t.dg, &t.db, &t.gg, &t.ggx, &t.ggy, &a.sx, &a.sy, &a.sxa, &a.sya};
 #pragma unroll
   for (int k = 0; k < 10; ++k) {
 #pragma unroll
-    for (int o = 8; o > 0; o >>= 1) *s[k] += __shfl_xor(*s[k], o, 16);
+    for (int o = L / 2; o > 0; o >>= 1) *s[k] += __shfl_xor(*s[k], o, L);
   }
-  store_gradients(sp, i, live, t, a, lane, 16, d_x, d_color);
+  if (i < n) store_gradients(sp, i, live, t, a, lane, L, d_x, d_color);
 }
 
 // The tile by tile backward serves patches up to kTilesMaxRadius whose pixels
@@ -591,12 +684,16 @@ __global__ __launch_bounds__(256) void k_splat_backward_sum(SplatParams sp, cons
 // with kTilesMinPixels of them in all its two further launches, with at most
 // kTilesMaxBytes of records.  Measured (us of the whole call, tiles against a
 // wave a particle; 4096 particles an image): 8 x 256^2 at radius 10 (14 M
-// pixels, search above) 41 and 39, at 20 (55 M) 51 and 75, at 32 (138 M) 71
-// and 150; 8 x 128^2 at 20 47 and 69; 1 x 512^2 at 32 (17 M) 45 and 37.
-// Particles all within a few tiles leave waves idle (a cloud a tenth as wide,
-// 8 x 256^2 at 20: 147 and 75, after a forward of 354 that took 1002);
-// kTilesBlocks workgroups, a share of the particles each, rather than one a
-// tile (231) bound that, and cost the even cloud 3.
+// pixels, search above) 41 and 39, at 16 (36 M) 58 and 59, at 20 (55 M) 63 and
+// 76, at 32 (138 M) 91 and 163; 8 x 128^2 at 20 59 and 71; 1 x 512^2 at 32 (17
+// M) 45 and 37.
+// Of those images it takes the ones at least kTilesMinShare of whose tiles do
+// the work (k_splat_backward_prep): in the others most of the chip waits for
+// the few tiles' waves.  Tiles against waves, shares .48-.56: 103-113 and
+// 148-156 (radius 32, 128^2); .45: 108 and 70 (10, 64^2); .33: 80 and 65 (20,
+// 128^2); .16: 110 and 65 (20, 256^2); .04: 397 and 156 (32, 512^2); .06: 203
+// and 70 (10, 128^2, 100 000 particles), now 83.  An image that is left to the
+// waves pays the look and the empty launch, 8 to 12 us up to 32 768 particles.
 constexpr int kTilesMaxRadius = 32;
 constexpr int64_t kTilesMinPixels = (int64_t)1 << 25;
 constexpr int64_t kTilesMaxBytes = (int64_t)1 << 30;
@@ -609,7 +706,7 @@ int tile_side(int r) { return (2 * r + kTile - 1) / kTile + 1; }
 
 int64_t splat_tiles_bytes(const SplatParams& sp, int64_t n) {
   const int64_t tiles = (sp.H + kTile - 1) / kTile, side = tile_side(sp.r), patch = 2 * sp.r + 1;
-  const int64_t bytes = n * 32 * (1 + side * side);
+  const int64_t bytes = n * (32 * (1 + side * side) + 4);
   return sp.r <= kTilesMaxRadius && n * patch * patch >= kTilesMinPixels && 2 * tiles * tiles <= patch * patch &&
                  bytes <= kTilesMaxBytes
              ? bytes
@@ -643,20 +740,29 @@ void run_splat_backward(const SplatParams& sp, const float* x, const float* colo
   raw.normalize = 0;  // the colours themselves
   const SplatRecords rec(work, n);
   float4* slots = static_cast<float4*>(work) + 2 * n;
-  hipLaunchKernelGGL(k_splat_prep, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, raw, x, color, n, rec);
-  SPHOPS_LAUNCHED();
   const uint32_t tiles = (uint32_t)((sp.H + kTile - 1) / kTile);
   const int side = tile_side(sp.r);
+  int* crowded = reinterpret_cast<int*>(slots + 2 * n * side * side);
+  hipLaunchKernelGGL(k_splat_backward_prep, dim3((uint32_t)((n + 255) / 256 + images)), dim3(256), 0, st, raw, x,
+                     color, starts, images, n, rec, crowded);
+  SPHOPS_LAUNCHED();
   const uint64_t blocks = (uint64_t)tiles * tiles * (uint64_t)images;
   // enough parts to fill the chip, each wave with two turns or more
   const uint64_t most = std::max<uint64_t>(1, (uint64_t)n / (uint64_t)images / (64 * 2 * kWavesPerTile));
   const int parts = (int)std::min<uint64_t>({most, std::max<uint64_t>(1, kTilesBlocks / blocks),
                                              65535ull / (uint64_t)images});
   hipLaunchKernelGGL(k_splat_backward_tiles, dim3(tiles, tiles, (uint32_t)(images * parts)), dim3(kTileThreads), 0,
-                     st, sp, rec, starts, parts, side, d_img, slots);
+                     st, sp, rec, starts, parts, side, d_img, crowded, slots);
   SPHOPS_LAUNCHED();
-  hipLaunchKernelGGL(k_splat_backward_sum, dim3((uint32_t)((n * 16 + 255) / 256)), dim3(256), 0, st, sp, x, n, side,
-                     slots, d_x, d_color);
+  // few particles: more waves for a crowded image's sweeps (16 x 1024 of radius
+  // 32, 256^2, in the same tiles: 101 us with 16 lanes a particle, 89 with 64,
+  // where an even cloud's sum takes 7 longer; 32 between them)
+#define SPHOPS_SPLAT_SUM(L)                                                                                       \
+  hipLaunchKernelGGL(k_splat_backward_sum<L>, dim3((uint32_t)((n * L + 255) / 256)), dim3(256), 0, st, sp, rec,  \
+                     starts, images, n, side, d_img, crowded, slots, d_x, d_color)
+  if (n <= 1 << 14) SPHOPS_SPLAT_SUM(32);
+  else SPHOPS_SPLAT_SUM(16);
+#undef SPHOPS_SPLAT_SUM
   SPHOPS_LAUNCHED();
 }
 

@@ -160,3 +160,34 @@ def test_large_pixels_outside_a_patch_add_nothing(monkeypatch):
         far = torch.isfinite(b).all(-1) & (b.abs().amax(-1) < 1e30)  # the patch does not reach column 20
         assert 0.5 < far.float().mean() < 1.0 and torch.isfinite(a[far]).all()
         assert torch.all((a - b)[far].abs() <= 72 * 2.0 ** -24 * 30 * b[far].abs().max())
+
+
+@pytest.mark.parametrize("normalize", [True, False])
+@pytest.mark.parametrize("N", [9000, 45000])
+def test_crowded_images_beside_even_ones(monkeypatch, normalize, N):
+    """Images whose particles lie in few tiles leave the tiles' route by
+    themselves, beside even ones, an empty one and ones of one and two
+    particles, few and many particles a wave; bound as above."""
+    from npa_amd import splatting as SP
+    lib = SP._lib
+    sizes = [N // 3, 0, 1, N // 3 + 5, 2, N - 2 * (N // 3) - 8]
+    # radius 32 and, without normalisation, sigma in pixels
+    kw = dict(img_size=256, sigma=6.3, normalize_color=normalize, pixel_size=2.0 / 256)
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.rand(N, 2, device="cuda", generator=g) * 2 - 1
+    x[:sizes[0]] *= 0.05  # one tile's worth
+    x[-sizes[5]:] = x[-sizes[5]:] * 0.2 + 0.9  # a corner, some patches cut, some outside
+    c = torch.rand(N, 4, device="cuda", generator=g)
+    up = torch.randn(6, 256, 256, 4, device="cuda", generator=g)
+    assert lib.sphops_splat_backward_workspace_bytes(N, 256, 6.3, -1.0, 1.0, int(normalize), 2.0 / 256) > 0
+    res = []
+    for tiled in (True, True, False):
+        if not tiled:
+            monkeypatch.setattr(lib, "sphops_splat_backward_workspace_bytes", lambda *a: 0)
+        xr, cr = x.clone().requires_grad_(True), c.clone().requires_grad_(True)
+        res.append(torch.autograd.grad(SP.splat_particles_sections(xr, cr, sizes, **kw), (xr, cr), up))
+    for a, again, b in zip(*res):
+        assert torch.equal(a, again)
+        assert torch.all((a - b).abs() <= 72 * 2.0 ** -24 * 30 * b.abs().max())
+    if not normalize:  # a crowded image's patches are swept in the same order on both routes: the same bits
+        assert all(torch.equal(a[:sizes[0]], b[:sizes[0]]) for a, b in zip(res[0], res[2]))
