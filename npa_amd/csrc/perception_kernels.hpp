@@ -1773,9 +1773,11 @@ __device__ __forceinline__ void store_entry(int32_t* __restrict__ nidx, uint32_t
 constexpr int kFillRounds = 48;
 // Rounds whose candidates it keeps there too (4 bytes each), so that the write
 // pass need not map them again: a mapping is two instructions a stencil range
-// and candidate, as much as testing a small unit.  With the units' counter
-// asked ahead (fill_items): 250 000 particles in particle mode 266 -> 243-257
-// us, 10^6 in a clamped grid 280 -> 272-281.
+// and candidate, as much as testing a small unit: 250 000 particles in
+// particle mode 237 -> 219 us, 8 x 4096 of 90 neighbours in a periodic box 94
+// -> 87.  The clamped grids' kernel needs two registers more for it than six
+// waves a SIMD have, so it is held to six: 10^6 particles 299 -> 276 us, 281
+// without the kept candidates.
 constexpr int kFillKept = 8;
 
 // Rows of the unit i0 .. i0 + ni - 1 (ni <= kUnitParticles particles of one
@@ -1948,30 +1950,27 @@ __device__ __forceinline__ void unit_rows(const GridParams& g, const float4* __r
       nx = xw[jn];
     }
     uint32_t bits = 0;
-    auto test = [&](auto near) {
-#pragma unroll
-      for (int t = 0; t < kUnitParticles; ++t) {
-        if (t < (int)ni) {
-          float r[3];
-          const float d2 = decltype(near)::value ? near_displacement<D>(g, xs[t], xj) : displacement<D, P>(g, xs[t], xj, r);
-          const bool in = d2 < g.eps2;
-          cnt[t] += (uint32_t)__popcll(__ballot(in));
-          if constexpr (OT) {
-            if (tiled && rd * kWave < po1 && rd * kWave + kWave > po0)
-              cown[t] += (uint32_t)__popcll(__ballot(in && own));
-          }
-          bits |= (in ? 1u : 0u) << t;
-        }
-      }
-    };
+    bool near = false;  // wave-uniform
     if constexpr (P) {
       bool outside = false;
 #pragma unroll
       for (int d = 0; d < D; ++d) outside = outside || xj[d] < near_lo[d] || xj[d] > near_hi[d];
-      if (inner && __ballot(outside) == 0) test(std::integral_constant<bool, true>{});
-      else test(std::integral_constant<bool, false>{});
-    } else {
-      test(std::integral_constant<bool, false>{});
+      near = inner && __ballot(outside) == 0;
+    }
+#pragma unroll
+    for (int t = 0; t < kUnitParticles; ++t) {
+      if (t < (int)ni) {
+        float r[3];
+        bool in;
+        if (P && near) in = near_displacement<D>(g, xs[t], xj) < g.eps2;
+        else in = displacement<D, P>(g, xs[t], xj, r) < g.eps2;
+        cnt[t] += (uint32_t)__popcll(__ballot(in));
+        if constexpr (OT) {
+          if (tiled && rd * kWave < po1 && rd * kWave + kWave > po0)
+            cown[t] += (uint32_t)__popcll(__ballot(in && own));
+        }
+        bits |= (in ? 1u : 0u) << t;
+      }
     }
     if (rd < (uint32_t)kFillRounds) hits[rd * kWave + lane] = (uint8_t)bits;
   }
@@ -2060,7 +2059,7 @@ __device__ __forceinline__ void unit_rows(const GridParams& g, const float4* __r
   }
 }
 
-// Periodic boxes: a lone particle of up to kLoneLight candidates is walked by
+// Full periodic boxes: a lone particle of up to kLoneLight candidates is walked by
 // its lane, one of up to 64 too where more than kLoneFew of the wave's lanes
 // have such a one (they walk at the same time).
 constexpr uint32_t kLoneLight = 24;
@@ -2079,7 +2078,9 @@ constexpr int kLoneFew = 3;
 // the whole wave unwalked (3 x 20011 particles in 3D, 8 a cell: 110 -> 83 us,
 // 4 x 16384 in 2D 40 -> 34).  In the clouds of clamped grids the lone
 // particles are the many of the sparse outskirts, where adding up first only
-// costs (10^6 particles: 272 -> 310 us).
+// costs (10^6 particles: 272 -> 310 us), and in a periodic box of less than a
+// particle a cell most are lone and light (0.7 a cell: 131 072 particles 213
+// -> 244 us, 10^6 494 -> 532; but at 2.8 a cell 369 -> 219).
 template <int D, bool P, int R, bool OT>
 __device__ __forceinline__ void lone_rows(const GridParams& g, const float4* __restrict__ xw,
                                           const int32_t* __restrict__ bo, const int32_t* __restrict__ unit_len,
@@ -2109,7 +2110,7 @@ __device__ __forceinline__ void lone_rows(const GridParams& g, const float4* __r
     w.init(g, xi, k);
   }
   bool walk = lone;
-  if constexpr (P) {
+  if (P && g.N >= 2u * g.G) {  // uniform
     uint32_t total = 0;
     if (lone) {
 #pragma unroll 1
@@ -2211,9 +2212,12 @@ __device__ __forceinline__ void lone_rows(const GridParams& g, const float4* __r
 // queue q holds the units u = q, q + kFillStripes, ... (a sample of the whole
 // cloud, so the queues carry about equal work), its counter at word
 // kUnitQueueWord of stripe q, and the waves w = q mod kFillStripes take its
-// units one at a time until it is empty: each its own first (number w /
-// kFillStripes), then the next one the counter gives, asked for while the
-// current unit is served.  A unit's cost runs from one round
+// units one at a time until it is empty.  (Units of their own first and the
+// next one asked for while the current is served hide the counter's latency,
+// 94 -> 88 us for 65 536 particles in 3D, but where the units are fewer than
+// the waves, or their costs uneven, waves that have ended leave units to waves
+// that have not: 8 x 4096 particles of 90 neighbours 57 -> 104 us, in a
+// periodic box 87 -> 188, 131 072 uneven ones 272 -> 410.)  A unit's cost runs from one round
 // to dozens (crowded cells sit together), so a fixed share per wave leaves
 // the waves that drew crowded cells running long after the others.  Even
 // waves take their chunks first, odd waves their units first, so that the
@@ -2238,16 +2242,15 @@ __device__ __forceinline__ void fill_items(const GridParams& g, const float4* __
     } else {
       const uint32_t q = wave & (kFillStripes - 1u);
       const uint32_t in_queue = q < nunits ? (nunits - q + kFillStripes - 1u) / kFillStripes : 0u;
-      const uint32_t sharers = nwaves / kFillStripes;
       unsigned long long* __restrict__ next = fs.ctr + (uint64_t)q * kStripeWords + kUnitQueueWord;
-      for (uint32_t i = wave / kFillStripes; i < in_queue;) {
-        uint32_t taken = 0;
-        if (in_queue > sharers && __lane_id() == 0) taken = (uint32_t)atomicAdd(next, 1ull);
+      for (;;) {
+        uint32_t i = 0;
+        if (__lane_id() == 0) i = (uint32_t)atomicAdd(next, 1ull);
+        i = (uint32_t)__builtin_amdgcn_readfirstlane((int)i);
+        if (i >= in_queue) break;
         const uint2 ud = units[i * kFillStripes + q];
         unit_rows<D, P, R, OT>(g, xw, bo, __builtin_amdgcn_readfirstlane(ud.x),
                                __builtin_amdgcn_readfirstlane(ud.y), wave, hits, nidx, nstart, ncnt, fs, ft);
-        if (in_queue <= sharers) break;
-        i = sharers + (uint32_t)__builtin_amdgcn_readfirstlane((int)taken);
       }
     }
   }
@@ -2256,7 +2259,7 @@ __device__ __forceinline__ void fill_items(const GridParams& g, const float4* __
 // M: particle mode (stencil of single cells) or grid mode (stencil rows);
 // OT: cell tiles (FillTiles).
 template <int D, bool P, bool M, bool OT>
-__global__ __launch_bounds__(kThreads) void k_fill(GridParams g, const float4* __restrict__ xw,
+__global__ __launch_bounds__(kThreads, P || OT ? 4 : 6) void k_fill(GridParams g, const float4* __restrict__ xw,
                                                    const int32_t* __restrict__ bo,
                                                    const int32_t* __restrict__ unit_len,
                                                    const uint2* __restrict__ units,

@@ -12,6 +12,9 @@ pytestmark = pytest.mark.gpu
 
 CASES = [(3, 5, 1500, 1.0, "grid"), (3, 8, 6001, 1.0, "particle"), (3, 4, 300, 1.0, "grid"), (3, 3, 90, 1.0, "grid"),
          (2, 8, 900, 1.0, "particle"), (2, 40, 20011, 1.0, "grid"), (3, 6, 1200, 2.6, "grid"), (2, 9, 70, 9.5, "grid")]
+# about one and about two particles a cell: many alone in theirs, on both sides
+# of the rule that adds their candidates up first
+CASES += [(3, 8, 500, 1.0, "grid"), (3, 8, 1100, 1.0, "particle"), (2, 32, 1000, 1.0, "grid"), (2, 32, 2100, 1.0, "grid")]
 
 
 @pytest.mark.parametrize("dim,gs,N,spread,mode", CASES)

@@ -163,3 +163,29 @@ def test_records_only_for_a_backward(monkeypatch):
     outs.append(PF.perceive(xr, sr, grid, 0.1, stopgrad_pos=False))
     assert kept == [(False, False), (True, True)]
     assert not outs[0][0].requires_grad and all(torch.equal(a, b) for a, b in zip(outs[0][:3], outs[1][:3]))
+
+
+@pytest.mark.parametrize("dim,per,mode,C", GRIDS[:3])
+def test_steps_in_flight_keep_their_own_lists(dim, per, mode, C):
+    """Several forwards on one grid before the first backward, the backwards
+    in reverse order: each reads its own list and records."""
+    from npa_amd import perceive as PF
+    grid, x, s = _grid(dim, per, mode, C)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    clouds = [(x, s), (x.roll(7, 1) * 0.9, s.flip(1)), (x * 0.8, s * 2)]
+
+    def forward(cloud):
+        xr, sr = (t.clone().requires_grad_(True) for t in cloud)
+        return xr, sr, PF.perceive(xr, sr, grid, 0.1, stopgrad_pos=False)[0]
+
+    W = PF.feature_width(C, dim, PF.STATE_GRAD | PF.DENSITY_GRAD)
+    up = torch.randn(2, 301, W, device="cuda", generator=g)
+    alone = []
+    for cloud in clouds:
+        xr, sr, z = forward(cloud)
+        z.backward(up)
+        alone.append((xr.grad, sr.grad))
+    steps = [forward(cloud) for cloud in clouds]
+    for (xr, sr, z), ref in zip(steps[::-1], alone[::-1]):
+        z.backward(up)
+        assert torch.equal(xr.grad, ref[0]) and torch.equal(sr.grad, ref[1])
