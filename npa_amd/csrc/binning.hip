@@ -567,8 +567,14 @@ __device__ __forceinline__ uint32_t run_end(const uint64_t* __restrict__ kv, uin
 // every cell takes at the same time, and needs no chunk table: with the
 // permutation in the same launch 6 us, where the chunk table, the chunks and
 // the permutation took 57 us for 8 K cells of 65536 particles (2D box), 56 us
-// for 8 K cells of 60033 and 68 us for 2 M cells of 250007.  The block-row
-// kernel loads its bounds from bin_offsets, which is in cache.
+// for 8 K cells of 60033.  The block-row kernel loads its bounds from
+// bin_offsets, which is in cache.  The line lies between two kinds of clouds.
+// Instantiate as a whole, chunks and searches, us, spread evenly over a 3D box
+// (1000, 90 000 and 10^6 particles): 262 K cells 30 and 25, 53 and 45, 109 and
+// 87; 1.0 M 29 and 28, 52 and 51, 101 and 98; 2.1 M 38 and 41, 67 and 77, 119
+// and 128; 4.1 M 37 and 49, 67 and 95, 118 and 151.  But the mixtures of the
+// growth workload, whose particles lie in few chunks, take 40 more with chunks
+// at 2.1 M cells (250 007 particles, Morton order: a traced step 575 and 615).
 constexpr uint64_t kRunSearchMinCells = 1ull << 22;
 
 // Permutation (destination slot of every input particle), in grid mode
