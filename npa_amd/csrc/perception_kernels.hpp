@@ -2059,11 +2059,13 @@ __device__ __forceinline__ void unit_rows(const GridParams& g, const float4* __r
   }
 }
 
-// Full periodic boxes: a lone particle of up to kLoneLight candidates is walked by
-// its lane, one of up to 64 too where more than kLoneFew of the wave's lanes
-// have such a one (they walk at the same time).
+// Full periodic boxes: a lone particle of up to kLoneLight candidates is walked
+// by its lane, the others go to the whole wave.  Limits of 8, 24 and 64, 131 072
+// particles of 12 neighbours in 2D: 101, 100 and 124 us, of 9: 124, 136 and 132;
+// in 3D of 9: 247 at 24 and 321 at 64.  Letting a wave with more than three
+// particles of 25 to 64 candidates walk them took 311 there, 220 for 204 at 12
+// neighbours, and gained 3 at most (2D, 9).
 constexpr uint32_t kLoneLight = 24;
-constexpr int kLoneFew = 3;
 
 // Lone particles of the chunk of 64 particles starting at k0, one lane each:
 // a first walk over the stencil counts the candidates and marks the in-radius
@@ -2080,7 +2082,7 @@ constexpr int kLoneFew = 3;
 // particles are the many of the sparse outskirts, where adding up first only
 // costs (10^6 particles: 272 -> 310 us), and in a periodic box of less than a
 // particle a cell most are lone and light (0.7 a cell: 131 072 particles 213
-// -> 244 us, 10^6 494 -> 532; but at 2.8 a cell 369 -> 219).
+// -> 244 us, 10^6 494 -> 532; but at 2.8 a cell 369 -> 204).
 template <int D, bool P, int R, bool OT>
 __device__ __forceinline__ void lone_rows(const GridParams& g, const float4* __restrict__ xw,
                                           const int32_t* __restrict__ bo, const int32_t* __restrict__ unit_len,
@@ -2119,8 +2121,7 @@ __device__ __forceinline__ void lone_rows(const GridParams& g, const float4* __r
         total += w.jend - w.j;
       }
     }
-    const uint64_t mid = __ballot(lone && total > kLoneLight && total <= (uint32_t)kWave);
-    walk = lone && total <= (__popcll(mid) > kLoneFew ? (uint32_t)kWave : kLoneLight);
+    walk = lone && total <= kLoneLight;
   }
   if (walk) {
 #pragma unroll 1
@@ -2481,7 +2482,9 @@ inline bool row_offsets_fit_32(const Grid& g, uint32_t C) {
 
 // Lane-split kernels (pass B, forward and backward): a list, its split
 // schedule, and rows of 16 or 32 channels on 16-byte bases, or of 8, 12, 20
-// or 24 (read in dword-aligned pieces) with row offsets of 32 bits.
+// or 24 (read in dword-aligned pieces) with row offsets of 32 bits.  Each width
+// is an instantiation of every pass-B kernel; those that no workload has (28)
+// keep the grouped kernels, unmeasured.
 inline bool split_ok(const Grid& g, const OpPtrs& a) {
   if (a.nidx == nullptr || a.waves2 == nullptr) return false;
   if (a.C == 16 || a.C == 32) return aligned16(a.s) && aligned16(a.g) && aligned16(a.g2);

@@ -168,7 +168,10 @@ def test_records_only_for_a_backward(monkeypatch):
 @pytest.mark.parametrize("dim,per,mode,C", GRIDS[:3])
 def test_steps_in_flight_keep_their_own_lists(dim, per, mode, C):
     """Several forwards on one grid before the first backward, the backwards
-    in reverse order: each reads its own list and records."""
+    in reverse order: each reads its own list and records (another cloud's
+    give other values altogether).  Which rows the first lists' estimated
+    buffers leave to the stencil, and so the order of their sums, may differ:
+    bound as for an overflowing list."""
     from npa_amd import perceive as PF
     grid, x, s = _grid(dim, per, mode, C)
     g = torch.Generator(device="cuda").manual_seed(3)
@@ -188,4 +191,5 @@ def test_steps_in_flight_keep_their_own_lists(dim, per, mode, C):
     steps = [forward(cloud) for cloud in clouds]
     for (xr, sr, z), ref in zip(steps[::-1], alone[::-1]):
         z.backward(up)
-        assert torch.equal(xr.grad, ref[0]) and torch.equal(sr.grad, ref[1])
+        for a, b in zip((xr.grad, sr.grad), ref):
+            assert torch.allclose(a, b, rtol=1e-4, atol=1e-4 * b.abs().max().item())
